@@ -487,14 +487,14 @@ int qwen_matmul_dispatch(const void* weight, int type, uint64_t num_elements, co
 /* rows GEMVs of one matrix: y[t][m] = sum_{k<K} W[element_offset + m*K + k] * x[t][k]
  * for t < rows, m < M (x fp32 [rows x K], y fp32 [rows x M], row-major) -- the
  * reference's per-token matmul_dispatch over a prompt as one call. Q4_K and
- * Q6_K with K % 256 == 0, element_offset % 256 == 0, x 16-byte aligned and
- * rows >= 16 run on the matrix cores: each token row is scaled by a power of
- * two and split exactly into two fp16 parts (prep kernel, into the workspace),
- * the quants enter as exact fp16 integers, products are exact and sums fp32 --
- * an fp32 dot product's accuracy, not the reference's bits. Those cases need a
- * 16-byte aligned workspace of qwen_matmul_rows_workspace_bytes(rows, K)
- * bytes (QWEN_STATUS_INVALID_ARGUMENT otherwise); the other cases run
- * qwen_matmul_dispatch once per token and ignore it. A row of x holding an
+ * Q6_K with K % 256 == 0, element_offset % 256 == 0, x 16-byte aligned and 3
+ * rows or more (4 from K = 2304) run on the matrix cores: each token row is
+ * scaled by a power of two and split exactly into two fp16 parts, the quants
+ * enter as exact fp16 integers, products are exact and sums fp32 -- an fp32 dot
+ * product's accuracy, not the reference's bits. From 16 rows on those cases
+ * need a 16-byte aligned workspace of qwen_matmul_rows_workspace_bytes(rows, K)
+ * bytes (QWEN_STATUS_INVALID_ARGUMENT otherwise); fewer rows ignore it, and the
+ * other cases run qwen_matmul_dispatch once per token. A row of x holding an
  * infinity gives non-finite outputs (the NaN / infinity pattern may differ
  * from the reference's). rows == 0 is a no-op. Statuses and messages as
  * qwen_matmul_dispatch; rows < 0 or a NULL x / y -> QWEN_STATUS_INVALID_ARGUMENT.
@@ -505,7 +505,7 @@ int qwen_matmul_rows(const void* weight, int type, uint64_t num_elements, const 
                      size_t workspace_bytes, void* stream);
 
 /* Workspace bytes qwen_matmul_rows needs for rows tokens of K elements (0 when
- * the call takes the per-token path: rows < 16 or K % 256 != 0). */
+ * it needs none: rows < 16 or K % 256 != 0). */
 size_t qwen_matmul_rows_workspace_bytes(int rows, int K);
 
 /* One projection of qwen_matmul_dispatch_multi: the arguments of one
@@ -537,10 +537,10 @@ int qwen_matmul_dispatch_multi(const qwen_gemv_desc* descs, int n, const float* 
 
 /* qwen_matmul_rows for n matrices of the same x [rows x K]: y_j [rows x M_j] =
  * x W_j^T for each descriptor (split must be 0), with the results of n
- * qwen_matmul_rows calls bit for bit. x is prepared once (one prep launch) and
- * the Q4_K / Q6_K matrices of one type run in one GEMM launch (up to 8 per
- * launch), so small matrices (a layer's 32-row gate projections) share the
- * launch of the large ones; other types and offsets take the per-token path.
+ * qwen_matmul_rows calls bit for bit. x is prepared once (at most one prep
+ * launch) and the Q4_K / Q6_K matrices of one type run in one GEMM launch (up
+ * to 8 per launch; from 769 rows on, matrices of up to 64 rows in one of their
+ * own); other types and offsets take the per-token path.
  * Validation as qwen_matmul_dispatch_multi; workspace as qwen_matmul_rows
  * (qwen_matmul_rows_workspace_bytes(rows, K)). 0 <= n <= 64.
  * ref: the per-token calls of src/layer_gdn.cpp:83-86, src/layer_attn.cpp:85-87 over a prompt */

@@ -16,27 +16,28 @@
 //         with S_g the group sums of v; the min terms are one fp16 MFMA per
 //         tile and block (v_mfma_f32_16x16x16_f16, k = 8 groups x 2 parts):
 //         m_g exact, S_g 2^-5 split into two fp16 parts like x (22 bits).
-//   Q6_K: B = q - 32 (exact); the signed 8-bit scales do not fit in the fp16
-//         operand, so per 16-element group y += (d sc) P_g (one FMA).
+//   Q6_K: (q - 32) * sc reaches 12 bits, so B = Bh + Bl (exact, |Bl| <= 1) and
+//         three products per operand pair, h Bh + l Bh + h Bl (l Bl is below
+//         2^-22 of h Bh); the wide tiles instead take B = q - 32 and apply the
+//         scale per 16-element group, y += (d sc) P_g (one FMA): fewer MFMAs.
 // The result is scaled back by 2^-e (exact). Products of fp16 values are exact
 // in the MFMA's fp32 accumulation, so the roundings are those of an fp32 sum.
 //
-// fp16 operands are built with v_perm / v_pk_add_f16 only: bytes b < 1024
-// placed under 0x64 give the fp16 1024 + b, and one packed fp16 add of -1024
-// (Q4_K after the integer q * sc, Q6_K -1056 for q - 32) leaves the exact
-// value. The perm pairs bytes (0, 2) and (1, 3) of a word, so the prep kernel
-// stores x in that order within each 4 consecutive elements (0, 2, 1, 3);
-// A and B then agree slot by slot.
+// fp16 operands are built from bits: a byte b under 0x64 is the fp16 1024 + b,
+// so one and-or places two quants and one packed fused multiply-add with sc
+// and -1024 sc leaves q * sc (Q4_K; a shift more for every second pair). The
+// pairs are bytes (0, 2) and (1, 3) of a word; x is stored in that order.
 //
-// Work, per 32-element stage (one barrier per stage): a workgroup of 8 waves
-// owns 128 tokens x 256 weight rows, wave w rows 64 (w % 4) .. +63 of token half
-// w / 4, and the next stage's B operands are decoded (each wave pair splitting
-// the work, through LDS) while the current stage's products run. Q4_K: 16 x 16
-// tiles on v_mfma_f32_16x16x32_f16, operands through an LDS ring filled three
-// stages ahead by global -> LDS loads. Q6_K: 32 x 32 tiles on
-// v_mfma_f32_32x32x16_f16 (K = one 16-element scale group), x staged through
-// LDS from registers, quant bytes and scales per half-block through LDS. The
-// kernels' own comments have the details.
+// Four kernels, by token count (gemm_path below has the lines and both sides'
+// times): gemm_few (up to 16 tokens, 160 from K = 4096) converts x itself and
+// splits K over its waves; gemm_kquant splits K in 4 or 2 slices over waves of
+// a workgroup with the tile shape that fills the 256 CUs in the fewest rounds;
+// gemm_q4k_wide and gemm_q6k_wide (128 x 256 tiles) take long prompts.
+// Measured, us for the GDN layer's input projections (M = 8192, 4096, 32, 32 at
+// K = 2048, one call) and output projection (M = 2048 at K = 4096), Q4_K:
+//   tokens                            9        77        300       777      4096
+//   one form for all (before)     103 / 30  71 / 131  77 / 134  146 / 136  510 / 175
+//   these kernels                  13 / 12  31 /  21  56 /  42  137 /  58  413 / 152
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
@@ -55,14 +56,12 @@ typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kGR = 256;           // weight rows per workgroup (64 per wave)
-constexpr int kGemmMinRows = 16;   // fewer tokens: one GEMV per token
-constexpr int kGemmMaxRows = 65535 * 128;   // token blocks of 128 in grid.y
-constexpr int kXRow = 40;          // halves per staged token row (32 + 8 padding)
+constexpr int kGemmMinRows = 16;   // fewer tokens need no workspace
+constexpr int kGemmMaxRows = 65535 * 128;
 
 // Matrices of one launch (all of one K-quant type, one x): workgroup column
-// blockIdx.x in [start[j], start[j+1]) works on rows (blockIdx.x - start[j]) * kGR ..
-// of matrix j.
+// c in [start[j], start[j+1]) works on matrix j's rows from
+// (column - start[j]) * the tile's rows.
 constexpr int kGemmJobs = 8;
 struct GemmJobs {
     const uint8_t* w[kGemmJobs];
@@ -80,8 +79,7 @@ struct GemmJob {
     int M, mb;
 };
 
-__device__ __forceinline__ GemmJob gemm_job(const GemmJobs& jobs) {
-    const int bx = static_cast<int>(blockIdx.x);
+__device__ __forceinline__ GemmJob gemm_job(const GemmJobs& jobs, int bx) {
     int j = 0;
     while (j + 1 < jobs.n && bx >= jobs.start[j + 1]) ++j;
     return GemmJob{jobs.w[j], jobs.y[j], jobs.ub0[j], jobs.M[j], bx - jobs.start[j]};
@@ -102,28 +100,6 @@ __device__ __forceinline__ float wave_max_abs(float v) {
 
 __device__ __forceinline__ uint32_t half_bits_of(float v) {
     return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
-}
-
-// The two fp16 parts of v (element order 0, 2, 1, 3) and the sums of v per 32
-// elements, for the 4 values of lane `lane` at k (k = 4 lane + 256 i).
-__device__ __forceinline__ void prep_store(const float4 v4, int e, int k, int lane, size_t t, int nst,
-                                           float* __restrict__ sx, uint16_t* __restrict__ xp) {
-    const float v[4] = {ldexpf(v4.x, e), ldexpf(v4.y, e), ldexpf(v4.z, e), ldexpf(v4.w, e)};
-    uint32_t h[4], l[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const _Float16 hh = static_cast<_Float16>(v[i]);
-        h[i] = __builtin_bit_cast(uint16_t, hh);
-        l[i] = half_bits_of(v[i] - static_cast<float>(hh));
-    }
-    uint16_t* dst = xp + (t * nst + (k >> 5)) * 64 + (k & 31);
-    *reinterpret_cast<uint2*>(dst) = make_uint2(h[0] | (h[2] << 16), h[1] | (h[3] << 16));
-    *reinterpret_cast<uint2*>(dst + 32) = make_uint2(l[0] | (l[2] << 16), l[1] | (l[3] << 16));
-    float s = (v[0] + v[1]) + (v[2] + v[3]);
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
-    if ((lane & 7) == 0) sx[t * nst + (k >> 5)] = s;
 }
 
 // Exponent slot of a token row holding an infinity: the fp16 split cannot carry
@@ -159,95 +135,327 @@ __device__ __forceinline__ float max_abs4(float m, const float4& v) {
     return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
 }
 
-// One wave per token: e, the two fp16 parts of x * 2^e (element order 0, 2, 1, 3
-// within each 4) and the sums of x * 2^e per 32 elements. K % 256 == 0. NIT > 0:
-// K == 256 NIT, the row is held in registers (read once); NIT == 0: any K, read twice.
+// ------------------------------------------------------------------ x in fragment order
+// A token tile is 16 tokens (the last one of a call T % 16, r of them); a block's 256 elements are 8 MFMA
+// depths of 32. Lane (lr, lk) = (token or weight row, k group) of depth s = 2 u + j takes the 8 elements
+//   128 (lk / 2) + 32 u + 16 (lk % 2) + 8 j + (0, 2, 1, 3, 4, 6, 5, 7)
+// of its row, for x and for the weights alike: a lane's share of a weight block is then whole 16-byte pieces
+// (Q4_K 2, Q6_K 3), and the order within 8 is the one in which pairs of quants leave a word (below).
+// The fp16 parts of a tile are stored fragment by fragment, [block][depth][part][lk][lr] x 16 bytes, so that a
+// wave's load of one A operand is 1 KB in a row.
+constexpr int kTile = 16;
+
+__device__ __forceinline__ size_t tile_base(int tile, int K) { return static_cast<size_t>(tile) * kTile * K * 4; }
+
+// The fp16 parts of 8 values times 2^e, in the operand's order (packed pairs), and the sum of the scaled values.
+__device__ __forceinline__ float split8(const float4& a, const float4& b, int e, uint32_t (&hi)[4], uint32_t (&lo)[4]) {
+    const float f[8] = {ldexpf(a.x, e), ldexpf(a.y, e), ldexpf(a.z, e), ldexpf(a.w, e),
+                        ldexpf(b.x, e), ldexpf(b.y, e), ldexpf(b.z, e), ldexpf(b.w, e)};
+    uint32_t h[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const _Float16 hh = static_cast<_Float16>(f[i]);
+        h[i] = __builtin_bit_cast(uint16_t, hh);
+        l[i] = half_bits_of(f[i] - static_cast<float>(hh));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int k = 4 * (i >> 1) + (i & 1);
+        hi[i] = h[k] | (h[k + 2] << 16);
+        lo[i] = l[k] | (l[k + 2] << 16);
+    }
+    return ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+}
+
+// One workgroup of 16 waves per token tile, wave = token; 512 elements (a chunk of 8 per lane) per round. Each
+// lane's two 16-byte pieces go to the round's LDS image of the fragments (slot lr ^ (chunk % 16) of its 16, so
+// neither side conflicts) and the workgroup writes the image out in order.
+// NIT > 0: K == 512 NIT, the row is held in registers (read once); NIT == 0: any K % 256 == 0, read twice.
 template <int NIT>
-__global__ __launch_bounds__(256) void gemm_prep_x(const float* __restrict__ x, int* __restrict__ ex,
-                                                   float* __restrict__ sx, uint16_t* __restrict__ xp, int T, int K) {
-    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (t >= T) return;   // the whole wave
-    const float* row = x + static_cast<size_t>(t) * K;
-    const int nst = K >> 5;
+__global__ __launch_bounds__(1024) void gemm_prep_x(const float* __restrict__ x, int* __restrict__ ex,
+                                                    float* __restrict__ sx, uint8_t* __restrict__ xp, int T, int K) {
+    __shared__ __align__(16) uint4 img[2][2048];
+    const int wv = wave_in_block(), lane = threadIdx.x & 63;
+    const int t = blockIdx.x * kTile + wv;
+    const int r = min(kTile, T - static_cast<int>(blockIdx.x) * kTile);   // tokens of this tile
+    const bool live = wv < r;
+    const float* row = x + static_cast<size_t>(live ? t : T - 1) * K;
+    const int nst = K >> 5, nit = NIT ? NIT : (K + 511) >> 9;
     float m = 0.f;
+    float4 v[NIT ? 2 * NIT : 2];
+    auto load = [&](int it, float4* d) {   // the lane's 8 elements of round `it` (zero past K)
+        const int k = 512 * it + 8 * lane;
+        const bool in = NIT || k < K;
+        d[0] = in ? ld4(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        d[1] = in ? ld4(row + k + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
     if constexpr (NIT > 0) {
-        float4 v[NIT];
 #pragma unroll
-        for (int i = 0; i < NIT; ++i) {
-            v[i] = ld4(row + 4 * lane + 256 * i);
-            m = max_abs4(m, v[i]);
-        }
-        const int e = prep_exponent(wave_max_abs(m));
-        if (lane == 0) ex[t] = e;
-        const int es = e == kRowNonFinite ? 0 : e;   // a marked row's parts are not used
+        for (int it = 0; it < NIT; ++it) load(it, v + 2 * it);
 #pragma unroll
-        for (int i = 0; i < NIT; ++i) prep_store(v[i], es, 4 * lane + 256 * i, lane, t, nst, sx, xp);
+        for (int i = 0; i < 2 * NIT; ++i) m = max_abs4(m, v[i]);
     } else {
-        for (int k = 4 * lane; k < K; k += 256) m = max_abs4(m, ld4(row + k));
-        const int e = prep_exponent(wave_max_abs(m));
-        if (lane == 0) ex[t] = e;
-        const int es = e == kRowNonFinite ? 0 : e;
-        for (int k = 4 * lane; k < K; k += 256) prep_store(ld4(row + k), es, k, lane, t, nst, sx, xp);
+        for (int it = 0; it < nit; ++it) {
+            load(it, v);
+            m = max_abs4(max_abs4(m, v[0]), v[1]);
+        }
+    }
+    const int e = prep_exponent(wave_max_abs(m));
+    if (live && lane == 0) ex[t] = e;
+    const int es = e == kRowNonFinite ? 0 : e;   // a marked row's parts are not used
+    uint8_t* out = xp + tile_base(blockIdx.x, K);
+    const int c16 = lane & 15;                                             // chunk % 16 = 4 u + 2 (lk % 2) + j
+    const int frag = ((lane >> 5) * 8 + 2 * (c16 >> 2) + (c16 & 1)) * 2;   // of part 0: (block of the round, depth)
+    const int lk = 2 * ((lane >> 4) & 1) + ((c16 >> 1) & 1);
+    const int slot = (frag * 4 + lk) * 16 + (wv ^ c16);
+    auto round = [&](int it, const float4* d) {
+        uint32_t h[4], l[4];
+        float s = split8(d[0], d[1], es, h, l);
+        uint4* im = img[it & 1];
+        im[slot] = make_uint4(h[0], h[1], h[2], h[3]);
+        im[slot + 64] = make_uint4(l[0], l[1], l[2], l[3]);
+        s += __shfl_xor(s, 1);
+        s += __shfl_xor(s, 2);
+        const int k = 512 * it + 8 * lane;
+        if (live && (lane & 3) == 0 && (NIT || k < K)) sx[static_cast<size_t>(t) * nst + (k >> 5)] = s;
+        __syncthreads();
+        // 2048 pieces of the image: piece p = (fragment p / 64, lane (lk, lr) = p % 64)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int p = threadIdx.x + 1024 * i;
+            const int f2 = p >> 6, k4 = (p >> 4) & 3, lr = p & 15;
+            const int dep = (f2 >> 1) & 7;   // 2 u + j
+            const int cc = 4 * (dep >> 1) + 2 * (k4 & 1) + (dep & 1);
+            if (lr < r && (NIT || 512 * it + 256 * (f2 >> 4) < K))
+                st16(out + 16 * (static_cast<size_t>((32 * it + f2) * 4 + k4) * r + lr), im[(p & ~15) + (lr ^ cc)]);
+        }
+    };
+    if constexpr (NIT > 0) {
+#pragma unroll
+        for (int it = 0; it < NIT; ++it) round(it, v + 2 * it);
+    } else {
+        for (int it = 0; it < nit; ++it) {
+            load(it, v);
+            round(it, v);
+        }
     }
 }
 
-// A thread's share of one stage of x: 32 bytes (part p: fp16 part p/2, halves
-// 16 (p%2) .. +15 of its token's 32).
-struct XRegs {
-    uint4 a, b;
+// ------------------------------------------------------------------ the GEMM
+__device__ __forceinline__ f16x2_t h2(uint32_t w) { return __builtin_bit_cast(f16x2_t, w); }
+__device__ __forceinline__ uint32_t w2(f16x2_t h) { return __builtin_bit_cast(uint32_t, h); }
+__device__ __forceinline__ f16x2_t fma2(f16x2_t a, f16x2_t b, f16x2_t c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ f16x2_t dup2(float v) {
+    const _Float16 h = static_cast<_Float16>(v);
+    return f16x2_t{h, h};
+}
+
+// 16 bytes at a 2-byte aligned address (gfx950 global loads take any byte
+// alignment; Q6_K blocks are 210 bytes).
+__device__ __forceinline__ uint4 ldg16_a2(const uint8_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
+    return v;
+}
+__device__ __forceinline__ uint2 ldg8_a2(const uint8_t* p) {
+    uint2 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 8);
+    return v;
+}
+
+// A lane's share of one block of its weight row (the mapping above). Q4_K, element i of a block
+// (src/cuda/matmul_q4.cu:76-96): qs byte 16 + 32 (i / 64) + i % 32, low nibble if i % 64 < 32, scale i / 32:
+// q[g] holds the bytes of depths u = 2 g, 2 g + 1 (both nibbles), hd the 16-byte header. Q6_K
+// (src/cuda/matmul_q4.cu:105-126): ql byte 64 (i / 128) + 32 ((i % 128) / 32 & 1) + i % 32, low nibble in quarters
+// 0, 1 of a half, qh byte 128 + 32 (i / 128) + i % 32 bits 2 quarter, scale byte 192 + i / 16, d at 208: q[0], q[1]
+// the ql bytes of even and odd u, qh, the half's 8 scales and d.
+template <int TYPE>
+struct WBlock;
+template <>
+struct WBlock<kQ4_K> {
+    uint4 q[2], hd;
+    __device__ __forceinline__ void load(const uint8_t* base, uint32_t row, int lk) {
+        const uint32_t o = row + 16u + 64u * (lk >> 1) + 16u * (lk & 1);
+        hd = ld16(base + row);
+        q[0] = ld16(base + o);
+        q[1] = ld16(base + (o + 32u));
+    }
+};
+template <>
+struct WBlock<kQ6_K> {
+    uint4 q[2], qh;
+    uint2 sc;
+    uint16_t d;
+    __device__ __forceinline__ void load(const uint8_t* base, uint32_t row, int lk) {
+        const uint32_t h = lk >> 1, l = lk & 1, o = row + 64u * h + 16u * l;
+        q[0] = ldg16_a2(base + o);
+        q[1] = ldg16_a2(base + (o + 32u));
+        qh = ldg16_a2(base + (row + 128u + 32u * h + 16u * l));
+        sc = ldg8_a2(base + (row + 192u + 8u * h));
+        d = *reinterpret_cast<const uint16_t*>(base + (row + 208u));
+    }
 };
 
-__device__ __forceinline__ XRegs load_x(const uint16_t* __restrict__ src) {
-    return XRegs{ld16(src), ld16(src + 8)};
+__device__ __forceinline__ uint32_t word_of(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+// Scale of depth u of the lane's half-block, as the fp16 operands need it.
+template <int TYPE>
+struct WScale;
+template <>
+struct WScale<kQ4_K> {
+    f16x2_t s, c;   // q sc = fma(1024 + q, sc, -1024 sc); high nibbles fma(1024 + 16 q, sc / 16, -64 sc): exact
+    template <int U>
+    __device__ __forceinline__ void set(const WBlock<kQ4_K>& b, int lk) {
+        // scale_min_k4 (src/cuda/matmul_q4.cu:18-26): group 4 (lk / 2) + U
+        const uint32_t lo = (b.hd.y >> (8 * U)) & 63u;
+        const uint32_t hi = ((b.hd.w >> (8 * U)) & 15u) | ((b.hd.y >> (8 * U + 2)) & 0x30u);
+        from<U>((lk & 2) ? hi : lo);
+    }
+    // (q - 8) sc = fma(16 + q, sc, -24 sc), exact
+    template <int U>
+    __device__ __forceinline__ void set_centred(const WBlock<kQ4_K>& b, int lk) {
+        const uint32_t lo = (b.hd.y >> (8 * U)) & 63u;
+        const uint32_t hi = ((b.hd.w >> (8 * U)) & 15u) | ((b.hd.y >> (8 * U + 2)) & 0x30u);
+        s = h2(((lk & 2) ? hi : lo) * 0x00010001u + 0x64006400u) - dup2(1024.f);
+        c = s * dup2(-24.f);
+    }
+    template <int U>
+    __device__ __forceinline__ void from(uint32_t v) {
+        const f16x2_t sc = h2(v * 0x00010001u + 0x64006400u) - dup2(1024.f);   // exact
+        s = (U & 1) ? sc * dup2(0.0625f) : sc;
+        c = sc * ((U & 1) ? dup2(-64.f) : dup2(-1024.f));
+    }
+};
+template <>
+struct WScale<kQ6_K> {
+    f16x2_t s;
+    template <int U>
+    __device__ __forceinline__ void set(const WBlock<kQ6_K>& b, int lk) {
+        const uint32_t w = U < 2 ? b.sc.x : b.sc.y;   // scales 2 U, 2 U + 1 of the half
+        const uint32_t v = ((w >> (16 * (U & 1) + 8 * (lk & 1))) & 0xffu) ^ 0x80u;
+        s = h2(v * 0x00010001u + 0x64006400u) - dup2(1152.f);   // signed 8 bits, exact
+    }
+};
+
+// B operand(s) of depth (U, J). Bits 0x64bb are the fp16 1024 + bb, so quants placed under 0x64 by one and-or
+// become exact small integers by one packed add or fused multiply-add.
+template <int U, int J>
+__device__ __forceinline__ void decode_q4(const uint4& q, const WScale<kQ4_K>& sc, uint32_t k64, f16x8_t (&B)[1]) {
+    constexpr uint32_t mask = (U & 1) ? 0x00f000f0u : 0x000f000fu;
+    uint32_t e[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t w = word_of(q, 2 * J + i);
+        e[2 * i] = w2(fma2(h2((w & mask) | k64), sc.s, sc.c));
+        e[2 * i + 1] = w2(fma2(h2(((w >> 8) & mask) | k64), sc.s, sc.c));
+    }
+    __builtin_memcpy(&B[0], e, 16);
 }
 
-// Bytes (0, 2) and (1, 3) of n placed under `hi` (byte values 0 or 0x64).
-__device__ __forceinline__ uint32_t bytes02(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04020400u); }
-__device__ __forceinline__ uint32_t bytes13(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04030401u); }
-
-__device__ __forceinline__ uint32_t hadd2(uint32_t w, _Float16 c) {
-    const f16x2_t r = __builtin_bit_cast(f16x2_t, w) + f16x2_t{c, c};
-    return __builtin_bit_cast(uint32_t, r);
+template <int U, int J>
+__device__ __forceinline__ void decode(const WBlock<kQ4_K>& b, const WScale<kQ4_K>& sc, uint32_t k64, f16x8_t (&B)[1]) {
+    decode_q4<U, J>(b.q[U >> 1], sc, k64, B);
 }
 
-// fp16 q * sc of four quants (bytes of n, each < 16), sc < 64: two words in
-// the order (0, 2), (1, 3).
-__device__ __forceinline__ void q4_operand(uint32_t n, uint32_t sc, uint32_t& w02, uint32_t& w13) {
-    w02 = hadd2(__umul24(bytes02(0, n), sc) + 0x64006400u, static_cast<_Float16>(-1024.0f));
-    w13 = hadd2(__umul24(bytes13(0, n), sc) + 0x64006400u, static_cast<_Float16>(-1024.0f));
+// (q - 8) sc: a nibble in the top four mantissa bits under 0x4c00 is the fp16 16 + q.
+template <int U, int J>
+__device__ __forceinline__ void decode_centred(const WBlock<kQ4_K>& b, const WScale<kQ4_K>& sc, f16x8_t (&B)[1]) {
+    constexpr int lo = (U & 1) ? 2 : 6, hi = (U & 1) ? 6 : 2;   // left shift of bytes 0, 2; right shift of bytes 1, 3
+    uint32_t e[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t w = word_of(b.q[U >> 1], 2 * J + i);
+        e[2 * i] = w2(fma2(h2(((w << lo) & 0x03c003c0u) | 0x4c004c00u), sc.s, sc.c));
+        e[2 * i + 1] = w2(fma2(h2(((w >> hi) & 0x03c003c0u) | 0x4c004c00u), sc.s, sc.c));
+    }
+    __builtin_memcpy(&B[0], e, 16);
 }
 
-// fp16 q - 32 of four 6-bit quants (bytes of q): two words in the order (0, 2), (1, 3).
-__device__ __forceinline__ void q6_operand(uint32_t q, uint32_t& w02, uint32_t& w13) {
-    w02 = hadd2(bytes02(0x64646464u, q), static_cast<_Float16>(-1056.0f));
-    w13 = hadd2(bytes13(0x64646464u, q), static_cast<_Float16>(-1056.0f));
+// (q - 32) sc in two fp16 parts, exactly: magnitudes up to 2048 fit the first one.
+template <int U, int J>
+__device__ __forceinline__ void decode(const WBlock<kQ6_K>& b, const WScale<kQ6_K>& sc, uint32_t k64, f16x8_t (&B)[2]) {
+    uint32_t e[4], l[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t w = word_of(b.q[U & 1], 2 * J + i), h = word_of(b.qh, 2 * J + i);
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+            const uint32_t n = (w >> (8 * o + 4 * (U >> 1))) & 0x000f000fu;
+            constexpr int up = 4 - 2 * U;   // bits 2 U of qh to bits 4, 5
+            const int sh = up - 8 * o;
+            const uint32_t t = (sh >= 0 ? h << (sh & 31) : h >> (-sh & 31)) & 0x00300030u;
+            const f16x2_t q = h2(n | (t | k64)) - dup2(1056.f);
+            const f16x2_t p = q * sc.s;
+            e[2 * i + o] = w2(p);
+            l[2 * i + o] = w2(fma2(q, sc.s, -p));
+        }
+    }
+    __builtin_memcpy(&B[0], e, 16);
+    __builtin_memcpy(&B[1], l, 16);
 }
 
-// ------------------------------------------------------------------ Q4_K
-// Element i of a block: qs byte 16 + 32(i/64) + i%32, low nibble if i%64 < 32,
-// sub-block i/32 (src/cuda/matmul_q4.cu:76-96). Lane (lr, lk) of stage sb
-// takes elements 32 sb + 8 lk .. +7: qs bytes 16 + 32(sb/2) + 8 lk .. +7,
-// nibble sb%2.
+// Q4_K's min terms, sum_g m_g S_g of a block, as one v_mfma_f32_16x16x16_f16 per tile: k = 8 groups x the two fp16
+// parts of S_g 2^-5 (|S_g| < 2^20) against m_g twice. Lane (lr, lk): groups 2 lk, 2 lk + 1 of token (row) lr.
+__device__ __forceinline__ f16x4_t min_operand(const float2& v) {
+    const float s0 = v.x * 0.03125f, s1 = v.y * 0.03125f;
+    const _Float16 a0 = static_cast<_Float16>(s0), a1 = static_cast<_Float16>(s1);
+    return f16x4_t{a0, static_cast<_Float16>(s0 - static_cast<float>(a0)), a1,
+                   static_cast<_Float16>(s1 - static_cast<float>(a1))};
+}
+__device__ __forceinline__ f16x4_t min_weights(const uint4& h, int lk) {
+    const uint32_t sh = 16u * (lk & 1);
+    const uint32_t l = (h.z >> sh) & 0x3f3fu;
+    const uint32_t g = ((h.w >> (sh + 4)) & 0x0f0fu) | ((h.z >> (sh + 2)) & 0x3030u);
+    const uint32_t m = lk < 2 ? l : g;
+    const f16x2_t p = h2(((m & 0xffu) | ((m >> 8) << 16)) + 0x64006400u) - dup2(1024.f);   // exact
+    return f16x4_t{p[0], p[0], p[1], p[1]};
+}
+
+// The same form with the block's scales in the place of its minima.
+__device__ __forceinline__ f16x4_t scale_weights(const uint4& h, int lk) {
+    const uint32_t sh = 16u * (lk & 1);
+    const uint32_t l = (h.y >> sh) & 0x3f3fu;
+    const uint32_t g = ((h.w >> sh) & 0x0f0fu) | ((h.y >> (sh + 2)) & 0x3030u);
+    const uint32_t m = lk < 2 ? l : g;
+    const f16x2_t p = h2(((m & 0xffu) | ((m >> 8) << 16)) + 0x64006400u) - dup2(1024.f);   // exact
+    return f16x4_t{p[0], p[0], p[1], p[1]};
+}
+
+// A workgroup of 8 waves: RW row groups x KW slices of K (RW = 8 / KW); a wave owns 16 WT tokens x 16 WR rows of
+// its slice's blocks, as 16 x 16 tiles on v_mfma_f32_16x16x32_f16. A step is two depths (64 elements) of every
+// slice. x goes global -> VGPR -> LDS, four step slots deep: step st writes st + 2's fragments (loaded two steps
+// earlier), requests st + 4's and reads its own, the next two token tiles' A operands always requested ahead, so
+// the one barrier per step finds the first operands of the next step in registers. Weights: a lane loads its share
+// of the next block during the current one and decodes it in registers (9 VALU instructions per Q4_K operand of 8
+// quants), so no weight passes through LDS and no wave waits for another's decode. A block's products sum into C
+// from zero; its epilogue applies the block scales in fp32: Q4_K acc += d C - 32 dmin P_min (P_min above); Q6_K
+// acc += d C, with three products per depth, h Bh + l Bh + h Bl (l Bl is below 2^-22 of h Bh).
 //
-// A workgroup (8 waves, one per CU) owns 128 tokens x 256 weight rows; wave w
-// owns rows 64 (w % 4) .. +63 for tokens 64 (w / 4) .. +63. Its operands come
-// through an LDS ring filled by global_load_lds_dwordx4 (no VGPRs, no LDS store
-// instructions) kQ4Dist stages ahead: x per stage, the quant bytes per pair of
-// stages (both nibbles), the headers and group sums per block. While stage g's
-// products run, waves w and w + 4 (same rows) each decode two of the four row
-// tiles of stage g + 1's B operands into an LDS slot that both read after the
-// stage's barrier, so the decode's VALU work hides under the matrix cores.
-constexpr int kQ4Waves = 8;
-constexpr int kQ4Block = kQ4Waves * kWave;
-constexpr int kQ4T = 128;                   // tokens per workgroup
-constexpr int kQ4Dist = 3;                  // ring distance (stages)
-constexpr int kQ4XSlots = 4;                // x slots (one stage each)
-constexpr int kQ4QSlots = 2;                // quant slots (one pair of stages each)
-typedef uint16_t Q4XSlot[2][kQ4T][32];      // one stage of x: [fp16 part][token][k], 16-byte chunks swizzled
-typedef uint8_t Q4QSlot[kGR][32];           // one pair's quant bytes
-typedef uint8_t Q4HSlot[kGR][16];           // one block's headers (d, dmin, scales)
-typedef float Q4SSlot[kQ4T][8];             // one block's group sums
-typedef f16x8_t Q4BSlot[4][4][kWave];       // B operands: [row group][row tile][lane]
+// The sums are over SL slices of K, each in block order, added in slice order: a wave that holds two slices
+// (SL = 2 KW) puts the first one's sums by in LDS. So the bits do not depend on KW, WT or WR, and the shape is free
+// to follow the launch: at 77 tokens and M = 12352 the 48 x 128 tile (KW = 2, two token blocks, 194 workgroups)
+// takes 26 us where 64 x 256 tiles (98 workgroups, the whole of K serially) take 44.
+//
+// What bounds it: issue. A SIMD's MFMAs, the VALU work of decode and epilogue, LDS reads and the CU's vector
+// loads add up rather than overlap (each one's removal took off its own time: of 55 us at 64 x 256, weight loads
+// 7, x 8, A operands 8, decode 13); a round of one workgroup per CU is 12-46 us whatever its MFMA work, so the
+// rounds are what the shape has to save.
+template <int TYPE, int WT, int WR, int KW, int SL>
+struct GemmShape {
+    static constexpr int RW = 8 / KW, FR = WT * KW * 4, XF = FR / 8, SPW = SL / KW;
+    static constexpr int tokens = 16 * WT, rows = 16 * WR * RW;
+    static constexpr size_t ring = size_t{4} * FR * 1024, fold = KW > 1 ? size_t{8} * SPW * WT * WR * 1024 : 0;
+    static constexpr size_t kept = SPW == 2 ? size_t{8} * WT * WR * 1024 : 0;
+    static constexpr size_t lds = ring + kept > fold ? ring + kept : fold;
+    static_assert(FR % 8 == 0 && SPW >= 1 && SPW <= 2 && (KW > 1 || SPW == SL), "shape");
+};
+
+// A value the compiler may not fold into its users (keeps v_fmac_f32 from
+// becoming v_fma_mix_f32, which issues at half the rate).
+__device__ __forceinline__ float opaque(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
 
 template <int S>
 using IC = std::integral_constant<int, S>;
@@ -261,12 +469,454 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-// A value the compiler may not fold into its users (keeps v_fmac_f32 from
-// becoming v_fma_mix_f32, which issues at half the rate).
-__device__ __forceinline__ float opaque(float v) {
-    asm volatile("" : "+v"(v));
-    return v;
+template <int TYPE, int WT, int WR, int KW, int SL>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kquant(
+    const GemmJobs jobs, const int* __restrict__ ex, const float* __restrict__ sx, const uint8_t* __restrict__ xp,
+    const float* __restrict__ x, int T, int K) {
+    using G = GemmShape<TYPE, WT, WR, KW, SL>;
+    constexpr int BB = TYPE == kQ4_K ? 144 : 210, NB = TYPE == kQ4_K ? 1 : 2;
+    __shared__ __align__(16) uint8_t smem[G::lds];
+    uint4* xs = reinterpret_cast<uint4*>(smem);
+    const int cols = jobs.start[jobs.n];
+    const int tb = static_cast<int>(blockIdx.x) / cols;
+    const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x) - tb * cols);
+    float* __restrict__ y = job.y;
+    const int M = job.M;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = wave_in_block();
+    const int kw = wv / G::RW, rw = wv % G::RW;
+    const int nb = K >> 8, nbk = nb / KW, steps = 4 * nbk, nst = K >> 5;
+    const int tile0 = tb * WT, tiles = (T + kTile - 1) / kTile;
+    const int rw0 = job.mb * G::rows, r0 = rw0 + 16 * WR * rw;
+    const uint8_t* wbase = job.w + (job.ub0 + static_cast<uint64_t>(rw0) * nb + static_cast<uint64_t>(kw) * nbk) * BB;
+    uint32_t wo[WR];   // the lane's row, from the workgroup's first
+#pragma unroll
+    for (int rt = 0; rt < WR; ++rt)
+        wo[rt] = static_cast<uint32_t>(min(r0 + 16 * rt + lr, M - 1) - rw0) * static_cast<uint32_t>(nb) * BB;
+
+    // this wave's fragments of a step: fragment id -> (slice, tile of the workgroup, (depth, part))
+    const uint8_t* xb[G::XF];
+    uint32_t xo[G::XF], xstep[G::XF];
+#pragma unroll
+    for (int i = 0; i < G::XF; ++i) {
+        const int id = wv * G::XF + i;
+        const int ti = min(tile0 + id / 4 % WT, tiles - 1), ks = id / (4 * WT);
+        const int r = min(kTile, T - kTile * ti);
+        xb[i] = xp + tile_base(ti, K);
+        xo[i] = 16u * static_cast<uint32_t>((ks * nbk * 16 + id % 4) * 4 * r + lk * r + min(lr, r - 1));
+        xstep[i] = 256u * r;
+    }
+    uint4 xr[2][G::XF];
+    auto x_load = [&](uint4 (&d)[G::XF], int st) {
+#pragma unroll
+        for (int i = 0; i < G::XF; ++i) d[i] = ld16(xb[i] + (xo[i] + static_cast<uint32_t>(min(st, steps - 1)) * xstep[i]));
+    };
+    auto x_store = [&](const uint4 (&d)[G::XF], int slot) {
+#pragma unroll
+        for (int i = 0; i < G::XF; ++i) xs[(slot * G::FR + wv * G::XF + i) * 64 + lane] = d[i];
+    };
+    const uint4* as = xs + kw * WT * 4 * 64 + lane;   // this wave's first A fragment of slot 0
+    constexpr int PT = WT < 2 ? WT : 2;   // token tiles whose A operands are requested at a time
+    f16x8_t An[PT][2];
+    auto a_load = [&](f16x8_t (&d)[PT][2], int slot, int j, int t0) {
+#pragma unroll
+        for (int i = 0; i < PT; ++i)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                d[i][p] = *reinterpret_cast<const f16x8_t*>(&as[(slot * G::FR + 4 * min(t0 + i, WT - 1) + 2 * j + p) * 64]);
+    };
+    auto barrier = []() {   // this wave's LDS stores are done, then the workgroup meets (loads stay in flight)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    f32x4_t acc[WT][WR], C[WT][WR];
+#pragma unroll
+    for (int tt = 0; tt < WT; ++tt)
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) acc[tt][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    uint32_t k64 = 0x64006400u;   // kept in a register: v_and_or_b32 takes one constant
+    asm volatile("" : "+v"(k64));
+    WBlock<TYPE> wc[WR], wn[WR];
+    WScale<TYPE> sc[WR];
+    f16x8_t B[2][WR][NB];
+    auto w_load = [&](int b) {   // the lane's share of block b of its rows (the last block again past the end)
+        const uint8_t* p = wbase + static_cast<size_t>(min(b, nbk - 1)) * BB;
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) wn[rt].load(p, wo[rt], lk);
+    };
+    auto w_take = [&]() {
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) wc[rt] = wn[rt];
+    };
+    auto b_make = [&](auto dI) {   // B operands of depth D of the block in wc
+        constexpr int D = decltype(dI)::value;
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) {
+            if constexpr ((D & 1) == 0) sc[rt].template set<(D >> 1)>(wc[rt], lk);
+            decode<(D >> 1), (D & 1)>(wc[rt], sc[rt], k64, B[D & 1][rt]);
+        }
+    };
+    w_load(0);
+    x_load(xr[0], 0);
+    x_load(xr[1], 1);
+    w_take();
+    w_load(1);
+    x_store(xr[0], 0);
+    x_load(xr[0], 2);
+    x_store(xr[1], 1);
+    x_load(xr[1], 3);
+    b_make(IC<0>{});
+    barrier();
+    a_load(An, 0, 0, 0);
+
+    f32x4_t* kept = reinterpret_cast<f32x4_t*>(smem + G::ring) + wv * WT * WR * 64 + lane;   // the first slice's sums
+    for (int b = 0; b < nbk; ++b) {
+        if (G::SPW == 2 && b == nbk / 2) {
+#pragma unroll
+            for (int tt = 0; tt < WT; ++tt)
+#pragma unroll
+                for (int rt = 0; rt < WR; ++rt) {
+                    kept[(tt * WR + rt) * 64] = acc[tt][rt];
+                    acc[tt][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        // the block's epilogue operands
+        f16x4_t Bm[WR];
+        float dsc[WR], dmn[WR];
+        float2 sg[WT];
+        if constexpr (TYPE == kQ4_K) {
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) {
+                Bm[rt] = min_weights(wc[rt].hd, lk);
+                dsc[rt] = opaque(half_bits(wc[rt].hd.x & 0xffffu));
+                dmn[rt] = opaque(-32.0f * half_bits(wc[rt].hd.x >> 16));
+            }
+#pragma unroll
+            for (int tt = 0; tt < WT; ++tt) {   // group sums 2 lk, 2 lk + 1 of token lr
+                const int t = min((tile0 + tt) * kTile + lr, T - 1);
+                sg[tt] = *reinterpret_cast<const float2*>(sx + static_cast<size_t>(t) * nst + 8 * (kw * nbk + b) + 2 * lk);
+            }
+        } else {
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) dsc[rt] = opaque(half_bits(wc[rt].d));
+        }
+        static_for<8>([&](auto dI) {
+            constexpr int D = decltype(dI)::value, U = D >> 1, J = D & 1;
+            const int st = 4 * b + U;
+            if constexpr (D == 7) {
+                w_take();
+                w_load(b + 2);
+            }
+            if constexpr (J == 0) {
+                x_store(xr[U & 1], (U + 2) & 3);
+                x_load(xr[U & 1], st + 4);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            b_make(IC<(D + 1) & 7>{});
+            static_for<(WT + 1) / 2>([&](auto pI) {   // pairs of token tiles
+                constexpr int P0 = 2 * decltype(pI)::value, PN = P0 + 2 <= WT ? 2 : 1;
+                f16x8_t A[2][2];
+#pragma unroll
+                for (int i = 0; i < PN; ++i) {
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) A[i][p] = An[i][p];
+                }
+                if constexpr (P0 + 2 < WT)
+                    a_load(An, U, J, P0 + 2);
+                else
+                    a_load(An, J == 0 ? U : (U + 1) & 3, J ^ 1, 0);
+#pragma unroll
+                for (int i = 0; i < PN; ++i)
+#pragma unroll
+                    for (int rt = 0; rt < WR; ++rt)   // a block's first depth starts its sums from zero
+                        C[P0 + i][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            A[i][0], B[J][rt][0], D == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : C[P0 + i][rt], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < PN; ++i)
+#pragma unroll
+                    for (int rt = 0; rt < WR; ++rt)
+                        C[P0 + i][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[i][1], B[J][rt][0], C[P0 + i][rt], 0, 0, 0);
+                if constexpr (NB == 2) {
+#pragma unroll
+                    for (int i = 0; i < PN; ++i)
+#pragma unroll
+                        for (int rt = 0; rt < WR; ++rt)
+                            C[P0 + i][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[i][0], B[J][rt][NB - 1], C[P0 + i][rt], 0, 0, 0);
+                }
+#pragma unroll
+                for (int tt = P0; D == 7 && tt < P0 + PN; ++tt) {
+                    f16x4_t As;
+                    if constexpr (TYPE == kQ4_K) As = min_operand(sg[tt]);
+#pragma unroll
+                    for (int rt = 0; rt < WR; ++rt) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[tt][rt][i] = __builtin_fmaf(dsc[rt], C[tt][rt][i], acc[tt][rt][i]);
+                        if constexpr (TYPE == kQ4_K) {
+                            const f32x4_t pm =
+                                __builtin_amdgcn_mfma_f32_16x16x16f16(As, Bm[rt], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[tt][rt][i] = __builtin_fmaf(dmn[rt], pm[i], acc[tt][rt][i]);
+                        }
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (J == 1) barrier();
+        });
+    }
+
+    // lane L holds elements [4 (L / 16) + i][L % 16] of tile (tt, rt): token 4 lk + i, row lr
+    auto put = [&](int tt, int rt, const f32x4_t& v) {
+        const int row = r0 + 16 * rt + lr;
+        if (row >= M) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = (tile0 + tt) * kTile + 4 * lk + i;
+            if (t >= T) continue;
+            const int et = ex[t];
+            y[static_cast<size_t>(t) * M + row] =
+                et == kRowNonFinite ? row_dot_per_element(job.w, TYPE, (job.ub0 + static_cast<uint64_t>(row) * nb) * 256,
+                                                          x + static_cast<size_t>(t) * K, K)
+                                    : ldexpf(v[i], -et);
+        }
+    };
+    if constexpr (KW == 1) {
+#pragma unroll
+        for (int tt = 0; tt < WT; ++tt)
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) put(tt, rt, G::SPW == 2 ? kept[(tt * WR + rt) * 64] + acc[tt][rt] : acc[tt][rt]);
+    } else {   // every slice's sums to LDS; wave kw of a row group adds the tiles tt * WR + rt = kw (mod KW)
+        f32x4_t* part = reinterpret_cast<f32x4_t*>(smem);   // the ring and the kept sums are done with
+        constexpr int tiles_w = WT * WR;
+        auto at = [&](int slice, int tile) { return ((slice * G::RW + rw) * tiles_w + tile) * 64 + lane; };
+        f32x4_t first[G::SPW == 2 ? tiles_w : 1];
+        if constexpr (G::SPW == 2) {
+#pragma unroll
+            for (int i = 0; i < tiles_w; ++i) first[i] = kept[i * 64];
+            barrier();
+        }
+#pragma unroll
+        for (int tt = 0; tt < WT; ++tt)
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) {
+                if constexpr (G::SPW == 2) part[at(2 * kw, tt * WR + rt)] = first[tt * WR + rt];
+                part[at(G::SPW * kw + G::SPW - 1, tt * WR + rt)] = acc[tt][rt];
+            }
+        barrier();
+#pragma unroll
+        for (int tt = 0; tt < WT; ++tt)
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) {
+                if ((tt * WR + rt) % KW != kw) continue;
+                f32x4_t v = part[at(0, tt * WR + rt)];
+#pragma unroll
+                for (int sl = 1; sl < SL; ++sl) v += part[at(sl, tt * WR + rt)];
+                put(tt, rt, v);
+            }
+    }
 }
+
+// ------------------------------------------------------------------ a few tokens
+// Up to 16 tokens per workgroup and no prep pass (nor workspace): the workgroup converts its tokens' rows itself,
+// 2048 elements of K (a round: 8 blocks) at a time, into an LDS image of the fragments (slot lr ^ c of its 16,
+// c = 4 u + 2 (lk % 2) + j, so that neither the stores nor the loads conflict), with one exponent per token and
+// round. Wave w takes block w of every round for the workgroup's 16 WR rows; its first block's weights are
+// requested before the conversion. A round's sums are unscaled (exactly) and added to the wave's totals, and the
+// 8 waves' totals are added in wave order through LDS.
+//
+// These counts were one fp32 GEMV per token before, so the sums are kept to its accuracy (relative errors against
+// 64 bits at K = 2048 / 4096: GEMV Q4_K 1.8e-7, Q6_K 1.6e-7): the products of x's low parts, 2^-11 of the others,
+// have an accumulator of their own, and Q4_K's quants enter as q - 8, so that a block's sum is no larger than its
+// result; the 8 d sum_g sc_g S_g taken out joins the min terms in fp32.
+template <int TYPE, int WR>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_few(
+    const GemmJobs jobs, const float* __restrict__ x, int T, int K) {
+    constexpr int BB = TYPE == kQ4_K ? 144 : 210, NB = TYPE == kQ4_K ? 1 : 2;
+    __shared__ __align__(16) uint4 xs[8 * 8 * 2 * 64];
+    __shared__ __align__(16) float sums[16][64];
+    __shared__ int exps[16], bad[16];
+    const int cols = jobs.start[jobs.n];
+    const int tb = static_cast<int>(blockIdx.x) / cols;
+    const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x) - tb * cols);
+    float* __restrict__ y = job.y;
+    const int M = job.M, t0 = tb * kTile;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = wave_in_block();
+    const int nb = K >> 8, rounds = (nb + 7) >> 3;
+    const int r0 = job.mb * 16 * WR;
+    const uint8_t* wbase = job.w + (job.ub0 + static_cast<uint64_t>(r0) * nb) * BB;
+    uint32_t wo[WR];
+#pragma unroll
+    for (int rt = 0; rt < WR; ++rt)
+        wo[rt] = static_cast<uint32_t>(min(16 * rt + lr, M - 1 - r0)) * static_cast<uint32_t>(nb) * BB;
+    [[maybe_unused]] uint32_t k64 = 0x64006400u;   // kept in a register: v_and_or_b32 takes one constant
+    asm volatile("" : "+v"(k64));
+    WBlock<TYPE> wc[WR];
+    auto w_load = [&](int b) {
+        const uint8_t* p = wbase + static_cast<size_t>(min(b, nb - 1)) * BB;
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) wc[rt].load(p, wo[rt], lk);
+    };
+    // conversion: 32 threads per token, 8 pieces of 8 elements each
+    const int tok = tid >> 5, ch0 = tid & 31;
+    const bool live = t0 + tok < T;
+    const float* row = x + static_cast<size_t>(live ? t0 + tok : 0) * K;
+    float4 v[16];
+    auto x_load = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int k = 2048 * c + 256 * i + 8 * ch0;
+            const bool in = live && k < K;
+            v[2 * i] = in ? ld4(row + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[2 * i + 1] = in ? ld4(row + k + 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    x_load(0);
+    w_load(wv);
+    if (tid < 16) bad[tid] = 0;
+
+    f32x4_t tot[WR];
+#pragma unroll
+    for (int rt = 0; rt < WR; ++rt) tot[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < rounds; ++c) {
+        __syncthreads();   // the previous round's fragments have been read
+        {
+            float m = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m = max_abs4(m, v[i]);
+#pragma unroll
+            for (int o = 16; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+            const int e = prep_exponent(m);
+            if (ch0 == 0) {
+                exps[tok] = e == kRowNonFinite ? 0 : e;
+                if (e == kRowNonFinite) bad[tok] = 1;   // evaluated per element at the end
+            }
+            const int es = e == kRowNonFinite ? 0 : e;
+            const int c16 = ch0 & 15;                                   // 4 u + 2 (lk % 2) + j
+            const int dep = 2 * (c16 >> 2) + (c16 & 1), k4 = 2 * (ch0 >> 4) + ((c16 >> 1) & 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint32_t h[4], l[4];
+                const float s0 = split8(v[2 * i], v[2 * i + 1], es, h, l);
+                const int slot = ((i * 8 + dep) * 2 * 4 + k4) * 16 + (tok ^ c16);
+                xs[slot] = make_uint4(h[0], h[1], h[2], h[3]);
+                xs[slot + 64] = make_uint4(l[0], l[1], l[2], l[3]);
+                float s = s0 + __shfl_xor(s0, 1);
+                s += __shfl_xor(s, 2);
+                if ((ch0 & 3) == 0) sums[tok][8 * i + (ch0 >> 2)] = s;
+            }
+        }
+        if (c + 1 < rounds) x_load(c + 1);
+        __syncthreads();
+        if (8 * c + wv >= nb) continue;   // the whole wave; the next barrier is met at the loop's head
+        f32x4_t C[WR], Cl[WR];
+        WScale<TYPE> sc[WR];
+        const uint4* xw = xs + wv * 8 * 2 * 64 + lk * 16;
+        const int sw = lr ^ (2 * (lk & 1));
+        f16x8_t A[2][2];
+        auto a_load = [&](auto dI) {
+            constexpr int D = decltype(dI)::value;
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                A[D & 1][p] = *reinterpret_cast<const f16x8_t*>(&xw[(2 * D + p) * 64 + (sw ^ (4 * (D >> 1) + (D & 1)))]);
+        };
+        a_load(IC<0>{});
+        static_for<8>([&](auto dI) {
+            constexpr int D = decltype(dI)::value, U = D >> 1, J = D & 1;
+            if constexpr (D < 7) a_load(IC<D + 1>{});
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) {
+                if constexpr (J == 0) {
+                    if constexpr (TYPE == kQ4_K)
+                        sc[rt].template set_centred<U>(wc[rt], lk);
+                    else
+                        sc[rt].template set<U>(wc[rt], lk);
+                }
+                f16x8_t B[NB];
+                if constexpr (TYPE == kQ4_K)
+                    decode_centred<U, J>(wc[rt], sc[rt], B);
+                else
+                    decode<U, J>(wc[rt], sc[rt], k64, B);
+                const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+                C[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[J][0], B[0], D == 0 ? zero : C[rt], 0, 0, 0);
+                Cl[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[J][1], B[0], D == 0 ? zero : Cl[rt], 0, 0, 0);
+                if constexpr (NB == 2) Cl[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[J][0], B[NB - 1], Cl[rt], 0, 0, 0);
+            }
+        });
+        f16x4_t As;
+        if constexpr (TYPE == kQ4_K) As = min_operand(*reinterpret_cast<const float2*>(&sums[lr][8 * wv + 2 * lk]));
+        int et[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) et[i] = -exps[4 * lk + i];
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) {
+            float d, d8 = 0.f, dmn = 0.f;
+            f32x4_t pm, ps;
+            if constexpr (TYPE == kQ4_K) {
+                d = half_bits(wc[rt].hd.x & 0xffffu);
+                d8 = 256.0f * d;   // 8 d, and the 2^5 of S 2^-5
+                dmn = -32.0f * half_bits(wc[rt].hd.x >> 16);
+                const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+                pm = __builtin_amdgcn_mfma_f32_16x16x16f16(As, min_weights(wc[rt].hd, lk), zero, 0, 0, 0);
+                ps = __builtin_amdgcn_mfma_f32_16x16x16f16(As, scale_weights(wc[rt].hd, lk), zero, 0, 0, 0);
+            } else {
+                d = half_bits(wc[rt].d);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float s = d * (C[rt][i] + Cl[rt][i]);
+                if constexpr (TYPE == kQ4_K) s += __builtin_fmaf(d8, ps[i], dmn * pm[i]);
+                tot[rt][i] += ldexpf(s, et[i]);
+            }
+        }
+        if (c + 1 < rounds) w_load(8 * (c + 1) + wv);
+    }
+    __syncthreads();
+    f32x4_t* part = reinterpret_cast<f32x4_t*>(xs);
+#pragma unroll
+    for (int rt = 0; rt < WR; ++rt) part[(wv * WR + rt) * 64 + lane] = tot[rt];
+    __syncthreads();
+    if (wv >= WR) return;
+    f32x4_t s = part[wv * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) s += part[(w * WR + wv) * 64 + lane];
+    const int mrow = r0 + 16 * wv + lr;
+    if (mrow >= M) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int t = t0 + 4 * lk + i;
+        if (t >= T) continue;
+        y[static_cast<size_t>(t) * M + mrow] =
+            bad[4 * lk + i] ? row_dot_per_element(job.w, TYPE, (job.ub0 + static_cast<uint64_t>(mrow) * nb) * 256,
+                                                  x + static_cast<size_t>(t) * K, K)
+                            : s[i];
+    }
+}
+
+// ------------------------------------------------------------------ Q4_K, many tokens
+// A workgroup (8 waves, one per CU) owns 128 tokens x 256 weight rows; wave w owns rows 64 (w % 4) .. +63 for
+// tokens 64 (w / 4) .. +63, as 4 x 4 tiles. Operands arrive through an LDS ring filled by global_load_lds_dwordx4
+// (no VGPRs, no LDS store instructions) kQ4Dist depths ahead: x fragments per depth, the quant bytes per half
+// block (the 16-byte pieces of depths u = 2 g, 2 g + 1, row by row, which is also the order of a wave's B reads:
+// no bank conflicts), headers and group sums per block. Each wave decodes the B operands of its own 64 rows in
+// registers, a depth ahead, 9 VALU instructions per operand, and requests the next token tile's A operands before
+// the current one's products; each MFMA is followed by two VALU instructions of the decode (the scheduling groups),
+// which issue while it runs. Measured at 4096 x 8192 x 2048 and the other three projections, six rounds of 256
+// workgroups: 370 us, 230 of them the MFMAs' own time; with the decode shared by wave pairs through LDS (24 VALU instructions
+// per operand then) and no A operands ahead 437 us. Without its decode, DMA, A reads or epilogue it takes 72, 54,
+// 60 and 37 us less: the parts add up, so fewer instructions is what is left to gain.
+constexpr int kQ4Waves = 8;
+constexpr int kQ4Block = kQ4Waves * kWave;
+constexpr int kQ4R = 256;                   // weight rows per workgroup (64 per wave)
+constexpr int kQ4T = 128;                   // tokens per workgroup
+constexpr int kQ4Dist = 3;                  // ring distance (depths)
+constexpr int kQ4XSlots = 4;                // x slots (one depth each)
+typedef uint4 Q4XSlot[kQ4T / kTile][2][kWave];   // one depth of x: [tile][fp16 part][lane]
+typedef uint4 Q4QSlot[kQ4R][4];             // one half block's quant bytes: [row][lk]
+typedef uint8_t Q4HSlot[kQ4R][16];          // one block's headers (d, dmin, scales)
+typedef float Q4SSlot[kQ4T][8];             // one block's group sums
 
 // 16 bytes per lane global -> LDS (m0 + 16 lane). As inline assembly the
 // compiler neither counts these loads nor waits for them; the kernel waits on
@@ -282,50 +932,50 @@ __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
 }
 
-// This wave's loads in ring group j: 2 (x) + 1 (a pair's quant bytes, even j) +
-// 2 (headers and group sums, a block's first stage).
+// This wave's loads in ring group j: 2 (x) + 2 (a half block's quant bytes, j % 4 == 0) +
+// 2 (headers and group sums, a block's first depth).
 __host__ __device__ constexpr int q4_group_loads(int j) {
-    return 2 + ((j & 1) == 0 ? 1 : 0) + ((j & 7) == 0 ? 2 : 0);
+    return 2 + ((j & 3) == 0 ? 2 : 0) + ((j & 7) == 0 ? 2 : 0);
 }
 
-__global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, const int* __restrict__ ex,
-                                                         const float* __restrict__ sx, const uint16_t* __restrict__ xp,
-                                                         const float* __restrict__ x, int T, int K) {
+__global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k_wide(const GemmJobs jobs, const int* __restrict__ ex,
+                                                              const float* __restrict__ sx, const uint8_t* __restrict__ xp,
+                                                              const float* __restrict__ x, int T, int K) {
     __shared__ __align__(16) Q4XSlot xr[kQ4XSlots];
-    __shared__ __align__(16) Q4QSlot qr[kQ4QSlots];
+    __shared__ __align__(16) Q4QSlot qr[2];
     __shared__ __align__(16) Q4HSlot hr[2];
     __shared__ __align__(16) Q4SSlot sr[2];
-    __shared__ __align__(16) Q4BSlot bs[2];
-    const GemmJob job = gemm_job(jobs);
+    const int cols = jobs.start[jobs.n];
+    const int tb = static_cast<int>(blockIdx.x) / cols;
+    const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x) - tb * cols);
     const uint8_t* __restrict__ w = job.w;
     float* __restrict__ y = job.y;
     const int M = job.M;
     const uint64_t ub0 = job.ub0;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
+    const int lane = threadIdx.x & 63;
+    const int wv = wave_in_block();
     const int rg = wv & 3, th = wv >> 2;                       // row group, token half
-    const int t0w = blockIdx.y * kQ4T;                         // the workgroup's first token
+    const int t0w = tb * kQ4T;                                 // the workgroup's first token
     const int tw = t0w + 64 * th;                              // this wave's first token
-    const int rw0 = job.mb * kGR;                              // the workgroup's first row
+    const int rw0 = job.mb * kQ4R;                             // the workgroup's first row
     const int r0 = rw0 + 64 * rg;                              // this wave's first row
     const int nb = K >> 8, nst = K >> 5;
     const int lr = lane & 15, lk = lane >> 4;
     const uint8_t* wbase = w + ub0 * 144;
-    const uint8_t* xpb = reinterpret_cast<const uint8_t*>(xp);
-    // Ring loads of a wave (byte offsets; stage and block offsets go into the
-    // scalar base). x: part wv / 4, tokens 32 (wv % 4) + 16 i + lane / 4 (i < 2);
-    // the lane at chunk c of its token's 64 bytes loads chunk c ^ ((token / 4) % 4),
-    // which spreads the A reads over the LDS banks. Quant bytes: rows 32 wv + lane / 2.
-    // Headers: rows 64 (wv % 4) + lane; group sums: tokens 32 (wv % 4) + lane / 2
-    // (waves 4-7 repeat 0-3: the same bytes to the same place).
-    const int xtk0 = 32 * (wv & 3);
-    auto xoff = [&](int i) {
-        const int tk = xtk0 + 16 * i + (lane >> 2);
-        const int ch = (lane & 3) ^ ((tk >> 2) & 3);
-        return 2u * (static_cast<uint32_t>(min(t0w + tk, T - 1)) * static_cast<uint32_t>(nst) * 64u + 32u * (wv >> 2) + 8u * ch);
+    // Ring loads of a wave (byte offsets; depth and block offsets go into the scalar base). x: tile wv of the
+    // workgroup (its last one again past the end), both parts. Quant bytes: rows 32 wv + 16 i + lane / 4, piece
+    // lane % 4. Headers: rows 64 (wv % 4) + lane; group sums: tokens 32 (wv % 4) + lane / 2 (waves 4-7 repeat
+    // 0-3: the same bytes to the same place).
+    const int xt = min(tb * (kQ4T / kTile) + wv, (T + kTile - 1) / kTile - 1);
+    const int xrn = min(kTile, T - kTile * xt);
+    const uint8_t* xbase = xp + tile_base(xt, K);
+    const uint32_t xo = 16u * static_cast<uint32_t>(lk * xrn + min(lr, xrn - 1));
+    const uint32_t xpart = 64u * xrn;   // bytes of one part of one depth
+    auto qo = [&](int i) {
+        const int row = min(rw0 + 32 * wv + 16 * i + (lane >> 2), M - 1), pc = lane & 3;
+        return static_cast<uint32_t>(row) * static_cast<uint32_t>(nb) * 144u + 16u + 64u * (pc >> 1) + 16u * (pc & 1);
     };
-    const uint32_t qo = static_cast<uint32_t>(min(rw0 + 32 * wv + (lane >> 1), M - 1)) * static_cast<uint32_t>(nb) * 144u + 16u +
-                        16u * (lane & 1);
+    const uint32_t qo0 = qo(0), qo1 = qo(1);
     const uint32_t ho = static_cast<uint32_t>(min(r0 + lane, M - 1)) * static_cast<uint32_t>(nb) * 144u;
     const uint32_t so = 4u * (static_cast<uint32_t>(min(t0w + 32 * rg + (lane >> 1), T - 1)) * static_cast<uint32_t>(nst) +
                               4u * (lane & 1));
@@ -333,58 +983,61 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, con
         return __builtin_amdgcn_readfirstlane(
             static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const void __attribute__((address_space(3)))*)(l))));
     };
-    const uint32_t xr_a = lds_addr(&xr[0][0][0][0]), qr_a = lds_addr(&qr[0][0][0]), hr_a = lds_addr(&hr[0][0][0]),
-                   sr_a = lds_addr(&sr[0][0][0]);
-    // ring group gs, in 4 parts: x (2 halves), the pair's quant bytes (even gs),
-    // the block's headers and group sums (its first stage)
-    auto issue_part = [&](int gs, int part) {
+    const uint32_t xr_a = lds_addr(&xr[0][wv][0][0]), qr_a = lds_addr(&qr[0][32 * wv][0]), hr_a = lds_addr(&hr[0][64 * rg][0]),
+                   sr_a = lds_addr(&sr[0][32 * rg][0]);
+    // ring group gs, in 4 parts: x (2), the half block's quant bytes, the block's headers and group sums
+    auto issue_part = [&](int gs, int part) {   // past the last depth: the last group again, into slots not read any more
+        const int ge = min(gs, nst - 1), gb = min(gs >> 3, nb - 1);
         if (part < 2) {
-            dma16(xoff(part), xpb + static_cast<size_t>(gs) * 128,
-                  xr_a + static_cast<uint32_t>(gs % kQ4XSlots) * sizeof(Q4XSlot) + ((wv >> 2) * kQ4T + xtk0 + 16 * part) * 64u);
+            dma16(xo, xbase + static_cast<size_t>(2 * ge + part) * xpart,
+                  xr_a + static_cast<uint32_t>(gs % kQ4XSlots) * sizeof(Q4XSlot) + 1024u * part);
         } else if (part == 2) {
-            if ((gs & 1) == 0)
-                dma16(qo, wbase + static_cast<size_t>(gs >> 3) * 144 + 32 * ((gs & 7) >> 1),
-                      qr_a + static_cast<uint32_t>((gs >> 1) % kQ4QSlots) * sizeof(Q4QSlot) + 32u * wv * 32u);
+            if ((gs & 3) == 0) {
+                const uint8_t* b = wbase + static_cast<size_t>(gb) * 144 + 32 * ((gs >> 2) & 1);
+                const uint32_t l = qr_a + static_cast<uint32_t>((gs >> 2) & 1) * sizeof(Q4QSlot);
+                dma16(qo0, b, l);
+                dma16(qo1, b, l + 1024u);
+            }
         } else if ((gs & 7) == 0) {
             const uint32_t hb = (gs >> 3) & 1;
-            dma16(ho, wbase + static_cast<size_t>(gs >> 3) * 144, hr_a + hb * sizeof(Q4HSlot) + 64u * rg * 16u);
-            dma16(so, sx + gs, sr_a + hb * sizeof(Q4SSlot) + 32u * rg * 32u);
+            dma16(ho, wbase + static_cast<size_t>(gb) * 144, hr_a + hb * sizeof(Q4HSlot));
+            dma16(so, sx + 8 * gb, sr_a + hb * sizeof(Q4SSlot));
         }
     };
-    // B operand of row tile rt of stage gs (scale group SB of its block)
-    auto decode_rt = [&](auto sbI, int gs, int rt) {
-        constexpr int SB = decltype(sbI)::value;
-        const int qs = (gs >> 1) % kQ4QSlots, hb = (gs >> 3) & 1;
-        const uint32_t* hw = reinterpret_cast<const uint32_t*>(&hr[hb][64 * rg + 16 * rt + lr][0]);
-        uint32_t sc;   // scale_min_k4 (src/cuda/matmul_q4.cu:18-26), scale part
-        if constexpr (SB < 4)
-            sc = (hw[1] >> (8 * SB)) & 63u;
-        else
-            sc = ((hw[3] >> (8 * (SB - 4))) & 15u) | (((hw[1] >> (8 * (SB - 4) + 6)) & 3u) << 4);
-        const uint2 qb = *reinterpret_cast<const uint2*>(&qr[qs][64 * rg + 16 * rt + lr][8 * lk]);
-        const uint32_t n0 = ((SB & 1) ? (qb.x >> 4) : qb.x) & 0x0f0f0f0fu;
-        const uint32_t n1 = ((SB & 1) ? (qb.y >> 4) : qb.y) & 0x0f0f0f0fu;
-        uint32_t e[4];
-        q4_operand(n0, sc, e[0], e[1]);
-        q4_operand(n1, sc, e[2], e[3]);
-        f16x8_t r;
-        __builtin_memcpy(&r, e, 16);
-        return r;
-    };
-    auto wait_ring = [](int n) {   // at most n of this wave's ring loads in flight
-        switch (n) {
-            case 2: wait_vm<2>(); break;
-            case 3: wait_vm<3>(); break;
-            case 5: wait_vm<5>(); break;
-            default: wait_vm<0>(); break;
-        }
-    };
-    auto barrier = []() {   // LDS stores (the B slot) complete; the ring's loads stay in flight
+    auto barrier = []() {   // the ring's loads stay in flight
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    uint32_t k64 = 0x64006400u;   // kept in a register: v_and_or_b32 takes one constant
+    asm volatile("" : "+v"(k64));
+    // B operands of this wave's rows: q[rt] holds the lane's piece of the current half block, sc[rt] the scales of
+    // the half-block's depths
+    uint4 q[4];
+    uint32_t scb[4];   // the lane's four scale bytes (u = 0..3)
+    f16x8_t B[2][4];
+    auto take_hdr = [&](int blk) {
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) {
+            const uint4 h = *reinterpret_cast<const uint4*>(&hr[blk & 1][64 * rg + 16 * rt + lr][0]);
+            const uint32_t lo = h.y & 0x3f3f3f3fu, hi = (h.w & 0x0f0f0f0fu) | ((h.y >> 2) & 0x30303030u);
+            scb[rt] = lk < 2 ? lo : hi;   // scale_min_k4 (src/cuda/matmul_q4.cu:18-26): groups 4 (lk / 2) + u
+        }
+    };
+    auto take_q = [&](int half) {   // half block index: block 2 * half
+#pragma unroll
+        for (int rt = 0; rt < 4; ++rt) q[rt] = qr[half & 1][64 * rg + 16 * rt + lr][lk];
+    };
+    WScale<kQ4_K> sc[4];
+    auto b_make = [&](auto dI, int rt) {   // B operand rt of depth D of the block
+        constexpr int D = decltype(dI)::value, U = D >> 1, J = D & 1;
+        if constexpr (J == 0) sc[rt].template from<U>((scb[rt] >> (8 * U)) & 0xffu);
+        f16x8_t b1[1];
+        decode_q4<U, J>(q[rt], sc[rt], k64, b1);
+        B[J][rt] = b1[0];
+    };
 
+    f16x8_t An[2];
     f32x4_t acc[4][4], C[4][4];
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)
@@ -392,82 +1045,61 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, con
         for (int rt = 0; rt < 4; ++rt) acc[tt][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     // groups 0 .. kQ4Dist - 1 (nst >= 8); groups 0 and 1 complete
-    {
-        int pend = 0;
-        for (int gs = 0; gs < kQ4Dist; ++gs) {
+    for (int gs = 0; gs < kQ4Dist; ++gs)
 #pragma unroll
-            for (int part = 0; part < 4; ++part) issue_part(gs, part);
-            if (gs >= 2) pend += q4_group_loads(gs);
-        }
-        wait_ring(pend);
-    }
+        for (int part = 0; part < 4; ++part) issue_part(gs, part);
+    wait_vm<q4_group_loads(2)>();
     barrier();
+    take_hdr(0);
+    take_q(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) bs[0][rg][2 * th + i][lane] = decode_rt(IC<0>{}, 0, 2 * th + i);
-    barrier();
+    for (int p = 0; p < 2; ++p) An[p] = *reinterpret_cast<const f16x8_t*>(&xr[0][4 * th][p][lane]);
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) b_make(IC<0>{}, rt);
 
-    // the A operand of lane (lr, lk): token 16 tt + lr, k 8 lk .. + 7 = chunk lk ^ ((lr / 4) % 4)
-    const int ach = 8 * (lk ^ ((lr >> 2) & 3));
-    // the min-term operand of lane (lr, lk): groups 2 lk, 2 lk + 1
-    const bool mlo = lk < 2;
-    const uint32_t msh = 16u * (lk & 1);
     for (int b = 0; b < nb; ++b) {
         const int g0 = 8 * b;
         static_for<8>([&](auto sI) {
             constexpr int S = decltype(sI)::value;
             const int g = g0 + S;
-            const bool iss = g + kQ4Dist < nst;
-            const bool dec = g + 1 < nst;
-            f16x8_t B[4];
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt) B[rt] = bs[S & 1][rg][rt][lane];
-            // the block's epilogue operands (last stage): d, -32 dmin and m_g
+            // the block's epilogue operands (last depth): d, -32 dmin and m_g
             float dsc[4], dmn5[4];
             f16x4_t Bm[4];
             if constexpr (S == 7) {
 #pragma unroll
                 for (int rt = 0; rt < 4; ++rt) {
                     const uint4 h = *reinterpret_cast<const uint4*>(&hr[b & 1][64 * rg + 16 * rt + lr][0]);
-                    const uint32_t z = h.z, wq = h.w;
-                    const uint32_t l0 = (z >> msh) & 63u, l1 = (z >> (msh + 8)) & 63u;
-                    const uint32_t h0 = ((wq >> (msh + 4)) & 15u) | (((z >> (msh + 6)) & 3u) << 4);
-                    const uint32_t h1 = ((wq >> (msh + 12)) & 15u) | (((z >> (msh + 14)) & 3u) << 4);
-                    const uint32_t m0 = mlo ? l0 : h0, m1 = mlo ? l1 : h1;
-                    // fp16 1024 + m (bits 0x6400 | m) minus 1024: the exact small integers
-                    const uint32_t pk = hadd2(((m1 << 16) | m0) + 0x64006400u, static_cast<_Float16>(-1024.0f));
-                    const f16x2_t p2 = __builtin_bit_cast(f16x2_t, pk);
-                    Bm[rt] = f16x4_t{p2[0], p2[0], p2[1], p2[1]};
+                    Bm[rt] = min_weights(h, lk);
                     dsc[rt] = opaque(half_bits(h.x & 0xffffu));
                     dmn5[rt] = opaque(-32.0f * half_bits(h.x >> 16));
                 }
             }
-            const Q4XSlot& xc = xr[g % kQ4XSlots];
+            // pieces and scales of the next depth's half block / block (stale ones after the last: not used)
+            if constexpr (S == 3) take_q(2 * b + 1);
+            if constexpr (S == 7) {
+                take_q(2 * b + 2);
+                take_hdr(b + 1);
+            }
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) {
-                if (iss) issue_part(g + kQ4Dist, tt);
-                if (dec && (tt & 1)) {
-                    const int rt = 2 * th + (tt >> 1);
-                    bs[(S + 1) & 1][rg][rt][lane] = decode_rt(IC<(S + 1) & 7>{}, g + 1, rt);
-                }
+                issue_part(g + kQ4Dist, tt);
+                __builtin_amdgcn_sched_barrier(0);
                 f16x8_t A[2];
 #pragma unroll
-                for (int p = 0; p < 2; ++p) A[p] = *reinterpret_cast<const f16x8_t*>(&xc[p][64 * th + 16 * tt + lr][ach]);
-                // a block's first stage starts its sums from zero
+                for (int p = 0; p < 2; ++p) {   // this tile's parts; the next tile's are requested
+                    A[p] = An[p];
+                    An[p] = *reinterpret_cast<const f16x8_t*>(&xr[(g + (tt == 3)) % kQ4XSlots][4 * th + ((tt + 1) & 3)][p][lane]);
+                }
+                // a block's first depth starts its sums from zero
 #pragma unroll
                 for (int rt = 0; rt < 4; ++rt)
-                    C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[0], B[rt], S == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : C[tt][rt], 0, 0, 0);
+                    C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[0], B[S & 1][rt], S == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : C[tt][rt], 0, 0, 0);
 #pragma unroll
-                for (int rt = 0; rt < 4; ++rt) C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[1], B[rt], C[tt][rt], 0, 0, 0);
+                for (int rt = 0; rt < 4; ++rt) C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[1], B[S & 1][rt], C[tt][rt], 0, 0, 0);
+                b_make(IC<(S + 1) & 7>{}, tt);
                 if constexpr (S == 7) {
-                    // token tile tt of the block is complete: acc += d P_block - 32 dmin P_min with
-                    // P_min = sum_g m_g (S_g 2^-5) as one [16 tokens x 16] x [16 x 16 rows] fp16
-                    // product, k = (group 2 lk + i / 2, part i % 2): the two fp16 parts of S 2^-5
-                    // (|S| < 2^20) against m_g twice
-                    const float2 v = *reinterpret_cast<const float2*>(&sr[b & 1][64 * th + 16 * tt + lr][2 * lk]);
-                    const float s0 = v.x * 0.03125f, s1 = v.y * 0.03125f;
-                    const _Float16 a0 = static_cast<_Float16>(s0), a1 = static_cast<_Float16>(s1);
-                    const f16x4_t As = f16x4_t{a0, static_cast<_Float16>(s0 - static_cast<float>(a0)), a1,
-                                               static_cast<_Float16>(s1 - static_cast<float>(a1))};
+                    // token tile tt of the block is complete: acc += d P_block - 32 dmin P_min
+                    const f16x4_t As = min_operand(*reinterpret_cast<const float2*>(&sr[b & 1][64 * th + 16 * tt + lr][2 * lk]));
 #pragma unroll
                     for (int rt = 0; rt < 4; ++rt) {
                         const f32x4_t pm = __builtin_amdgcn_mfma_f32_16x16x16f16(As, Bm[rt], f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -477,12 +1109,19 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, con
                         for (int r = 0; r < 4; ++r) acc[tt][rt][r] = __builtin_fmaf(dmn5[rt], pm[r], acc[tt][rt][r]);
                     }
                 }
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+                for (int i = 0; i < (S == 7 ? 12 : 8); ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, S == 7 ? 4 : 2, 0);
+                }
             }
-            // group g + 2 (the next stage's decode) complete; group g + 3 may stay in flight
-            wait_ring(g + 3 < nst ? q4_group_loads((S + 3) & 7) : 0);
+            // group g + 2 complete; group g + 3 may stay in flight
+            wait_vm<q4_group_loads((S + 3) & 7)>();
             barrier();
         });
     }
+    wait_vm<0>();
     // lane L holds C[4 (L/16) + r][L % 16] of tile (tt, rt): token 16 tt + 4 lk + r, row 16 rt + lr
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)
@@ -508,7 +1147,22 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, con
         }
 }
 
-// ------------------------------------------------------------------ Q6_K
+// ------------------------------------------------------------------ Q6_K, many tokens
+// Bytes (0, 2) and (1, 3) of n placed under `hi` (byte values 0 or 0x64).
+__device__ __forceinline__ uint32_t bytes02(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04020400u); }
+__device__ __forceinline__ uint32_t bytes13(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04030401u); }
+
+__device__ __forceinline__ uint32_t hadd2(uint32_t w, _Float16 c) {
+    const f16x2_t r = __builtin_bit_cast(f16x2_t, w) + f16x2_t{c, c};
+    return __builtin_bit_cast(uint32_t, r);
+}
+
+// fp16 q - 32 of four 6-bit quants (bytes of q): two words in the order (0, 2), (1, 3).
+__device__ __forceinline__ void q6_operand(uint32_t q, uint32_t& w02, uint32_t& w13) {
+    w02 = hadd2(bytes02(0x64646464u, q), static_cast<_Float16>(-1056.0f));
+    w13 = hadd2(bytes13(0x64646464u, q), static_cast<_Float16>(-1056.0f));
+}
+
 // Element i of a block (src/cuda/matmul_q4.cu:105-126): ql byte 64(i/128) +
 // 32((i%128)/32 & 1) + i%32 (low nibble in quarters 0, 1 of a half, high in
 // 2, 3), qh byte 128 + 32(i/128) + i%32 bits 2*quarter, scale byte 192 + i/16,
@@ -528,29 +1182,29 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k(const GemmJobs jobs, con
 // an LDS slot both read after the stage's barrier.
 constexpr int kQ6Waves = 8;
 constexpr int kQ6Block = kQ6Waves * kWave;
+constexpr int kQ6R = 256;                    // weight rows per workgroup (64 per wave)
 constexpr int kQ6T = 128;                    // tokens per workgroup
+constexpr int kXRow = 40;                    // halves per staged token row (32 + 8 padding)
+// A thread's share of one stage of x: 16 halves of one fp16 part of its token.
+struct XRegs {
+    uint4 a, b;
+};
 typedef uint16_t Q6XStage[2][kQ6T][kXRow];   // one stage of x: the two fp16 parts
 typedef f16x8_t Q6BSlot[4][2][2][kWave];     // B operands: [row group][step h][row tile][lane]
 // One half-block of a row: ql bytes 64 half .. +63 | qh bytes 128 + 32 half .. +31 |
 // scales (block bytes 192..207) | block bytes 194..209 (d in the last two) | pad (row
 // stride 36 dwords spreads a wave's 32 rows over the LDS banks)
-typedef uint8_t Q6WSlot[kGR][144];
+typedef uint8_t Q6WSlot[kQ6R][144];
 
-// 16 bytes at a 2-byte aligned address (gfx950 global loads take any byte
-// alignment; Q6_K blocks are 210 bytes).
-__device__ __forceinline__ uint4 ldg16_a2(const uint8_t* p) {
-    uint4 v;
-    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
-    return v;
-}
-
-__global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k(const GemmJobs jobs, const int* __restrict__ ex,
-                                                         const uint16_t* __restrict__ xp, const float* __restrict__ x,
+__global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k_wide(const GemmJobs jobs, const int* __restrict__ ex,
+                                                         const uint8_t* __restrict__ xp, const float* __restrict__ x,
                                                          int T, int K) {
     __shared__ __align__(16) Q6XStage xs[2];
     __shared__ __align__(16) Q6BSlot bs[2];
     __shared__ __align__(16) Q6WSlot wsl[2];
-    const GemmJob job = gemm_job(jobs);
+    const int cols = jobs.start[jobs.n];
+    const int tb = static_cast<int>(blockIdx.x) / cols;
+    const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x) - tb * cols);
     const uint8_t* __restrict__ w = job.w;
     float* __restrict__ y = job.y;
     const int M = job.M;
@@ -558,13 +1212,21 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k(const GemmJobs jobs, con
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
     const int rg = wv & 3, th = wv >> 2;                       // row group, token half (= decode step)
-    const int t0w = blockIdx.y * kQ6T;
+    const int t0w = tb * kQ6T;
     const int tw = t0w + 64 * th;
-    const int rw0 = job.mb * kGR;
+    const int rw0 = job.mb * kQ6R;
     const int r0 = rw0 + 64 * rg;
     const int nb = K >> 8, nst = K >> 5, nhb = nst >> 2;
     const int tok = tid >> 2, part = tid & 3;
-    const uint16_t* xsrc = xp + static_cast<size_t>(min(t0w + tok, T - 1)) * nst * 64 + 32 * (part >> 1) + 16 * (part & 1);
+    // stage g = 8 block + 4 h + u is the natural 32 elements 32 g ..: the thread's 16 halves (fp16 part p, k half
+    // l = lk % 2) are the pieces of depths 2 u, 2 u + 1 at lk = 2 h + l
+    const int xt = min(t0w + tok, T - 1) / kTile, xlr = min(t0w + tok, T - 1) % kTile;
+    const int xrn = min(kTile, T - kTile * xt);
+    const uint8_t* xbase = xp + tile_base(xt, K) + 16 * (static_cast<uint32_t>(part & 1) * xrn + xlr) + 64 * (part >> 1) * xrn;
+    auto load_x = [&](int g) {
+        const uint32_t o = (static_cast<uint32_t>(g >> 3) * 16 + 4 * (g & 3)) * 64 + 32 * ((g >> 2) & 1);
+        return XRegs{ld16(xbase + static_cast<size_t>(o) * xrn), ld16(xbase + static_cast<size_t>(o + 128) * xrn)};
+    };
     const int l32 = lane & 31, lh = lane >> 5;
     auto store_xs = [&](const XRegs& r, Q6XStage& d) {
         uint16_t* p = &d[part >> 1][tok][16 * (part & 1)];
@@ -633,7 +1295,7 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k(const GemmJobs jobs, con
         wstage_load(1);
         wstage_store(1);
     }
-    store_xs(load_x(xsrc), xs[0]);
+    store_xs(load_x(0), xs[0]);
     barrier();
     decode(0);
     barrier();
@@ -657,7 +1319,7 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k(const GemmJobs jobs, con
             }
         }
         XRegs xn;
-        if (more) xn = load_x(xsrc + static_cast<size_t>(gn) * 64);
+        if (more) xn = load_x(gn);
         // half-block k + 1 (loaded at half-block k - 1's first stage) goes into k - 1's
         // slot at half-block k's first stage (k - 1's decodes and scale reads ended with
         // the previous barrier); then half-block k + 2 is loaded
@@ -720,10 +1382,10 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k(const GemmJobs jobs, con
         }
 }
 
-// The Q4_K kernel's ring loads address x's fp16 parts and the weight rows with
-// 32-bit byte offsets.
+// Token rows that the matrix-core paths take; x's fragments and a matrix's rows are addressed with 32-bit byte
+// offsets (Q6_K: within a workgroup's rows only).
 bool gemm_rows_ok(int rows, int K, const float* x) {
-    return rows >= kGemmMinRows && K % 256 == 0 && aligned16(x) && rows <= kGemmMaxRows &&
+    return K % 256 == 0 && aligned16(x) && rows <= kGemmMaxRows &&
            4 * static_cast<uint64_t>(rows) * static_cast<uint64_t>(K) < (uint64_t{1} << 32);
 }
 
@@ -733,40 +1395,130 @@ bool gemm_job_ok(int type, uint64_t element_offset, int M, int K) {
     return type == kQ4_K && static_cast<uint64_t>(M) * static_cast<uint64_t>(K / 256) * 144 < (uint64_t{1} << 32);
 }
 
+// Workgroup columns of `rows` weight rows each, matrix after matrix.
+unsigned columns(GemmJobs& jobs, int rows) {
+    jobs.start[0] = 0;
+    for (int j = 0; j < jobs.n; ++j) jobs.start[j + 1] = jobs.start[j] + static_cast<int>(blocks_for(jobs.M[j], rows));
+    return static_cast<unsigned>(jobs.start[jobs.n]);
+}
+
 struct Prepared {
     const int* ex;
     const float* sx;
-    const uint16_t* xp;
+    const uint8_t* xp;
     const float* x;   // the token rows themselves (rows holding an infinity)
 };
 
-// Checks the workspace and launches the prep kernel.
-int prepare_x(const float* x, int rows, int K, void* workspace, size_t workspace_bytes, hipStream_t s, Prepared& p) {
+// Checks the workspace (wanted from 16 rows on, whichever path runs) and launches the prep kernel if a path needs it.
+int prepare_x(bool prep, const float* x, int rows, int K, void* workspace, size_t workspace_bytes, hipStream_t s,
+              Prepared& p) {
     const size_t need = ws_bytes(rows, K);
-    QK_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
+    if (rows >= kGemmMinRows) QK_REQUIRE(workspace && workspace_bytes >= need && aligned16(workspace),
                "matmul_rows: workspace of %zu bytes (16-byte aligned) needed, got %zu", need,
                workspace ? workspace_bytes : size_t{0});
+    p = Prepared{nullptr, nullptr, nullptr, x};
+    if (!prep) return ok();
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     int* ex = reinterpret_cast<int*>(ws);
     float* sx = reinterpret_cast<float*>(ws + ws_exp_bytes(rows));
-    uint16_t* xp = reinterpret_cast<uint16_t*>(ws + ws_exp_bytes(rows) + ws_sum_bytes(rows, K));
-    const unsigned grid = blocks_for(rows, 4);
+    uint8_t* xp = ws + ws_exp_bytes(rows) + ws_sum_bytes(rows, K);
+    const unsigned grid = blocks_for(rows, kTile);
     switch (K) {
-        case 512: gemm_prep_x<2><<<grid, 256, 0, s>>>(x, ex, sx, xp, rows, K); break;
-        case 1024: gemm_prep_x<4><<<grid, 256, 0, s>>>(x, ex, sx, xp, rows, K); break;
-        case 2048: gemm_prep_x<8><<<grid, 256, 0, s>>>(x, ex, sx, xp, rows, K); break;
-        case 4096: gemm_prep_x<16><<<grid, 256, 0, s>>>(x, ex, sx, xp, rows, K); break;
-        default: gemm_prep_x<0><<<grid, 256, 0, s>>>(x, ex, sx, xp, rows, K); break;
+        case 512: gemm_prep_x<1><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
+        case 1024: gemm_prep_x<2><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
+        case 2048: gemm_prep_x<4><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
+        case 4096: gemm_prep_x<8><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
+        default: gemm_prep_x<0><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
     }
     p = Prepared{ex, sx, xp, x};
     return check_launch("matmul_rows prep");
 }
 
-void launch_gemm(int type, const GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
+// How a matrix of a call is computed. A matrix alone and among others takes the same path and adds in the same
+// order, so the rule looks at the token count, K and the matrix itself only; which tile shape a path then uses
+// (sums are the same bits in all of them) depends on the whole launch.
+enum class Path { gemv, few, sliced4, sliced2, wide };
+
+// Measured at K = 2048 (M = 12352 in four matrices) and K = 4096 (M = 2048), Q4_K, us including the prep pass:
+//   few against one GEMV per token: 12 / 12 at every count up to 16; GEMV 6 / 3.6 per token, so it starts at 3
+//     tokens (4 where K takes two rounds). Against sliced4 at 17..32 tokens 22 / 12 and 18 / 26, at 128 tokens
+//     74 / 19 and 44 / 26, at 300 tokens sliced2 42 at K = 4096: few up to 16 tokens, up to 160 from K = 4096.
+//   sliced4 against sliced2, 77 tokens: 31 and 36; 200 tokens: 58 and 54.
+//   sliced2 against wide: 768 tokens 130 / 58 and 128 / 109; 1100 tokens 185 / 85 and 135 / 109; 2100 tokens
+//     300 / 160 and 249 / 113. A matrix of up to 64 rows would leave most of a wide tile idle for a whole round.
+// Q6_K times are about 1.5x these on every path but wide (1.75x); the same lines hold within 10%.
+Path gemm_path(int rows, int K, int M) {
+    const int nb = K / 256;
+    if (rows < (nb > 8 ? 4 : 3)) return Path::gemv;
+    if (rows <= (nb >= 16 ? 160 : nb % 4 ? 128 : 16)) return Path::few;
+    if (rows <= 128) return Path::sliced4;
+    const int most = nb >= 16 && M < 4096 ? 2048 : 768;
+    if (nb % 2 == 0 && (rows <= most || M <= 64)) return Path::sliced2;
+    return Path::wide;
+}
+
+template <int TYPE, int WT, int WR, int KW, int SL>
+struct Shape {
+    using G = GemmShape<TYPE, WT, WR, KW, SL>;
+    // Workgroups of the launch in rounds of 256 (one per CU) times a round's measured time (us at K = 2048, Q4_K).
+    static float cost(GemmJobs& jobs, int rows, float round) {
+        const unsigned wgs = columns(jobs, G::rows) * blocks_for(rows, G::tokens);
+        return round * static_cast<float>(blocks_for(wgs, 256));
+    }
+    static void launch(GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
+        const unsigned grid = columns(jobs, G::rows) * blocks_for(rows, G::tokens);
+        gemm_kquant<TYPE, WT, WR, KW, SL><<<grid, 512, 0, s>>>(jobs, p.ex, p.sx, p.xp, p.x, rows, K);
+    }
+};
+
+template <int TYPE>
+void launch_gemm(Path path, GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
+    if (path == Path::few) {
+        const unsigned tb = blocks_for(rows, kTile);
+        if (columns(jobs, 16) * tb <= 256)
+            gemm_few<TYPE, 1><<<columns(jobs, 16) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
+        else if (columns(jobs, 32) * tb <= 256)
+            gemm_few<TYPE, 2><<<columns(jobs, 32) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
+        else
+            gemm_few<TYPE, 4><<<columns(jobs, 64) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
+    } else if (path == Path::sliced4) {
+        using S1 = Shape<TYPE, 2, 2, 4, 4>;
+        using S2 = Shape<TYPE, 2, 2, 2, 4>;
+        using S3 = Shape<TYPE, 3, 2, 2, 4>;
+        const float c1 = S1::cost(jobs, rows, 12.5f), c2 = S2::cost(jobs, rows, 20.f), c3 = S3::cost(jobs, rows, 25.f);
+        if (c1 <= c2 && c1 <= c3)
+            S1::launch(jobs, p, rows, K, s);
+        else if (c2 <= c3)
+            S2::launch(jobs, p, rows, K, s);
+        else
+            S3::launch(jobs, p, rows, K, s);
+    } else if (path == Path::sliced2) {
+        using S1 = Shape<TYPE, 2, 2, 2, 2>;
+        using S2 = Shape<TYPE, 3, 2, 2, 2>;
+        using S3 = Shape<TYPE, 4, 2, 2, 2>;
+        using S4 = Shape<TYPE, 4, 2, 1, 2>;
+        const float c1 = S1::cost(jobs, rows, 20.f), c2 = S2::cost(jobs, rows, 25.f), c3 = S3::cost(jobs, rows, 31.f),
+                    c4 = S4::cost(jobs, rows, 46.f);
+        if (c1 <= c2 && c1 <= c3 && c1 <= c4)
+            S1::launch(jobs, p, rows, K, s);
+        else if (c2 <= c3 && c2 <= c4)
+            S2::launch(jobs, p, rows, K, s);
+        else if (c3 <= c4)
+            S3::launch(jobs, p, rows, K, s);
+        else
+            S4::launch(jobs, p, rows, K, s);
+    } else if constexpr (TYPE == kQ4_K) {
+        gemm_q4k_wide<<<columns(jobs, kQ4R) * blocks_for(rows, kQ4T), kQ4Block, 0, s>>>(jobs, p.ex, p.sx, p.xp, p.x, rows, K);
+    } else {
+        gemm_q6k_wide<<<columns(jobs, kQ6R) * blocks_for(rows, kQ6T), kQ6Block, 0, s>>>(jobs, p.ex, p.xp, p.x, rows, K);
+    }
+}
+
+void launch_gemm(Path path, int type, GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
     if (type == kQ4_K)
-        gemm_q4k<<<dim3(jobs.start[jobs.n], blocks_for(rows, kQ4T)), kQ4Block, 0, s>>>(jobs, p.ex, p.sx, p.xp, p.x, rows, K);
+        launch_gemm<kQ4_K>(path, jobs, p, rows, K, s);
     else
-        gemm_q6k<<<dim3(jobs.start[jobs.n], blocks_for(rows, kQ6T)), kQ6Block, 0, s>>>(jobs, p.ex, p.xp, p.x, rows, K);
+        launch_gemm<kQ6_K>(path, jobs, p, rows, K, s);
 }
 
 // One GEMV per token (the reference's own loop).
@@ -802,20 +1554,18 @@ int qwen_matmul_rows(const void* weight, int type, uint64_t num_elements, const 
     QK_REQUIRE(rows >= 0, "matmul_rows: negative rows %d", rows);
     if (rows == 0) return ok();
     QK_REQUIRE(x && y, "matmul_rows: null pointer");
-    if (!gemm_rows_ok(rows, K, x) || !gemm_job_ok(type, element_offset, M, K))
-        return per_token(weight, type, num_elements, x, y, rows, M, K, element_offset, stream);
+    const Path path = gemm_rows_ok(rows, K, x) && gemm_job_ok(type, element_offset, M, K) ? gemm_path(rows, K, M) : Path::gemv;
+    if (path == Path::gemv) return per_token(weight, type, num_elements, x, y, rows, M, K, element_offset, stream);
     const hipStream_t s = as_stream(stream);
     Prepared p;
-    if (const int rc = prepare_x(x, rows, K, workspace, workspace_bytes, s, p)) return rc;
+    if (const int rc = prepare_x(path != Path::few, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
     GemmJobs jobs{};
     jobs.w[0] = static_cast<const uint8_t*>(weight);
     jobs.y[0] = y;
     jobs.ub0[0] = element_offset / 256;
     jobs.M[0] = M;
-    jobs.start[0] = 0;
-    jobs.start[1] = static_cast<int>(blocks_for(M, kGR));
     jobs.n = 1;
-    launch_gemm(type, jobs, p, rows, K, s);
+    launch_gemm(path, type, jobs, p, rows, K, s);
     return check_launch("matmul_rows");
 }
 
@@ -839,40 +1589,53 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
     if (rows == 0) return ok();
     QK_REQUIRE(x, "matmul_rows_multi: null x");
     const bool gemm = gemm_rows_ok(rows, K, x);
+    Path path[64];
+    bool any = false, prep = false, all_gemv = true;
+    for (int j = 0; j < n; ++j) {
+        const qwen_gemv_desc& e = descs[j];
+        path[j] = gemm && gemm_job_ok(e.type, e.element_offset, e.M, K) ? gemm_path(rows, K, e.M) : Path::gemv;
+        any |= path[j] != Path::gemv;
+        prep |= path[j] != Path::gemv && path[j] != Path::few;
+        all_gemv &= path[j] == Path::gemv;
+    }
+    if (all_gemv) {   // every matrix in one call per token (each output the bits of its own GEMV)
+        qwen_gemv_desc d[64];
+        for (int t = 0; t < rows; ++t) {
+            for (int j = 0; j < n; ++j) {
+                d[j] = descs[j];
+                d[j].y = descs[j].y + static_cast<size_t>(t) * descs[j].M;
+            }
+            if (const int rc = qwen_matmul_dispatch_multi(d, n, x + static_cast<size_t>(t) * K, K, stream)) return rc;
+        }
+        return ok();
+    }
     const hipStream_t s = as_stream(stream);
     Prepared p{};
-    bool prepared = false;
-    for (const int type : {static_cast<int>(kQ4_K), static_cast<int>(kQ6_K)}) {
-        GemmJobs jobs{};
-        auto flush = [&]() {
-            if (jobs.n == 0) return;
-            launch_gemm(type, jobs, p, rows, K, s);
-            jobs.n = 0;
-        };
-        for (int j = 0; gemm && j < n; ++j) {
-            const qwen_gemv_desc& e = descs[j];
-            if (e.type != type || !gemm_job_ok(e.type, e.element_offset, e.M, K)) continue;
-            if (!prepared) {
-                if (const int rc = prepare_x(x, rows, K, workspace, workspace_bytes, s, p)) return rc;
-                prepared = true;
+    if (any)
+        if (const int rc = prepare_x(prep, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
+    for (const int type : {static_cast<int>(kQ4_K), static_cast<int>(kQ6_K)})
+        for (const Path to : {Path::few, Path::sliced4, Path::sliced2, Path::wide}) {
+            GemmJobs jobs{};
+            for (int j = 0; j < n; ++j) {
+                const qwen_gemv_desc& e = descs[j];
+                if (e.type != type || path[j] != to) continue;
+                const int k = jobs.n++;
+                jobs.w[k] = static_cast<const uint8_t*>(e.weight);
+                jobs.y[k] = e.y;
+                jobs.ub0[k] = e.element_offset / 256;
+                jobs.M[k] = e.M;
+                if (jobs.n == kGemmJobs) {
+                    launch_gemm(to, type, jobs, p, rows, K, s);
+                    jobs.n = 0;
+                }
             }
-            const int k = jobs.n;
-            jobs.w[k] = static_cast<const uint8_t*>(e.weight);
-            jobs.y[k] = e.y;
-            jobs.ub0[k] = e.element_offset / 256;
-            jobs.M[k] = e.M;
-            if (k == 0) jobs.start[0] = 0;
-            jobs.start[k + 1] = jobs.start[k] + static_cast<int>(blocks_for(e.M, kGR));
-            jobs.n = k + 1;
-            if (jobs.n == kGemmJobs) flush();
+            if (jobs.n) launch_gemm(to, type, jobs, p, rows, K, s);
         }
-        flush();
-    }
-    if (prepared)
+    if (any)
         if (const int rc = check_launch("matmul_rows_multi")) return rc;
     for (int j = 0; j < n; ++j) {   // the rest: one GEMV per token
         const qwen_gemv_desc& e = descs[j];
-        if (gemm && gemm_job_ok(e.type, e.element_offset, e.M, K)) continue;
+        if (path[j] != Path::gemv) continue;
         if (const int rc = per_token(e.weight, e.type, e.num_elements, x, e.y, rows, e.M, K, e.element_offset, stream))
             return rc;
     }

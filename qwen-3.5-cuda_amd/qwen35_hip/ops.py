@@ -826,7 +826,7 @@ def matmul_rows(weight, ggml_type, num_elements: int, x, M: int, K: int, element
                 workspace=None, stream=None):
     """matmul_dispatch for every row of x: x float32 [rows, K] -> y float32 [rows, M],
     y[t, m] = sum_k W[element_offset + m*K + k] * x[t, k] (one call; matrix cores for
-    Q4_K / Q6_K at 16 rows or more, with a workspace allocated here unless given)."""
+    Q4_K / Q6_K at 3 rows (4 for long rows) or more, with a workspace allocated here unless given)."""
     _dev(weight, dtype=torch.uint8)
     _dev(x, dtype=torch.float32)
     if x.dim() != 2 or x.shape[1] != K:

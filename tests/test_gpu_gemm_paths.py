@@ -1,0 +1,104 @@
+"""matmul_rows over the token counts where its kernels and tile shapes change.
+
+The rule (csrc/gemm.hip, gemm_path) takes a GEMV per token below 3 (4) tokens, then three
+matrix-core forms and the wide tiles; the sliced forms choose a tile shape by the launch's
+total. Each case sits at an edge of that rule, of a tile (16, 32, 48, 64, 128 tokens; 16 to 256
+rows) or of a K split (blocks per row that 2, 4 or 8 slices do not divide), against the oracle's
+GEMV at the fp32 bar and half of it against the outputs' rms, as the other GEMV tests.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import assert_bits_equal, assert_f32_close, rel_err
+from qwen35_hip import ops, synth
+
+pytestmark = pytest.mark.gpu
+
+F32 = np.float32
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _weight(kind, rows, K, seed):
+    t = synth.q4k_table(rows, K, seed_tensor=seed) if kind == "Q4_K" else synth.q6k_table(rows, K, seed_tensor=seed)
+    return t
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T,M,K", [
+    (2, 48, 2048), (3, 17, 2048), (3, 300, 256), (4, 65, 4096), (15, 130, 2304),    # GEMV / few, partial rounds of K
+    (16, 4100, 2048), (17, 64, 2048), (33, 129, 1024), (47, 300, 2048), (49, 96, 512),
+    (127, 200, 2048), (128, 33, 2048), (129, 257, 2048), (129, 100, 1280),          # four slices / two / none (odd)
+    (160, 80, 4096), (161, 80, 4096), (191, 500, 4608), (700, 2048, 512),
+    (768, 130, 2048), (769, 130, 2048), (769, 64, 2048), (783, 65, 1280),           # wide; thin matrices stay sliced
+])
+def test_matmul_rows_edges(oracle, kind, T, M, K):
+    r = np.random.default_rng(T * 131 + M + K)
+    w = _weight(kind, M, K, 5)
+    x = r.standard_normal((T, K)).astype(F32)
+    out = torch.full((T + 1, M), 5.0, device="cuda")
+    ops.matmul_rows(_dev(w), kind, M * K, _dev(x), M, K, out=out)
+    got = out.cpu().numpy()
+    rows = sorted({0, 1, T // 2, T - 2, T - 1} | {t for t in (15, 16, 31, 47, 63, 64, 127, 128) if t < T})
+    for t in rows:
+        ref = oracle.gemv(w, ops.GGML_TYPES[kind], x[t], M, K)
+        assert_f32_close(got[t], ref, group=M, what=f"{kind} {T}x{M}x{K} token {t}")
+        rms = np.sqrt(np.mean(ref.astype(np.float64) ** 2))
+        assert np.abs(got[t].astype(np.float64) - ref).max() <= 5e-6 * rms
+    assert np.all(got[T] == 5.0)
+
+
+@pytest.mark.parametrize("T", [2, 9, 20, 100, 200, 800])
+def test_matmul_rows_multi_keeps_the_bits(T):
+    """Tile shapes follow the launch's total, sums do not: each matrix of a call gives the bits of its own call
+    (thin matrices and both types among them)."""
+    r = np.random.default_rng(T)
+    K = 2048
+    x = _dev(r.standard_normal((T, K)).astype(F32))
+    jobs = [(_dev(_weight(kind, M, K, 20 + i)), kind, M * K, M, 0, None)
+            for i, (kind, M) in enumerate([("Q4_K", 8192), ("Q4_K", 32), ("Q6_K", 512), ("Q4_K", 2048), ("Q6_K", 48)])]
+    for (w, kind, ne, M, off, _), got in zip(jobs, ops.matmul_rows_multi(jobs, x, K)):
+        assert_bits_equal(got.cpu().numpy(), ops.matmul_rows(w, kind, ne, x, M, K).cpu().numpy(), what=f"{kind} {M}")
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+def test_few_tokens_as_exact_as_the_gemv(kind):
+    """Below 16 tokens the matrix-core form replaces one fp32 GEMV per token: its 2-norm error against float64 is no
+    larger than the GEMV's (both sums have the same bound; the margin is the spread over inputs)."""
+    r = np.random.default_rng(3)
+    M, K, T = 1024, 2048, 12
+    w = _dev(_weight(kind, M, K, 9))
+    x = r.standard_normal((T, K)).astype(F32)
+    dx = _dev(x)
+    eye = ops.dequant_gather_rows(w, kind, M * K, torch.arange(M, dtype=torch.int32, device="cuda"), K)
+    ref = x.astype(np.float64) @ eye.cpu().numpy().astype(np.float64).T
+    few = ops.matmul_rows(w, kind, M * K, dx, M, K).cpu().numpy()
+    one = np.stack([ops.matmul_dispatch(w, kind, M * K, dx[t], M, K).cpu().numpy() for t in range(T)])
+    err = [np.linalg.norm(v - ref) / np.linalg.norm(ref) for v in (few, one)]
+    assert err[0] <= 1.1 * err[1], err
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T", [5, 40, 150, 800])
+def test_nonfinite_rows_in_every_form(oracle, kind, T):
+    """A token row with an infinity gives the reference's pattern, a NaN row NaN, a zero row +0; others are
+    unaffected (two rounds of K for the few-token form)."""
+    M, K = 96, 4096 if T == 150 else 2048
+    w = _weight(kind, M, K, 7)
+    x = np.random.default_rng(T).standard_normal((T, K)).astype(F32)
+    x[1, K - 1] = np.inf
+    x[2, 7] = np.nan
+    x[3] = 0.0
+    got = ops.matmul_rows(_dev(w), kind, M * K, _dev(x), M, K).cpu().numpy()
+    ref = oracle.gemv(w, ops.GGML_TYPES[kind], x[1], M, K)
+    assert np.array_equal(np.isnan(got[1]), np.isnan(ref)) and np.array_equal(got[1][np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.isnan(got[2]).all() and np.array_equal(got[3].view(np.uint32), np.zeros(M, np.uint32))
+    for t in (0, 4, T - 1):
+        ref = oracle.gemv(w, ops.GGML_TYPES[kind], x[t], M, K)
+        assert rel_err(got[t], ref, group=M).max() <= 1e-5
