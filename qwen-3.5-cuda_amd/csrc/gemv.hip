@@ -931,11 +931,15 @@ __global__ __launch_bounds__(kGemvBlock) void gemv_q6k_direct_multi(const float*
 // The rest of a MoE layer's decode step after the SwiGLU hidden rows
 // (src/layer_moe.cpp:135-147) in one launch, for routed experts of inter = 512
 // (2 blocks per row: rows 4q .. 4q+3 of one expert are one 8-block unit) and
-// a shared expert of shared_dim = 2048 * SS. A workgroup owns output rows
+// a shared expert of shared_dim = 2048 * SS, or of 512 (SS = 0: the model's
+// small shared expert, whose rows 4q .. 4q+3 are one unit like an expert's; as
+// five launches -- expert GEMVs, shared GEMV, fill, weighted sum, gated add --
+// that shape took 18.2 us a layer, here 6.5). A workgroup owns output rows
 // 4q .. 4q+3; wave w
 //   * decodes the unit of rows 4q .. 4q+3 of routed expert j = w + 4t (t < KT)
 //     against that expert's hidden row;
-//   * computes row 4q + w of the shared expert's down projection;
+//   * computes row 4q + w of the shared expert's down projection (SS = 0: wave
+//     3, which has one routed expert fewer when k < 8, all four rows);
 // with the per-row kernel's units, lane map and reductions, so each expert
 // output and the shared output have the bits of the separate launches (the
 // expert GEMVs, the shared GEMV). Lanes 0..3 of wave 0 then combine
@@ -952,7 +956,8 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_kernel(
     constexpr int BE = KQuant<TE>::kBlockBytes, BS = KQuant<TS>::kBlockBytes;
     constexpr int CE = BE * 8 / 16, CS = BS * 8 / 16;   // 16-byte chunks per unit (72 or 105)
     static_assert(CE > kWave && CE <= 2 * kWave && CS > kWave && CS <= 2 * kWave, "two chunks per lane");
-    constexpr int SLOT = KT * CE + SS * CS;
+    constexpr int SU = SS ? SS : 1;                     // shared units per wave
+    constexpr int SLOT = KT * CE + SU * CS;
     __shared__ uint4 stage[kGemvWaves][SLOT];
     __shared__ float part[4 * KT][4];
     __shared__ float spart[4];
@@ -962,7 +967,7 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_kernel(
     const bool tail = lane + kWave < CE;
 
     // Every unit's bytes requested before the first wait.
-    uint4 ce[KT][2], cs[SS][2];
+    uint4 ce[KT][2], cs[SU][2];
     bool valid[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
@@ -975,20 +980,20 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_kernel(
     }
     const int row = 4 * q + w;
 #pragma unroll
-    for (int s = 0; s < SS; ++s) {
-        const uint8_t* unit = wsd + (static_cast<uint64_t>(row) * 8 * SS + 8 * s) * BS;
+    for (int s = 0; s < SU; ++s) {
+        const uint8_t* unit = wsd + (SS ? static_cast<uint64_t>(row) * 8 * SS + 8 * s : static_cast<uint64_t>(8) * q) * BS;
         cs[s][0] = ld16_nt(unit + 16 * lane);
         cs[s][1] = lane + kWave < CS ? ld16_nt(unit + 16 * (lane + kWave)) : make_uint4(0, 0, 0, 0);
     }
     LaneX<TE> lxe[KT];
-    LaneX<TS> lxs[SS];
+    LaneX<TS> lxs[SU];
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
         const int j = min(w + 4 * t, k - 1);
         load_lane_x<TE>(lxe[t], hid + static_cast<size_t>(j) * kDcInter, b & 1, jj);
     }
 #pragma unroll
-    for (int s = 0; s < SS; ++s) load_lane_x<TS>(lxs[s], shid, 8 * s + b, jj);
+    for (int s = 0; s < SU; ++s) load_lane_x<TS>(lxs[s], shid, SS ? 8 * s + b : b & 1, jj);
 
     uint4* slot = stage[w];
 #pragma unroll
@@ -997,7 +1002,7 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_kernel(
         if (tail) slot[t * CE + kWave + lane] = ce[t][1];
     }
 #pragma unroll
-    for (int s = 0; s < SS; ++s) {
+    for (int s = 0; s < SU; ++s) {
         slot[KT * CE + s * CS + lane] = cs[s][0];
         if (lane + kWave < CS) slot[KT * CE + s * CS + kWave + lane] = cs[s][1];
     }
@@ -1014,9 +1019,13 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_kernel(
     {
         float a = 0.f;
 #pragma unroll
-        for (int s = 0; s < SS; ++s) a += block_dot<TS>(base + (KT * CE + s * CS) * 16 + b * BS, lxs[s], jj);
-        a = group_sum<64>(a);
-        if (lane == 0) spart[w] = a;
+        for (int s = 0; s < SU; ++s) a += block_dot<TS>(base + (KT * CE + s * CS) * 16 + b * BS, lxs[s], jj);
+        a = group_sum<SS ? 64 : 16>(a);
+        if (SS) {
+            if (lane == 0) spart[w] = a;
+        } else if (w == 3 && (lane & 15) == 0) {
+            spart[lane >> 4] = a;
+        }
     }
     __syncthreads();
     if (w == 0 && lane < 4) {
@@ -1043,9 +1052,10 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
         const float* __restrict__ shid, const float* __restrict__ slogit, float* __restrict__ out) {
     constexpr int BB = KQuant<kQ4_K>::kBlockBytes;
     constexpr int NXR = 4 * KT * (kDcInter / 4);   // float4 of the routed hidden rows
-    constexpr int NXS = SS * 512;                  // float4 of the shared hidden row (2048 SS)
-    constexpr int PR = NXR / kGemvBlock, PS = NXS / kGemvBlock;
-    static_assert(PR * kGemvBlock == NXR && PS * kGemvBlock == NXS, "x staging");
+    constexpr int SU = SS ? SS : 1;                // shared units per wave
+    constexpr int NXS = SS ? SS * 512 : 128;       // float4 of the shared hidden row (2048 SS, or 512)
+    constexpr int PR = NXR / kGemvBlock, PS = SS ? NXS / kGemvBlock : 1;
+    static_assert(PR * kGemvBlock == NXR && (!SS || PS * kGemvBlock == NXS), "x staging");
     __shared__ float4 xr[NXR];
     __shared__ float4 xsh[NXS];
     __shared__ float part[4 * KT][4];
@@ -1062,10 +1072,10 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
         tr[i] = ld4(hid + static_cast<size_t>(jr) * kDcInter + 4 * (c % (kDcInter / 4)));
     }
 #pragma unroll
-    for (int i = 0; i < PS; ++i) ts[i] = ld4(shid + 4 * (threadIdx.x + i * kGemvBlock));
+    for (int i = 0; i < PS; ++i) ts[i] = ld4(shid + 4 * (threadIdx.x % NXS + i * kGemvBlock));
     __builtin_amdgcn_sched_barrier(0);   // the hidden rows first
 
-    uint4 he[KT], qe[KT], hs[SS], qs[SS];
+    uint4 he[KT], qe[KT], hs[SU], qs[SU];
     bool valid[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
@@ -1078,8 +1088,8 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
     }
     const int row = 4 * q + w;
 #pragma unroll
-    for (int s = 0; s < SS; ++s) {
-        const uint8_t* blk = wsd + (static_cast<uint64_t>(row) * 8 * SS + 8 * s + b) * BB;
+    for (int s = 0; s < SU; ++s) {
+        const uint8_t* blk = wsd + (SS ? static_cast<uint64_t>(row) * 8 * SS + 8 * s + b : static_cast<uint64_t>(8) * q + b) * BB;
         hs[s] = ld16_nt(blk);
         qs[s] = ld16_nt(blk + 16 + 16 * jj);
     }
@@ -1087,7 +1097,7 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
 #pragma unroll
     for (int i = 0; i < PR; ++i) xr[threadIdx.x + i * kGemvBlock] = tr[i];
 #pragma unroll
-    for (int i = 0; i < PS; ++i) xsh[threadIdx.x + i * kGemvBlock] = ts[i];
+    for (int i = 0; i < PS; ++i) xsh[threadIdx.x % NXS + i * kGemvBlock] = ts[i];
     __syncthreads();
 
     const int xo = 64 * (jj >> 1) + 16 * (jj & 1);   // load_lane_x_values' offsets in a 256-element block
@@ -1110,9 +1120,9 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
     {
         float a = 0.f;
 #pragma unroll
-        for (int s = 0; s < SS; ++s) {
+        for (int s = 0; s < SU; ++s) {
             LaneX<kQ4_K> lx;
-            const float4* lo = xsh + ((8 * s + b) * 256 + xo) / 4;
+            const float4* lo = xsh + ((SS ? 8 * s + b : b & 1) * 256 + xo) / 4;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 lx.v[i] = lo[i];
@@ -1121,8 +1131,12 @@ __global__ __launch_bounds__(kGemvBlock) void moe_down_combine_q4k(
             lane_x_sums(lx);
             a += block_dot_q4k(hs[s], qs[s], lx, jj);
         }
-        a = group_sum<64>(a);
-        if (lane == 0) spart[w] = a;
+        a = group_sum<SS ? 64 : 16>(a);
+        if (SS) {
+            if (lane == 0) spart[w] = a;
+        } else if (w == 3 && (lane & 15) == 0) {
+            spart[lane >> 4] = a;
+        }
     }
     __syncthreads();
     if (w == 0 && lane < 4) {
@@ -1822,9 +1836,9 @@ void launch_dc(const DownCombine& a, hipStream_t s) {
 template <int TE, int TS>
 void launch_dc_t(const DownCombine& a, int ss, hipStream_t s) {
     if (a.k <= 4)
-        ss == 1 ? launch_dc<TE, TS, 1, 1>(a, s) : launch_dc<TE, TS, 1, 2>(a, s);
+        ss == 0 ? launch_dc<TE, TS, 1, 0>(a, s) : ss == 1 ? launch_dc<TE, TS, 1, 1>(a, s) : launch_dc<TE, TS, 1, 2>(a, s);
     else
-        ss == 1 ? launch_dc<TE, TS, 2, 1>(a, s) : launch_dc<TE, TS, 2, 2>(a, s);
+        ss == 0 ? launch_dc<TE, TS, 2, 0>(a, s) : ss == 1 ? launch_dc<TE, TS, 2, 1>(a, s) : launch_dc<TE, TS, 2, 2>(a, s);
 }
 
 void launch_down_combine(const DownCombine& a, int te, int ts, int ss, hipStream_t s) {
@@ -2158,8 +2172,8 @@ int qwen_moe_down_combine(const void* w_down, int down_type, uint64_t down_eleme
     const auto* wd = static_cast<const uint8_t*>(w_down);
     const auto* wsd = static_cast<const uint8_t*>(w_shared_down);
     const auto kq = [](int t) { return t == kQ4_K || t == kQ6_K; };
-    const bool fused = kq(down_type) && kq(shared_type) && inter == kDcInter && shared_dim % 2048 == 0 &&
-                       shared_dim <= 4096 && d_model % 4 == 0 && n_sel <= 8 && expert_stride % 2048 == 0 &&
+    const bool fused = kq(down_type) && kq(shared_type) && inter == kDcInter &&
+                       (shared_dim == 512 || (shared_dim % 2048 == 0 && shared_dim <= 4096)) && d_model % 4 == 0 && n_sel <= 8 && expert_stride % 2048 == 0 &&
                        aligned16(wd) && aligned16(wsd) && aligned16(hidden) && aligned16(shared_hidden);
     if (fused) {
         const DownCombine a{wd, expert_stride / 256, n_experts, idx, weights, n_sel, hidden, wsd, shared_hidden,
