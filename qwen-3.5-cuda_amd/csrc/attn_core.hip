@@ -156,19 +156,27 @@ struct ScoreTiles {
     static_assert(T * 16 == L && P * T == NT / kWave && G <= 16 && DP % 16 == 0, "score tiles");
     typedef float Part[T][16][17];
 
-    static __device__ __forceinline__ void run(const float4 (*q_lds)[kMaxDim / 4], const float (*k_lds)[kKeyStride],
-                                               Part* sc, int tid) {
+    // The lane's share of the query operands (float4 s of its dims), from queries staged in LDS, S floats a row.
+    template <int S>
+    static __device__ __forceinline__ void load_q(const float* q_lds, int tid, float4 (&qb)[DP / 16]) {
+        const int l = tid & (kWave - 1), part = wave_in_block() / T;
+        const float* qrow = q_lds + ((l & 15) % G) * S + part * DP + (l >> 4) * (DP / 4);
+#pragma unroll
+        for (int s = 0; s < DP / 16; ++s) qb[s] = *reinterpret_cast<const float4*>(qrow + 4 * s);
+    }
+
+    static __device__ __forceinline__ void run(const float4 (&q)[DP / 16], const float (*k_lds)[kKeyStride], Part* sc,
+                                               int tid) {
         typedef float v4f_t __attribute__((ext_vector_type(4)));
         const int w = wave_in_block(), l = tid & (kWave - 1);
         const int tile = w % T, part = w / T;
         const int m = l & 15, g = l >> 4;
         const float* krow = &k_lds[tile * 16 + m][part * DP + g * (DP / 4)];
-        const float4* qrow = &q_lds[m % G][(part * DP + g * (DP / 4)) / 4];
         v4f_t acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
+#pragma unroll
         for (int s = 0; s < DP / 16; ++s) {
             const float4 ka = *reinterpret_cast<const float4*>(krow + 4 * s);
-            const float4 qb = qrow[s];
+            const float4 qb = q[s];
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.x, qb.x, acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.y, qb.y, acc, 0, 0, 0);
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ka.z, qb.z, acc, 0, 0, 0);
@@ -228,7 +236,9 @@ __global__ __launch_bounds__(G * L) void scores_split(const float* __restrict__ 
         *reinterpret_cast<float4*>(&k_lds[c / D4][4 * (c % D4)]) = kr[i];
     }
     __syncthreads();
-    Tiles::run(q_lds, k_lds, sc_lds, tid);
+    float4 qb[Tiles::DP / 16];
+    Tiles::template load_q<D>(&q_lds[0][0].x, tid, qb);
+    Tiles::run(qb, k_lds, sc_lds, tid);
     __syncthreads();
     const int hh = tid / L, tt = tid % L;
     if (t0 + tt < n_keys)
@@ -395,7 +405,7 @@ struct KeyCache<true> {
 };
 
 template <int G, int L, bool NR = false>
-__global__ __launch_bounds__(G * L * kPairLanes) void decode_split(
+__global__ __launch_bounds__(G * L * kPairLanes) __attribute__((amdgpu_waves_per_eu(4))) void decode_split(
     const float* __restrict__ q, typename KeyCache<NR>::type kc, const float* __restrict__ vc,
     float* __restrict__ ws_acc, float* __restrict__ ws_m, float* __restrict__ ws_l, int kv_heads, int n_keys,
     int splits, float scale, NormRopeArgs nr = NormRopeArgs{}, RopeDen den = RopeDen{}) {
@@ -408,8 +418,7 @@ __global__ __launch_bounds__(G * L * kPairLanes) void decode_split(
     constexpr int KCH = L * D4 / NT;           // float4 chunks of the key tile per thread
     static_assert(NT % D == 0 && L % HALVES == 0 && (G * D4) % NT == 0 && (L * D4) % NT == 0 &&
                   L * kPairLanes <= kWave && kWave % (L * kPairLanes) == 0, "decode_split shape");
-    __shared__ float4 q_lds[G][D4];
-    __shared__ __align__(16) float k_lds[L][kKeyStride];
+    __shared__ __align__(16) float k_lds[L][kKeyStride];   // the queries first, then the keys
     __shared__ __align__(16) float p_lds[G][L];
     __shared__ typename ScoreTiles<G, L, NT>::Part sc_lds[ScoreTiles<G, L, NT>::P];   // partial score tiles
     __shared__ float acc_lds[HALVES > 1 ? HALVES - 1 : 1][HALVES > 1 ? G : 1][HALVES > 1 ? D : 1];
@@ -468,11 +477,19 @@ __global__ __launch_bounds__(G * L * kPairLanes) void decode_split(
             }
         }
     }
+    // The queries pass through the key tile's LDS into each lane's MFMA operands while the keys are still arriving:
+    // without a tile of their own, 39 KB a workgroup, four fit a CU.
+    using Tiles = ScoreTiles<G, L, NT>;
+    static_assert(G <= L, "queries fit the key tile");
+    float4 qb[Tiles::DP / 16];
 #pragma unroll
     for (int i = 0; i < QCH; ++i) {
         const int c = tid + i * NT;
-        q_lds[c / D4][c % D4] = qr[i];
+        *reinterpret_cast<float4*>(&k_lds[c / D4][4 * (c % D4)]) = qr[i];
     }
+    __syncthreads();
+    Tiles::template load_q<kKeyStride>(&k_lds[0][0], tid, qb);
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < KCH; ++i) {
         const int c = tid + i * NT;
@@ -486,8 +503,7 @@ __global__ __launch_bounds__(G * L * kPairLanes) void decode_split(
     const int pair = tid / kPairLanes, r = tid % kPairLanes;
     const int hh = pair / L, tt = pair % L;
     const bool valid = t0 + tt < n_keys;
-    using Tiles = ScoreTiles<G, L, NT>;
-    Tiles::run(q_lds, k_lds, sc_lds, tid);
+    Tiles::run(qb, k_lds, sc_lds, tid);
     __syncthreads();
     const float dot = Tiles::dot(sc_lds, hh, tt);
     const float sc = valid ? dot * scale : -INFINITY;
@@ -559,8 +575,11 @@ __global__ __launch_bounds__(G * L * kPairLanes) void decode_split(
 // The split pass stores the partials as [head][16-column block][split][16],
 // so a workgroup reads one contiguous run of splits x 64 bytes.
 constexpr int kCombineCols = 16;
-constexpr int kCombineBatch = 2;   // splits per thread and memory round trip
 
+// BATCH: splits per thread and memory round trip (64 BATCH splits a round for the workgroup). Up to 128 splits one
+// round of 2 has them all (9.2 us for the decode at 2048 keys either way); above, rounds of 8 and 16 statistics in
+// flight: the decode of 30011 keys 36.4 -> 34.6 us, of 6001 keys 13.7 -> 13.6.
+template <int BATCH>
 __global__ __launch_bounds__(kBlock) void decode_combine(const float* __restrict__ ws_acc,
                                                          const float* __restrict__ ws_m,
                                                          const float* __restrict__ ws_l,
@@ -568,7 +587,7 @@ __global__ __launch_bounds__(kBlock) void decode_combine(const float* __restrict
                                                          int splits) {
     constexpr int D = kMaxDim, NCB = D / kCombineCols, NW = kBlock / kWave;
     constexpr int SPW = kWave / 4;   // splits per wave and round (4 lanes per split)
-    constexpr int STEP = SPW * NW * kCombineBatch;
+    constexpr int STEP = SPW * NW * BATCH;
     __shared__ float4 zpart[NW][4];
     __shared__ float tpart[NW][4];
     const int h = blockIdx.x / NCB, cb = blockIdx.x - h * NCB;
@@ -586,11 +605,11 @@ __global__ __launch_bounds__(kBlock) void decode_combine(const float* __restrict
         for (int i = 0; i < 4; ++i) gv[i] = gate[j0 + i];
     }
     // the first batch's partials and statistics, requested with the max's loads
-    float4 a[kCombineBatch];
-    float mi[kCombineBatch], li[kCombineBatch];
+    float4 a[BATCH];
+    float mi[BATCH], li[BATCH];
     auto load_batch = [&](int base) {
 #pragma unroll
-        for (int i = 0; i < kCombineBatch; ++i) {
+        for (int i = 0; i < BATCH; ++i) {
             const size_t sc = static_cast<size_t>(min(base + i * SPW * NW, splits - 1));
             a[i] = ld4(accp + sc * kCombineCols);
             mi[i] = ws_m[s0 + sc];
@@ -599,13 +618,17 @@ __global__ __launch_bounds__(kBlock) void decode_combine(const float* __restrict
     };
     load_batch(first);
     float M = -INFINITY;
-    for (int s = lane; s < splits; s += kWave) M = fmaxf(M, ws_m[s0 + s]);
+    constexpr int MB = BATCH == 2 ? 2 : 16;   // loads in flight; clamped repeats do not change a maximum
+    for (int s = lane; s < splits; s += MB * kWave) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) M = fmaxf(M, ws_m[s0 + min(s + i * kWave, splits - 1)]);
+    }
     M = wave_max(M);
     float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
     float t = 0.f;
     for (int base = first;;) {
 #pragma unroll
-        for (int i = 0; i < kCombineBatch; ++i) {
+        for (int i = 0; i < BATCH; ++i) {
             const float e = base + i * SPW * NW < splits ? expf(mi[i] - M) : 0.f;
             t = __builtin_fmaf(e, li[i], t);
             z = make_float4(__builtin_fmaf(e, a[i].x, z.x), __builtin_fmaf(e, a[i].y, z.y),
@@ -829,7 +852,11 @@ int split_combine(const float* q, std::conditional_t<NR, float*, const float*> k
                                                                       n_keys, splits, scale, nr, den);
     int st = check_launch("attn_decode");
     if (st) return st;
-    decode_combine<<<heads * (kMaxDim / kCombineCols), kBlock, 0, s>>>(acc, m, l, gate, out, splits);
+    const unsigned cgrid = heads * (kMaxDim / kCombineCols);
+    if (splits <= 128)
+        decode_combine<2><<<cgrid, kBlock, 0, s>>>(acc, m, l, gate, out, splits);
+    else
+        decode_combine<8><<<cgrid, kBlock, 0, s>>>(acc, m, l, gate, out, splits);
     return check_launch("attn_decode");
 }
 

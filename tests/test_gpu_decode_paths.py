@@ -1,4 +1,5 @@
-"""Decode kernels at the edges of their shape rules: the MoE down projection with the 512-wide shared expert."""
+"""Decode kernels at the edges of their shape rules: the attention combine's batches (128 splits
+of 32 or 16 keys, more, many), and the MoE down projection with the 512-wide shared expert."""
 
 from __future__ import annotations
 
@@ -10,6 +11,27 @@ from conftest import assert_bits_equal
 from qwen35_hip import ops, synth
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv,pos", [
+    (16, 2, 0), (16, 2, 31), (16, 2, 4095), (16, 2, 4096), (16, 2, 16383), (16, 2, 16384), (16, 2, 20011),
+    (32, 2, 2047), (32, 2, 2048), (16, 1, 9000),
+])
+def test_attn_decode_splits(heads, kv, pos):
+    """Against float64 under the dot-product bar, |got - ref| <= 1e-5 max(|ref|, c) with c = sum_t p_t |v_t| (times the
+    gate): the fp32 sum over keys and the scores' rounding err by ulps of its terms, and an average over many keys is
+    far below them (20012 keys of N(0, 1): rms 0.01 of c)."""
+    g = torch.Generator(device="cuda").manual_seed(pos + heads)
+    q = torch.randn(heads * 256, generator=g, device="cuda")
+    k = torch.randn((pos + 1) * kv * 256, generator=g, device="cuda")
+    v = torch.randn((pos + 1) * kv * 256, generator=g, device="cuda")
+    gate = torch.randn(heads * 256, generator=g, device="cuda")
+    out = ops.attn_decode(q, k, v, heads, kv, 256, pos, gate=gate)
+    kk = k.double().view(pos + 1, kv, 256).permute(1, 2, 0).contiguous()
+    p = torch.softmax(torch.bmm(q.double().view(kv, heads // kv, 256), kk) / 16, -1)
+    vv, sg = v.double().view(pos + 1, kv, 256).transpose(0, 1).contiguous(), torch.sigmoid(gate.double())
+    ref, c = torch.bmm(p, vv).view(-1) * sg, torch.bmm(p, vv.abs()).view(-1) * sg
+    assert bool(((out.double() - ref).abs() <= 1e-5 * torch.maximum(ref.abs(), c)).all())
 
 
 @pytest.mark.parametrize("td,ts", [("Q4_K", "Q4_K"), ("Q4_K", "Q6_K"), ("Q6_K", "Q4_K"), ("Q6_K", "Q6_K")])
