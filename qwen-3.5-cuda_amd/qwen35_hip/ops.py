@@ -22,14 +22,16 @@ BF16 = torch.bfloat16  # bf16 storage (fp32 math inside the kernels)
 GGML_TYPES = {"F32": 0, "F16": 1, "Q4_0": 2, "Q5_0": 6, "Q8_0": 8, "Q4_K": 12, "Q5_K": 13, "Q6_K": 14, "BF16": 30}
 
 
-def _stream(stream) -> ctypes.c_void_p:
+def _stream(stream) -> int:
+    """The hipStream_t to enqueue on. The raw handle of the current device's current stream: building a
+    torch.cuda.Stream for it (torch.cuda.current_stream()) takes 2.8 us a call, this 0.1."""
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return stream.cuda_stream
 
 
-def _p(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
+def _p(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _dev(*ts: torch.Tensor, dtype=None) -> None:
