@@ -59,6 +59,8 @@ namespace {
 constexpr int kC = 64;                        // tokens per chunk
 constexpr int kDK = 128;                      // key dim of the chunked path
 constexpr int kNB = 16;                       // state columns per workgroup (kernel B)
+constexpr int kLoopRows = 28;       // up to this many rows the token loop runs (below)
+constexpr int kSpreadGroups = 256;  // prep workgroups at one per CU
 constexpr int kThreads = 256;                 // prep
 constexpr int kWalkThreads = 512;             // state walk: two waves per SIMD
 constexpr int64_t kMaxWalkStride = 0x7fffffff / (4 * 64);   // floats; 64 rows of 4-byte elements below 2^31 bytes
@@ -172,6 +174,10 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
     float(*Ab)[kLdA] = reinterpret_cast<float(*)[kLdA]>(kat);
     float(*T)[kLdA] = reinterpret_cast<float(*)[kLdA]>(kat + kC * kLdA);
     const int c = blockIdx.x, src = blockIdx.y;   // chunk, key head
+    // With gridDim.z > 1 a key head's value heads are dealt to that many workgroups, each with the products of its
+    // own; only the first writes K and Q out.
+    const int h0 = src + key_heads * static_cast<int>(blockIdx.z), hstep = key_heads * static_cast<int>(gridDim.z);
+    const bool writes_kq = blockIdx.z == 0;
     const int t0 = c * kC;
     const int lane = threadIdx.x & 63;
     const int wv = wave_in_block();
@@ -191,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
             dn = decay[static_cast<int64_t>(t) * value_heads + h];
         }
     };
-    load_gates(src);
+    load_gates(h0);
 
     // Lower-triangle 16x16 tiles (mt >= nt) of K K^T and Q K^T. Wave w loads
     // the K and Q rows of tokens 16w .. 16w+15 once (lane: token 16w + L%16,
@@ -238,13 +244,17 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
             for (int kb = 0; kb < 4; ++kb) {
                 u4_t hi, lo;
                 split8(kr + 8 * kb, eK, hi, lo);
-                *reinterpret_cast<u4_t*>(rk + 2048 * kb) = hi;
-                *reinterpret_cast<u4_t*>(rk + 2048 * kb + 1024) = lo;
+                if (writes_kq) {
+                    *reinterpret_cast<u4_t*>(rk + 2048 * kb) = hi;
+                    *reinterpret_cast<u4_t*>(rk + 2048 * kb + 1024) = lo;
+                }
                 KF[(wv * 8 + 2 * kb) * 64 + lane] = hi;
                 KF[(wv * 8 + 2 * kb + 1) * 64 + lane] = lo;
                 split8(qr + 8 * kb, eQ, qf[2 * kb], qf[2 * kb + 1]);
-                *reinterpret_cast<u4_t*>(rq + 2048 * kb) = qf[2 * kb];
-                *reinterpret_cast<u4_t*>(rq + 2048 * kb + 1024) = qf[2 * kb + 1];
+                if (writes_kq) {
+                    *reinterpret_cast<u4_t*>(rq + 2048 * kb) = qf[2 * kb];
+                    *reinterpret_cast<u4_t*>(rq + 2048 * kb + 1024) = qf[2 * kb + 1];
+                }
             }
         }
         __syncthreads();   // every tile's K pairs in LDS
@@ -280,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
     // The products depend on the key head only: every value head h with
     // h % key_heads == src (the heads that read this key head) takes them from
     // here, so K and Q are read and multiplied once per key head.
-    for (int h = src; h < value_heads; h += key_heads) {
+    for (int h = h0; h < value_heads; h += hstep) {
         float* wsc = ws + (static_cast<size_t>(c) * value_heads + h) * kWsFloats;
         float* Tp = wsc;
         float* Bm = wsc + kC * kC;
@@ -291,7 +301,7 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
             sb[threadIdx.x] = bn;
             sd[threadIdx.x] = dn;
         }
-        if (h + key_heads < value_heads) load_gates(h + key_heads);
+        if (h + hstep < value_heads) load_gates(h + hstep);
         __syncthreads();
 
         // Rows 16wv .. 16wv+15 per wave, lane i = column i: R[t][i] as a running
@@ -869,11 +879,21 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     const size_t need = qwen_gdn_recurrent_chunked_workspace_bytes(rows, value_heads);
     QK_REQUIRE(workspace_bytes >= need, "gdn_recurrent_chunked: workspace of %zu bytes, %zu needed", workspace_bytes,
                need);
+    // A few tokens: the token loop, 0.25 us a token from 8 us, against the two launches' 15.6 us for one chunk (9
+    // tokens 10.1 us, 32 tokens 16.0 against 15.6, 48 tokens 20.0 against 16.0). Its error is the smaller one.
+    if (rows <= kLoopRows)
+        return qwen_gdn_recurrent_rows(state, q, k, v, beta, decay, out, rows, key_heads, value_heads, key_dim,
+                                       value_dim, qkv_stride, out_stride, stream);
     const hipStream_t s = as_stream(stream);
     const int nchunks = (rows + kC - 1) / kC;
     float* ws = static_cast<float*>(workspace);
     unsigned char* kq = static_cast<unsigned char*>(workspace) + static_cast<size_t>(nchunks) * value_heads * kWsFloats * sizeof(float);
-    gdn_chunk_prep<<<dim3(nchunks, std::min(key_heads, value_heads)), kThreads, 0, s>>>(
+    // A value head's share is a third of a prep workgroup's serial chain: while one workgroup per (chunk, value head)
+    // has a CU to itself, a key head's value heads go to workgroups of their own (both launches, 64 tokens 20.0 ->
+    // 16.2 us, 128 24.1 -> 20.7, 400 38.9 -> 36.3; two to a CU gains nothing, 777 tokens 52.1 -> 52.9).
+    const int kh = std::min(key_heads, value_heads), group = (value_heads + kh - 1) / kh;
+    const bool spread = static_cast<int64_t>(nchunks) * kh * group <= kSpreadGroups;
+    gdn_chunk_prep<<<dim3(nchunks, kh, spread ? group : 1), kThreads, 0, s>>>(
         q, k, beta, decay, ws, kq, rows, key_heads, value_heads, qkv_stride);
     // One row: its stride is not used to step between rows, but the walk's
     // buffer range is one stride long, so it must cover the row's q, k, v and out.

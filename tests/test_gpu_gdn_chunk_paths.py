@@ -1,0 +1,54 @@
+"""The chunked recurrence at the edges of its routes: the token loop up to 28 rows, prep workgroups per value head
+while they have a CU each, one per key head above (and with one, two or three value heads per key head)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import assert_bits_equal
+from qwen35_hip import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,kh,vh", [(1, 16, 32), (28, 16, 32), (29, 16, 32), (64, 4, 4), (65, 4, 12), (512, 16, 32),
+                                        (513, 16, 32), (100, 8, 4)])
+def test_chunked_routes(rows, kh, vh):
+    """Output and state against the recurrence in float64, under the bar of the other recurrence tests: 1e-5 of the
+    larger of the value and its condition scale (here each head's largest terms, |q||S| of the readout)."""
+    g = torch.Generator(device="cuda").manual_seed(rows * 7 + vh)
+    n = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    qk = torch.nn.functional.normalize(n(rows, 2 * kh, 128), dim=-1)
+    qk[:, :kh] /= 128 ** 0.5
+    qkv = torch.cat([qk.reshape(rows, -1), n(rows, vh * 128)], 1).contiguous()
+    beta, decay = torch.sigmoid(n(rows, vh)), torch.exp(-torch.rand((rows, vh), generator=g, device="cuda") * 2)
+    state = 0.1 * n(vh, 128, 128)
+    got_s = state.clone()
+    got = ops.gdn_recurrent_chunked(got_s, qkv, beta, decay, kh, vh, 128, 128)
+    idx = torch.arange(vh, device="cuda") % kh
+    S, out, cond = state.double(), [], []
+    for t in range(rows):
+        q, k = qk[t, :kh][idx].double(), qk[t, kh:][idx].double()
+        v = qkv[t, 2 * kh * 128:].view(vh, 128).double()
+        S = S * decay[t].double()[:, None, None]
+        delta = (v - torch.bmm(k[:, None], S)[:, 0]) * beta[t].double()[:, None]
+        S = S + k[:, :, None] * delta[:, None, :]
+        out.append(torch.bmm(q[:, None], S)[:, 0])
+        cond.append(torch.bmm(q.abs()[:, None], S.abs())[:, 0])
+    ref, c = torch.stack(out).view(rows, -1), torch.stack(cond).view(rows, -1)
+    assert bool(((got.double() - ref).abs() <= 1e-5 * torch.maximum(ref.abs(), c)).all())
+    rms = S.square().mean((1, 2), keepdim=True).sqrt()
+    assert bool(((got_s.double() - S).abs() <= 1e-5 * torch.maximum(S.abs(), rms)).all())
+
+
+def test_up_to_28_rows_are_the_token_loop():
+    g = torch.Generator(device="cuda").manual_seed(5)
+    qkv = torch.randn((28, 8192), generator=g, device="cuda")
+    beta, decay = torch.rand((2, 28, 32), generator=g, device="cuda")
+    state = torch.randn((32, 128, 128), generator=g, device="cuda")
+    a, b = state.clone(), state.clone()
+    one = ops.gdn_recurrent_chunked(a, qkv, beta, decay, 16, 32, 128, 128)
+    two = ops.gdn_recurrent_rows(b, qkv, beta, decay, 16, 32, 128, 128)
+    assert_bits_equal(one.cpu().numpy(), two.cpu().numpy(), what="out")
+    assert_bits_equal(a.cpu().numpy(), b.cpu().numpy(), what="state")
