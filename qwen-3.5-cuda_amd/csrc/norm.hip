@@ -126,6 +126,7 @@ __global__ __launch_bounds__(STAGE ? kStageWaves * kWave : kWave) void rmsnorm_r
 // takes 1.87 us).
 constexpr int kSplitWaves = 2;   // the two chunk sets of row_sumsq
 constexpr int kSplitRows = 256;
+constexpr int kResidualSplitRows = 256;   // rows up to which a residual row has a wave per chunk
 
 // FULL: n4 == MAXC * kSplitWaves * 64 (every chunk inside the row: no clamps or
 // masks, so the loads take immediate offsets and the sum needs no selects).
@@ -253,6 +254,33 @@ __global__ __launch_bounds__(STAGE ? kStageWaves * kWave : kWave) void residual_
             st4_nt(normed + base + 4 * i, make_float4(v[c].x * r * wv[c].x, v[c].y * r * wv[c].y,
                                                       v[c].z * r * wv[c].z, v[c].w * r * wv[c].w));
     }
+}
+
+// Few rows (a decode token's one, above all): a wave per 64-float4 chunk, WAVES of them a row. Each lane's square sums
+// meet in LDS and every wave adds them in chunk order and over the lanes as the one-wave form does, so the bits are
+// its bits. One load round trip of three 16-byte loads instead of 24: one row of 2048
+// 1.84 us, 2.28 with one wave (4096: 2.32 and 3.12; 256 rows of 2048: 2.53 and 2.82; from there on equal).
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void residual_rmsnorm_f32_row(
+    const float* __restrict__ x, const float* __restrict__ b, const float* __restrict__ w, float* __restrict__ resid,
+    float* __restrict__ normed, int n, float eps) {
+    __shared__ float part[WAVES][kWave];
+    const int lane = threadIdx.x & 63, wv = wave_in_block();
+    const int i = wv * kWave + lane, n4 = n >> 2;
+    const int ic = min(i, n4 - 1);
+    const size_t base = static_cast<size_t>(blockIdx.x) * n;
+    const float4 a = ld4_nt(x + base + 4 * ic), d = ld4_nt(b + base + 4 * ic), wt = ld4(w + 4 * ic);
+    const float4 v = make_float4(a.x + d.x, a.y + d.y, a.z + d.z, a.w + d.w);
+    part[wv][lane] = i < n4 ? sumsq4(v) : 0.f;
+    if (i < n4) st4_nt(resid + base + 4 * i, v);
+    __syncthreads();
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < WAVES; ++c) ss += part[c][lane];
+    ss = group_sum<kWave>(ss);
+    const float r = rsqrtf(div_n(ss, n) + eps);
+    if (i < n4)
+        st4_nt(normed + base + 4 * i, make_float4(v.x * r * wt.x, v.y * r * wt.y, v.z * r * wt.z, v.w * r * wt.w));
 }
 
 __global__ __launch_bounds__(kBlock) void residual_rmsnorm_f32_any(const float* __restrict__ x,
@@ -500,7 +528,14 @@ int qwen_residual_rmsnorm_rows_f32(const float* x, const float* branch, const fl
     const int n4 = n / 4;
     const bool vec = n % 4 == 0 && aligned16(x) && aligned16(branch) && aligned16(weight) && aligned16(resid) &&
                      aligned16(normed);
-    if (vec && n4 <= 16 * kWave) {
+    if (vec && n4 > 2 * kWave && n4 <= 16 * kWave && rows <= kResidualSplitRows) {
+        if (n4 <= 4 * kWave)
+            residual_rmsnorm_f32_row<4><<<rows, 4 * kWave, 0, s>>>(x, branch, weight, resid, normed, n, eps);
+        else if (n4 <= 8 * kWave)
+            residual_rmsnorm_f32_row<8><<<rows, 8 * kWave, 0, s>>>(x, branch, weight, resid, normed, n, eps);
+        else
+            residual_rmsnorm_f32_row<16><<<rows, 16 * kWave, 0, s>>>(x, branch, weight, resid, normed, n, eps);
+    } else if (vec && n4 <= 16 * kWave) {
         launch_row_shape(rows, size_t(n4) * 16, [&](auto stage, dim3 grid, dim3 block, size_t lds) {
             constexpr bool S = decltype(stage)::value;
             if (n4 <= kWave)

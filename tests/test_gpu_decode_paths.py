@@ -1,5 +1,6 @@
 """Decode kernels at the edges of their shape rules: the attention combine's batches (128 splits
-of 32 or 16 keys, more, many), and the MoE down projection with the 512-wide shared expert."""
+of 32 or 16 keys, more, many), the MoE down projection with the 512-wide shared expert, and the
+residual norm's form for few rows."""
 
 from __future__ import annotations
 
@@ -61,3 +62,20 @@ def test_down_combine_small_shared_expert(td, ts, k, dm):
         got = ops.moe_down_combine(wd, td, E * dm * inter, dm * inter, E, idx, wts, hid, inter, wsd, ts, dm * S, shid,
                                    logit, dm)
         assert_bits_equal(got.cpu().numpy(), separate(idx).cpu().numpy(), what=f"{td} {ts} k={k} {dm}")
+
+
+@pytest.mark.parametrize("n", [512, 516, 1024, 2048, 2052, 4096])
+def test_residual_norm_of_few_rows_keeps_the_bits(n):
+    """Up to 256 rows a row has a wave per chunk, above one wave: a row gives the same bits alone, among 256 and among
+    257, also in place."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, b = torch.randn((2, 257, n), generator=g, device="cuda")
+    w = torch.randn(n, generator=g, device="cuda")
+    many = ops.residual_rmsnorm_rows(x, b, w)
+    for rows in (1, 3, 256):
+        for got, ref in zip(ops.residual_rmsnorm_rows(x[:rows].contiguous(), b[:rows].contiguous(), w), many):
+            assert_bits_equal(got.cpu().numpy(), ref[:rows].cpu().numpy(), what=f"{rows} x {n}")
+    y = x[:5].clone()
+    resid, normed = ops.residual_rmsnorm_rows(y, b[:5].contiguous(), w, resid=y)
+    assert_bits_equal(resid.cpu().numpy(), many[0][:5].cpu().numpy(), what="resid in place")
+    assert_bits_equal(normed.cpu().numpy(), many[1][:5].cpu().numpy(), what="normed in place")
