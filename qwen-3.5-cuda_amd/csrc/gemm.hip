@@ -18,8 +18,7 @@
 //         m_g exact, S_g 2^-5 split into two fp16 parts like x (22 bits).
 //   Q6_K: (q - 32) * sc reaches 12 bits, so B = Bh + Bl (exact, |Bl| <= 1) and
 //         three products per operand pair, h Bh + l Bh + h Bl (l Bl is below
-//         2^-22 of h Bh); the wide tiles instead take B = q - 32 and apply the
-//         scale per 16-element group, y += (d sc) P_g (one FMA): fewer MFMAs.
+//         2^-22 of h Bh).
 // The result is scaled back by 2^-e (exact). Products of fp16 values are exact
 // in the MFMA's fp32 accumulation, so the roundings are those of an fp32 sum.
 //
@@ -30,14 +29,14 @@
 //
 // Four kernels, by token count (gemm_path below has the lines and both sides'
 // times): gemm_few (up to 16 tokens, 160 from K = 4096) converts x itself and
-// splits K over its waves; gemm_kquant splits K in 4 or 2 slices over waves of
-// a workgroup with the tile shape that fills the 256 CUs in the fewest rounds;
-// gemm_q4k_wide and gemm_q6k_wide (128 x 256 tiles) take long prompts.
+// splits K over its waves; gemm_kquant splits K in 4, 2 or no slices over waves
+// of a workgroup with the tile shape that fills the 256 CUs in the fewest
+// rounds; gemm_q4k_wide and gemm_q6k_wide (128 x 256 tiles) take long prompts.
 // Measured, us for the GDN layer's input projections (M = 8192, 4096, 32, 32 at
 // K = 2048, one call) and output projection (M = 2048 at K = 4096), Q4_K:
 //   tokens                            9        77        300       777      4096
 //   one form for all (before)     103 / 30  71 / 131  77 / 134  146 / 136  510 / 175
-//   these kernels                  13 / 12  31 /  21  56 /  42  137 /  58  413 / 152
+//   these kernels                  13 / 12  31 /  21  56 /  42  132 /  62  438 / 152
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
@@ -54,7 +53,6 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kGemmMinRows = 16;   // fewer tokens need no workspace
 constexpr int kGemmMaxRows = 65535 * 128;
@@ -332,8 +330,10 @@ struct WScale<kQ6_K> {
     template <int U>
     __device__ __forceinline__ void set(const WBlock<kQ6_K>& b, int lk) {
         const uint32_t w = U < 2 ? b.sc.x : b.sc.y;   // scales 2 U, 2 U + 1 of the half
-        const uint32_t v = ((w >> (16 * (U & 1) + 8 * (lk & 1))) & 0xffu) ^ 0x80u;
-        s = h2(v * 0x00010001u + 0x64006400u) - dup2(1152.f);   // signed 8 bits, exact
+        s = from((w >> (16 * (U & 1) + 8 * (lk & 1))) & 0xffu);
+    }
+    static __device__ __forceinline__ f16x2_t from(uint32_t byte) {
+        return h2((byte ^ 0x80u) * 0x00010001u + 0x64006400u) - dup2(1152.f);   // signed 8 bits, exact
     }
 };
 
@@ -371,27 +371,39 @@ __device__ __forceinline__ void decode_centred(const WBlock<kQ4_K>& b, const WSc
     __builtin_memcpy(&B[0], e, 16);
 }
 
-// (q - 32) sc in two fp16 parts, exactly: magnitudes up to 2048 fit the first one.
-template <int U, int J>
-__device__ __forceinline__ void decode(const WBlock<kQ6_K>& b, const WScale<kQ6_K>& sc, uint32_t k64, f16x8_t (&B)[2]) {
+// (q - 32) sc in two fp16 parts, exactly: magnitudes up to 2048 fit the first one. wd, hd: the ql and qh words of the
+// operand's quants.
+template <int U>
+__device__ __forceinline__ void decode_q6(const uint32_t (&wd)[2], const uint32_t (&hd)[2], f16x2_t s, uint32_t k64,
+                                          uint32_t kf, uint32_t k30, f16x8_t (&B)[2]) {
+    f16x2_t q[4], p[4];
     uint32_t e[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t w = word_of(b.q[U & 1], 2 * J + i), h = word_of(b.qh, 2 * J + i);
-#pragma unroll
-        for (int o = 0; o < 2; ++o) {
-            const uint32_t n = (w >> (8 * o + 4 * (U >> 1))) & 0x000f000fu;
-            constexpr int up = 4 - 2 * U;   // bits 2 U of qh to bits 4, 5
-            const int sh = up - 8 * o;
-            const uint32_t t = (sh >= 0 ? h << (sh & 31) : h >> (-sh & 31)) & 0x00300030u;
-            const f16x2_t q = h2(n | (t | k64)) - dup2(1056.f);
-            const f16x2_t p = q * sc.s;
-            e[2 * i + o] = w2(p);
-            l[2 * i + o] = w2(fma2(q, sc.s, -p));
-        }
+    for (int i = 0; i < 4; ++i) {   // bytes (0, 2), (1, 3) of both words
+        const int o = i & 1;
+        constexpr int up = 4 - 2 * U;   // bits 2 U of qh to bits 4, 5
+        const int sh = up - 8 * o;
+        const uint32_t h = hd[i >> 1];
+        uint32_t t = ((sh >= 0 ? h << (sh & 31) : h >> (-sh & 31)) & k30) | k64;
+        asm("" : "+v"(t));   // two v_and_or_b32 rather than two ands and an or3
+        q[i] = h2(((wd[i >> 1] >> (8 * o + 4 * (U >> 1))) & kf) | t) - dup2(1056.f);
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        p[i] = q[i] * s;
+        e[i] = w2(p[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l[i] = w2(fma2(q[i], s, -p[i]));
     __builtin_memcpy(&B[0], e, 16);
     __builtin_memcpy(&B[1], l, 16);
+}
+
+template <int U, int J>
+__device__ __forceinline__ void decode(const WBlock<kQ6_K>& b, const WScale<kQ6_K>& sc, uint32_t k64, f16x8_t (&B)[2]) {
+    const uint32_t wd[2] = {word_of(b.q[U & 1], 2 * J), word_of(b.q[U & 1], 2 * J + 1)};
+    const uint32_t hd[2] = {word_of(b.qh, 2 * J), word_of(b.qh, 2 * J + 1)};
+    decode_q6<U>(wd, hd, sc.s, k64, 0x000f000fu, 0x00300030u, B);
 }
 
 // Q4_K's min terms, sum_g m_g S_g of a block, as one v_mfma_f32_16x16x16_f16 per tile: k = 8 groups x the two fp16
@@ -1148,60 +1160,32 @@ __global__ __launch_bounds__(kQ4Block, 1) void gemm_q4k_wide(const GemmJobs jobs
 }
 
 // ------------------------------------------------------------------ Q6_K, many tokens
-// Bytes (0, 2) and (1, 3) of n placed under `hi` (byte values 0 or 0x64).
-__device__ __forceinline__ uint32_t bytes02(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04020400u); }
-__device__ __forceinline__ uint32_t bytes13(uint32_t hi, uint32_t n) { return __builtin_amdgcn_perm(hi, n, 0x04030401u); }
-
-__device__ __forceinline__ uint32_t hadd2(uint32_t w, _Float16 c) {
-    const f16x2_t r = __builtin_bit_cast(f16x2_t, w) + f16x2_t{c, c};
-    return __builtin_bit_cast(uint32_t, r);
-}
-
-// fp16 q - 32 of four 6-bit quants (bytes of q): two words in the order (0, 2), (1, 3).
-__device__ __forceinline__ void q6_operand(uint32_t q, uint32_t& w02, uint32_t& w13) {
-    w02 = hadd2(bytes02(0x64646464u, q), static_cast<_Float16>(-1056.0f));
-    w13 = hadd2(bytes13(0x64646464u, q), static_cast<_Float16>(-1056.0f));
-}
-
-// Element i of a block (src/cuda/matmul_q4.cu:105-126): ql byte 64(i/128) +
-// 32((i%128)/32 & 1) + i%32 (low nibble in quarters 0, 1 of a half, high in
-// 2, 3), qh byte 128 + 32(i/128) + i%32 bits 2*quarter, scale byte 192 + i/16,
-// d at 208. Stage sg of a block (elements 32 sg ..) is half sg/4, quarter
-// sg%4; lane (l32, lh) of step h takes elements 32 sg + 16 h + 8 lh .. +7:
-// eight consecutive ql and qh bytes, scale 2 sg + h.
-//
-// A workgroup (8 waves, one per CU) owns 128 tokens x 256 weight rows; wave w
-// owns rows 64 (w % 4) .. +63 for tokens 64 (w / 4) .. +63 (2 x 2 tiles of
-// 32 x 32 on v_mfma_f32_32x32x16_f16, k = one 16-element scale group, so each
-// group's product is scaled by d * sc in fp32 before it joins the sums). x goes
-// through LDS from registers (the next stage loaded while the current one
-// computes). The quant bytes and scales of a half-block (4 stages: 64 ql
-// bytes, both nibbles; 32 qh bytes; the 16 scales and d) are staged per row in
-// LDS with coalesced 16-byte loads four stages ahead; waves w and w + 4 (same
-// rows) split the next stage's B decode (wave w / 4 takes step h = w / 4) into
-// an LDS slot both read after the stage's barrier.
+// A workgroup (8 waves, one per CU) owns 128 tokens x 256 weight rows; wave w owns rows 64 (w % 4) .. +63 for tokens
+// 64 (w / 4) .. +63, as 4 x 4 tiles, with the products and sums of gemm_kquant<kQ6_K, 4, 2, 1, 1> in its order (the
+// same bits). A block's rows are only 2-byte aligned, so weights and x go global -> VGPR -> LDS, the quant bytes and
+// scales in the lane order that decodes them. Work goes by row tile: the 12 products of one tile of 16 rows with the
+// wave's 4 token tiles run while the next row tile's operand is decoded (28 VALU instructions) and the one after it
+// is read from LDS; the A operands (4 tiles x 2 parts) stay in registers for the depth and the last row tile's
+// products release them to the next depth's. The barrier stands in the middle of a depth, where the LDS reads before
+// it are old: x needs two slots, and the ql bytes one (those of odd u are replaced while even u run and the other way
+// round). A round of 256 workgroups at K = 2048: 90 us, 49 of them the MFMAs' own time, two rounds of 64 x 256 tiles 134.
+// Before, B = q - 32 with a product and an FMA per 16 elements took 115 (fewer MFMAs, but 128 FMAs a stage beside 16
+// of 32 x 32): M = 8192, 4096, 32, 32 at 500, 1500 and 4096 tokens 123, 348, 702 us then, 92, 290, 588 now.
 constexpr int kQ6Waves = 8;
 constexpr int kQ6Block = kQ6Waves * kWave;
 constexpr int kQ6R = 256;                    // weight rows per workgroup (64 per wave)
 constexpr int kQ6T = 128;                    // tokens per workgroup
-constexpr int kXRow = 40;                    // halves per staged token row (32 + 8 padding)
-// A thread's share of one stage of x: 16 halves of one fp16 part of its token.
-struct XRegs {
-    uint4 a, b;
-};
-typedef uint16_t Q6XStage[2][kQ6T][kXRow];   // one stage of x: the two fp16 parts
-typedef f16x8_t Q6BSlot[4][2][2][kWave];     // B operands: [row group][step h][row tile][lane]
-// One half-block of a row: ql bytes 64 half .. +63 | qh bytes 128 + 32 half .. +31 |
-// scales (block bytes 192..207) | block bytes 194..209 (d in the last two) | pad (row
-// stride 36 dwords spreads a wave's 32 rows over the LDS banks)
-typedef uint8_t Q6WSlot[kQ6R][144];
+typedef uint4 Q6XSlot[kQ6T / kTile][2][kWave];   // one depth of x: [tile][fp16 part][lane]
+typedef uint2 Q6QSlot[2][kQ6R / kTile][kWave];   // 16 bytes a lane: [half, the depth of its u][row tile][lane]
 
-__global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k_wide(const GemmJobs jobs, const int* __restrict__ ex,
-                                                         const uint8_t* __restrict__ xp, const float* __restrict__ x,
-                                                         int T, int K) {
-    __shared__ __align__(16) Q6XStage xs[2];
-    __shared__ __align__(16) Q6BSlot bs[2];
-    __shared__ __align__(16) Q6WSlot wsl[2];
+__global__ __launch_bounds__(kQ6Block) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_q6k_wide(
+    const GemmJobs jobs, const int* __restrict__ ex, const uint8_t* __restrict__ xp, const float* __restrict__ x, int T,
+    int K) {
+    __shared__ __align__(16) Q6XSlot xs[2];
+    __shared__ __align__(16) Q6QSlot ql[2];        // of even and odd u
+    __shared__ __align__(16) Q6QSlot qh[2];        // by block
+    __shared__ __align__(16) uint8_t scl[2][kQ6R][16];
+    __shared__ uint16_t dl[2][kQ6R];
     const int cols = jobs.start[jobs.n];
     const int tb = static_cast<int>(blockIdx.x) / cols;
     const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x) - tb * cols);
@@ -1209,165 +1193,216 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k_wide(const GemmJobs jobs
     float* __restrict__ y = job.y;
     const int M = job.M;
     const uint64_t ub0 = job.ub0;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
-    const int rg = wv & 3, th = wv >> 2;                       // row group, token half (= decode step)
-    const int t0w = tb * kQ6T;
-    const int tw = t0w + 64 * th;
-    const int rw0 = job.mb * kQ6R;
-    const int r0 = rw0 + 64 * rg;
-    const int nb = K >> 8, nst = K >> 5, nhb = nst >> 2;
-    const int tok = tid >> 2, part = tid & 3;
-    // stage g = 8 block + 4 h + u is the natural 32 elements 32 g ..: the thread's 16 halves (fp16 part p, k half
-    // l = lk % 2) are the pieces of depths 2 u, 2 u + 1 at lk = 2 h + l
-    const int xt = min(t0w + tok, T - 1) / kTile, xlr = min(t0w + tok, T - 1) % kTile;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = wave_in_block();
+    const int rg = wv & 3, th = wv >> 2;                       // row group, token half
+    const int t0w = tb * kQ6T;                                 // the workgroup's first token
+    const int tw = t0w + 64 * th;                              // this wave's first token
+    const int rw0 = job.mb * kQ6R;                             // the workgroup's first row
+    const int r0 = rw0 + 64 * rg;                              // this wave's first row
+    const int nb = K >> 8, nst = K >> 5;
+
+    // x: wave wv brings tile wv of the workgroup (the last one again past the end), both parts
+    const int xt = min(tb * (kQ6T / kTile) + wv, (T + kTile - 1) / kTile - 1);
     const int xrn = min(kTile, T - kTile * xt);
-    const uint8_t* xbase = xp + tile_base(xt, K) + 16 * (static_cast<uint32_t>(part & 1) * xrn + xlr) + 64 * (part >> 1) * xrn;
-    auto load_x = [&](int g) {
-        const uint32_t o = (static_cast<uint32_t>(g >> 3) * 16 + 4 * (g & 3)) * 64 + 32 * ((g >> 2) & 1);
-        return XRegs{ld16(xbase + static_cast<size_t>(o) * xrn), ld16(xbase + static_cast<size_t>(o + 128) * xrn)};
-    };
-    const int l32 = lane & 31, lh = lane >> 5;
-    auto store_xs = [&](const XRegs& r, Q6XStage& d) {
-        uint16_t* p = &d[part >> 1][tok][16 * (part & 1)];
-        st16(p, r.a);
-        st16(p + 8, r.b);
-    };
-    // half-block j of every row: thread tid loads 16-byte pieces tid + 512 i (i < 4)
-    // of the 2048 (row c / 8, piece c % 8: ql 0-3, qh 4-5, scales 6, d 7)
-    uint4 wst[4];
-    auto wstage_load = [&](int j) {
-        const int half = j & 1;
+    const uint8_t* xbase = xp + tile_base(xt, K);
+    const uint32_t xo = 16u * static_cast<uint32_t>(lk * xrn + min(lr, xrn - 1));
+    const uint32_t xpart = 64u * xrn;   // bytes of one part of one depth
+    uint4 xr[2][2];
+    auto x_load = [&](uint4 (&d)[2], int g) {   // past the last depth: the last one again
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + 512 * i;
-            const int row = c >> 3, piece = c & 7;
-            const uint8_t* blk = w + (ub0 + static_cast<uint64_t>(min(rw0 + row, M - 1)) * nb + (j >> 1)) * 210;
-            const int off = piece < 4 ? 64 * half + 16 * piece
-                                      : piece < 6 ? 128 + 32 * half + 16 * (piece - 4) : 192 + 2 * (piece - 6);
-            wst[i] = ldg16_a2(blk + off);
-        }
+        for (int p = 0; p < 2; ++p) d[p] = ld16(xbase + (xo + static_cast<uint32_t>(2 * min(g, nst - 1) + p) * xpart));
     };
-    auto wstage_store = [&](int j) {
+    auto x_store = [&](const uint4 (&d)[2], int g) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int c = tid + 512 * i;
-            *reinterpret_cast<uint4*>(&wsl[j & 1][c >> 3][16 * (c & 7)]) = wst[i];
-        }
+        for (int p = 0; p < 2; ++p) xs[g & 1][wv][p][lane] = d[p];
     };
-    // this wave's share of stage g's B operands (step h = th, both row tiles): q - 32
-    auto decode = [&](int g) {
-        const int sg = g & 7, quarter = sg & 3;
-        const int nsh = 4 * (quarter >> 1), hsh = 2 * quarter;
-        const Q6WSlot& sl = wsl[(g >> 2) & 1];
+    // weights: 16-byte piece tid % 4 (the bytes of lanes lk = tid % 4) of rows tid / 4 and 128 + tid / 4; scales and d
+    // of row tid / 2
+    const uint8_t* wb = w + (ub0 + static_cast<uint64_t>(rw0) * nb) * 210;
+    const int rlast = M - 1 - rw0;
+    const uint32_t rbytes = 210u * static_cast<uint32_t>(nb);
+    const int pc = tid & 3, pr = tid >> 2;
+    const uint32_t wl[2] = {static_cast<uint32_t>(min(pr, rlast)) * rbytes + 64u * (pc >> 1) + 16u * (pc & 1),
+                            static_cast<uint32_t>(min(pr + 128, rlast)) * rbytes + 64u * (pc >> 1) + 16u * (pc & 1)};
+    const uint32_t wh = 128u - 32u * (pc >> 1);   // from there to the qh piece
+    const uint32_t so = static_cast<uint32_t>(min(tid >> 1, rlast)) * rbytes + 192u + 2u * (tid & 1);
+    auto block_at = [&](int b) { return 210u * static_cast<uint32_t>(min(b, nb - 1)); };   // the last block again
+    auto ql_load = [&](uint4 (&d)[2], int b, int odd) {
+        const uint32_t o = block_at(b) + 32u * odd;
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-            const int row = 64 * rg + 32 * rt + l32;
-            const uint2 ql = *reinterpret_cast<const uint2*>(&sl[row][32 * (quarter & 1) + 16 * th + 8 * lh]);
-            const uint2 qh = *reinterpret_cast<const uint2*>(&sl[row][64 + 16 * th + 8 * lh]);
-            const uint32_t q0 = ((ql.x >> nsh) & 0x0f0f0f0fu) | (((qh.x >> hsh) & 0x03030303u) << 4);
-            const uint32_t q1 = ((ql.y >> nsh) & 0x0f0f0f0fu) | (((qh.y >> hsh) & 0x03030303u) << 4);
-            uint32_t e[4];
-            q6_operand(q0, e[0], e[1]);
-            q6_operand(q1, e[2], e[3]);
-            f16x8_t r;
-            __builtin_memcpy(&r, e, 16);
-            bs[g & 1][rg][th][rt][lane] = r;
-        }
+        for (int i = 0; i < 2; ++i) d[i] = ldg16_a2(wb + (wl[i] + o));
     };
-    auto barrier = []() {   // LDS stores complete, then the workgroup meets
+    auto qh_load = [&](uint4 (&d)[2], int b) {
+        const uint32_t o = block_at(b);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) d[i] = ldg16_a2(wb + (wl[i] + (o + wh)));
+    };
+    auto sc_load = [&](int b) { return ldg16_a2(wb + (so + block_at(b))); };   // the scales, or d in the last two bytes
+    auto q_store = [&](const uint4& v, Q6QSlot& d, int i) {
+        const int t = (pr >> 4) + 8 * i, l = 16 * pc + (pr & 15);
+        d[0][t][l] = uint2{v.x, v.y};
+        d[1][t][l] = uint2{v.z, v.w};
+    };
+    auto sc_store = [&](const uint4& v, int b) {
+        if (tid & 1)
+            dl[b & 1][tid >> 1] = static_cast<uint16_t>(v.w >> 16);
+        else
+            *reinterpret_cast<uint4*>(&scl[b & 1][tid >> 1][0]) = v;
+    };
+    auto barrier = []() {   // this wave's LDS work is done, then the workgroup meets (loads stay in flight)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    uint32_t k64 = 0x64006400u;   // kept in a register: v_and_or_b32 takes one constant
+    asm volatile("" : "+v"(k64));
+    uint32_t kf = 0x000f000fu, k30 = 0x00300030u;
+    asm volatile("" : "+s"(kf), "+s"(k30));
 
-    f32x16_t acc[2][2];
+    // B operands: row tile rt's come from raw[rt & 1] into B[rt & 1]
+    struct Raw {
+        uint2 l, h;
+        uint32_t s;
+    } raw[2];
+    f16x2_t sc[4];   // of the current u
+    f16x8_t B[2][2], A[4][2];
+    auto raw_read = [&](auto dI, int rt, int b) {   // depth D of block b
+        constexpr int D = decltype(dI)::value, U = D >> 1, J = D & 1;
+        Raw& r = raw[rt & 1];
+        r.l = ql[U & 1][J][4 * rg + rt][lane];
+        r.h = qh[b & 1][J][4 * rg + rt][lane];
+        if constexpr (J == 0) r.s = scl[b & 1][64 * rg + 16 * rt + lr][8 * (lk >> 1) + 2 * U + (lk & 1)];
+    };
+    auto b_make = [&](auto dI, int rt) {
+        constexpr int D = decltype(dI)::value;
+        const Raw& r = raw[rt & 1];
+        if constexpr ((D & 1) == 0) sc[rt] = WScale<kQ6_K>::from(r.s);
+        const uint32_t wd[2] = {r.l.x, r.l.y}, hd[2] = {r.h.x, r.h.y};
+        decode_q6<(D >> 1)>(wd, hd, sc[rt], k64, kf, k30, B[rt & 1]);
+    };
+    f32x4_t acc[4][4], C[4][4];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+    for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[tt][rt][i] = 0.f;
+        for (int rt = 0; rt < 4; ++rt) acc[tt][rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    wstage_load(0);
-    wstage_store(0);
-    if (nhb > 1) {   // K >= 256: nhb >= 2
-        wstage_load(1);
-        wstage_store(1);
-    }
-    store_xs(load_x(0), xs[0]);
+    // blocks 0 (ql of odd u kept for the loop) and x of depths 0 .. 3 (nst >= 8)
+    uint4 st[2];   // the weights on their way
+    auto ql_put = [&](int odd) {
+        q_store(st[0], ql[odd], 0);
+        q_store(st[1], ql[odd], 1);
+    };
+    auto qh_put = [&](int b) {
+        q_store(st[0], qh[b & 1], 0);
+        q_store(st[1], qh[b & 1], 1);
+    };
+    x_load(xr[0], 0);
+    x_load(xr[1], 1);
+    ql_load(st, 0, 0);
+    ql_put(0);
+    qh_load(st, 0);
+    qh_put(0);
+    sc_store(sc_load(0), 0);
+    ql_load(st, 0, 1);
+    x_store(xr[0], 0);
+    x_load(xr[0], 2);
+    x_store(xr[1], 1);
+    x_load(xr[1], 3);
     barrier();
-    decode(0);
-    barrier();
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) A[tt][p] = *reinterpret_cast<const f16x8_t*>(&xs[0][4 * th + tt][p][lane]);
+    raw_read(IC<0>{}, 0, 0);
+    raw_read(IC<0>{}, 1, 0);
+    b_make(IC<0>{}, 0);
 
-    for (int g = 0; g < nst; ++g) {
-        const int sg = g & 7, cur = g & 1;
-        const int gn = g + 1;
-        const bool more = gn < nst;
-        // d * sc of this stage's two groups for the lane's two rows
-        float Ag[2][2];
-        {
-            const Q6WSlot& sl = wsl[(g >> 2) & 1];
+    for (int b = 0; b < nb; ++b) {
+        float dsc[4];
+        auto epilogue = [&](int rt) {   // the block's sums of row tile rt are complete: acc += d C
+            const float d = opaque(dsc[rt]);
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                const int row = 64 * rg + 32 * rt + l32;
-                const uint32_t sp = *reinterpret_cast<const uint16_t*>(&sl[row][96 + 2 * sg]);   // scales 2 sg, 2 sg + 1
-                const float d = half_bits(*reinterpret_cast<const uint16_t*>(&sl[row][126]));
+            for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    Ag[h][rt] = d * static_cast<float>(static_cast<int>(__builtin_amdgcn_sbfe(sp, 8 * h, 8)));
+                for (int r = 0; r < 4; ++r) acc[tt][rt][r] = __builtin_fmaf(d, C[tt][rt][r], acc[tt][rt][r]);
+        };
+        static_for<8>([&](auto sI) {
+            constexpr int D = decltype(sI)::value;
+            const int g = 8 * b + D;
+            // The LDS slots in use (the barrier of depth D: MD): ql of even u are read M7 .. M1 and M3 .. M5, of odd u
+            // M1 .. M3 and M5 .. M7, a block's qh M7 .. M7, x of depth g M(g - 1) .. Mg; scales with qh, d in depth 7.
+            if constexpr (D == 0) {
+                ql_put(1);
+                st[0] = sc_load(b + 1);
             }
-        }
-        XRegs xn;
-        if (more) xn = load_x(gn);
-        // half-block k + 1 (loaded at half-block k - 1's first stage) goes into k - 1's
-        // slot at half-block k's first stage (k - 1's decodes and scale reads ended with
-        // the previous barrier); then half-block k + 2 is loaded
-        const int jh = g >> 2;
-        if ((g & 3) == 0) {
-            if (jh >= 1 && jh + 1 < nhb) wstage_store(jh + 1);
-            if (jh + 2 < nhb) wstage_load(jh + 2);
-        }
-        f16x8_t B[2][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt) B[h][rt] = bs[cur][rg][h][rt][lane];
-        if (more) decode(gn);
-        const Q6XStage& xc = xs[cur];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                f16x8_t A[2];
-#pragma unroll
-                for (int p = 0; p < 2; ++p)
-                    A[p] = *reinterpret_cast<const f16x8_t*>(&xc[p][64 * th + 32 * tt + l32][16 * h + 8 * lh]);
-#pragma unroll
-                for (int rt = 0; rt < 2; ++rt) {
-                    f32x16_t Cq;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) Cq[i] = 0.f;
-                    Cq = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], B[h][rt], Cq, 0, 0, 0);
-                    Cq = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], B[h][rt], Cq, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[tt][rt][i] = __builtin_fmaf(Ag[h][rt], Cq[i], acc[tt][rt][i]);
+            if constexpr (D == 2) {
+                sc_store(st[0], b + 1);
+                qh_load(st, b + 1);
+            }
+            if constexpr (D == 4) {
+                qh_put(b + 1);
+                ql_load(st, b + 1, 0);
+            }
+            if constexpr (D == 6) {
+                ql_put(0);
+                ql_load(st, b + 1, 1);
+            }
+            static_for<4>([&](auto rI) {
+                constexpr int rt = decltype(rI)::value;
+                if constexpr (rt == 2) {
+                    barrier();
+                    x_store(xr[D & 1], g + 2);
+                    x_load(xr[D & 1], g + 4);
                 }
-            }
-        if (more) store_xs(xn, xs[cur ^ 1]);
-        barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (rt < 2)
+                    raw_read(IC<D>{}, rt + 2, b);
+                else
+                    raw_read(IC<(D + 1) & 7>{}, rt - 2, b + (D == 7));
+                if constexpr (D == 7) dsc[rt] = half_bits(dl[b & 1][64 * rg + 16 * rt + lr]);
+                if constexpr (rt < 3)
+                    b_make(IC<D>{}, rt + 1);
+                else
+                    b_make(IC<(D + 1) & 7>{}, 0);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt)   // a block's first depth starts its sums from zero
+                    C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        A[tt][0], B[rt & 1][0], D == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : C[tt][rt], 0, 0, 0);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[tt][1], B[rt & 1][0], C[tt][rt], 0, 0, 0);
+                    if constexpr (rt == 3) A[tt][1] = *reinterpret_cast<const f16x8_t*>(&xs[(D + 1) & 1][4 * th + tt][1][lane]);
+                }
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    C[tt][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[tt][0], B[rt & 1][1], C[tt][rt], 0, 0, 0);
+                    if constexpr (rt == 3) A[tt][0] = *reinterpret_cast<const f16x8_t*>(&xs[(D + 1) & 1][4 * th + tt][0][lane]);
+                }
+                if constexpr (D == 7 && rt > 0) epilogue(rt - 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 + ((rt < 2 ? D : D + 1) % 2 == 0) + (D == 7), 0);
+#pragma unroll
+                for (int i = 0; i < 12; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, D == 7 ? 4 : 3, 0);
+                    if (rt == 3 && i >= 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (D == 7) epilogue(3);
+        });
     }
-    // lane L holds C[8 (i/4) + 4 (L/32) + i%4][L % 32] of tile (tt, rt) in register i
+    // lane L holds C[4 (L/16) + r][L % 16] of tile (tt, rt): token 16 tt + 4 lk + r, row 16 rt + lr
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+    for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int t = tw + 32 * tt + 8 * (i >> 2) + 4 * lh + (i & 3);
+        for (int r = 0; r < 4; ++r) {
+            const int t = tw + 16 * tt + 4 * lk + r;
             if (t >= T) continue;
             const int et = ex[t];
             if (et == kRowNonFinite) {
-                for (int rt = 0; rt < 2; ++rt) {
-                    const int row = r0 + 32 * rt + l32;
+                for (int rt = 0; rt < 4; ++rt) {
+                    const int row = r0 + 16 * rt + lr;
                     if (row < M)
                         y[static_cast<size_t>(t) * M + row] = row_dot_per_element(
                             w, kQ6_K, (ub0 + static_cast<uint64_t>(row) * nb) * 256, x + static_cast<size_t>(t) * K, K);
@@ -1375,9 +1410,9 @@ __global__ __launch_bounds__(kQ6Block, 1) void gemm_q6k_wide(const GemmJobs jobs
                 continue;
             }
 #pragma unroll
-            for (int rt = 0; rt < 2; ++rt) {
-                const int row = r0 + 32 * rt + l32;
-                if (row < M) y[static_cast<size_t>(t) * M + row] = ldexpf(acc[tt][rt][i], -et);
+            for (int rt = 0; rt < 4; ++rt) {
+                const int row = r0 + 16 * rt + lr;
+                if (row < M) y[static_cast<size_t>(t) * M + row] = ldexpf(acc[tt][rt][r], -et);
             }
         }
 }
@@ -1436,26 +1471,35 @@ int prepare_x(bool prep, const float* x, int rows, int K, void* workspace, size_
 
 // How a matrix of a call is computed. A matrix alone and among others takes the same path and adds in the same
 // order, so the rule looks at the token count, K and the matrix itself only; which tile shape a path then uses
-// (sums are the same bits in all of them) depends on the whole launch.
-enum class Path { gemv, few, sliced4, sliced2, wide };
+// (the sums are the same bits in all of its shapes) depends on the whole launch.
+enum class Path { gemv, few, sliced4, sliced2, whole };
 
 // Measured at K = 2048 (M = 12352 in four matrices) and K = 4096 (M = 2048), Q4_K, us including the prep pass:
 //   few against one GEMV per token: 12 / 12 at every count up to 16; GEMV 6 / 3.6 per token, so it starts at 3
 //     tokens (4 where K takes two rounds). Against sliced4 at 17..32 tokens 22 / 12 and 18 / 26, at 128 tokens
-//     74 / 19 and 44 / 26, at 300 tokens sliced2 42 at K = 4096: few up to 16 tokens, up to 160 from K = 4096.
-//   sliced4 against sliced2, 77 tokens: 31 and 36; 200 tokens: 58 and 54.
-//   sliced2 against wide: 768 tokens 130 / 58 and 128 / 109; 1100 tokens 185 / 85 and 135 / 109; 2100 tokens
-//     300 / 160 and 249 / 113. A matrix of up to 64 rows would leave most of a wide tile idle for a whole round.
-// Q6_K times are about 1.5x these on every path but wide (1.75x); the same lines hold within 10%.
+//     74 / 19 and 44 / 26, against sliced2 at 300 tokens 50 and 42 at K = 4096: few up to 16 tokens, up to 160 from
+//     K = 4096.
+//   sliced4 against whole at K = 2048: 77 tokens 31 and 48, 128 tokens 44 and 49, 200 tokens 58 and 53.
+//   sliced2 against whole at K = 4096: 777 tokens 58 and 82, 1500 tokens 86 and 109, 2100 tokens 160 and 113. With
+//     many rows the chip is full without the slices.
+//   A matrix of up to 64 rows would leave most of a 256-row tile idle, a tile column more in every token block of the
+//     others' launch: up to 1024 tokens that is a fiftieth of it, above a round at worst (4096 tokens: 61 us against 20
+//     by sliced2 on its own).
+// Q6_K times are about 1.5x these; the same lines hold within 10%.
 Path gemm_path(int rows, int K, int M) {
     const int nb = K / 256;
     if (rows < (nb > 8 ? 4 : 3)) return Path::gemv;
     if (rows <= (nb >= 16 ? 160 : nb % 4 ? 128 : 16)) return Path::few;
     if (rows <= 128) return Path::sliced4;
-    const int most = nb >= 16 && M < 4096 ? 2048 : 768;
-    if (nb % 2 == 0 && (rows <= most || M <= 64)) return Path::sliced2;
-    return Path::wide;
+    if (M <= 64 && rows > 1024 && nb % 2 == 0) return Path::sliced2;
+    if (nb >= 16 && nb % 2 == 0 && M < 4096 && rows <= 2048) return Path::sliced2;
+    return Path::whole;
 }
+
+constexpr int kWideRows = 256, kWideTokens = 128;   // tile of the wide kernels
+static_assert(kQ4R == kWideRows && kQ4T == kWideTokens && kQ6R == kWideRows && kQ6T == kWideTokens, "wide tiles");
+
+unsigned wide_grid(GemmJobs& jobs, int rows) { return columns(jobs, kWideRows) * blocks_for(rows, kWideTokens); }
 
 template <int TYPE, int WT, int WR, int KW, int SL>
 struct Shape {
@@ -1474,10 +1518,13 @@ struct Shape {
 template <int TYPE>
 void launch_gemm(Path path, GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
     if (path == Path::few) {
-        const unsigned tb = blocks_for(rows, kTile);
-        if (columns(jobs, 16) * tb <= 256)
+        // rounds of 256 workgroups times a round's measured time, 16, 32 and 64 rows a workgroup
+        const int64_t tb = blocks_for(rows, kTile);
+        const float c1 = 8.5f * blocks_for(columns(jobs, 16) * tb, 256), c2 = 9.5f * blocks_for(columns(jobs, 32) * tb, 256),
+                    c4 = 13.f * blocks_for(columns(jobs, 64) * tb, 256);
+        if (c1 <= c2 && c1 <= c4)
             gemm_few<TYPE, 1><<<columns(jobs, 16) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
-        else if (columns(jobs, 32) * tb <= 256)
+        else if (c2 <= c4)
             gemm_few<TYPE, 2><<<columns(jobs, 32) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
         else
             gemm_few<TYPE, 4><<<columns(jobs, 64) * tb, 512, 0, s>>>(jobs, p.x, rows, K);
@@ -1496,21 +1543,24 @@ void launch_gemm(Path path, GemmJobs& jobs, const Prepared& p, int rows, int K, 
         using S1 = Shape<TYPE, 2, 2, 2, 2>;
         using S2 = Shape<TYPE, 3, 2, 2, 2>;
         using S3 = Shape<TYPE, 4, 2, 2, 2>;
-        using S4 = Shape<TYPE, 4, 2, 1, 2>;
-        const float c1 = S1::cost(jobs, rows, 20.f), c2 = S2::cost(jobs, rows, 25.f), c3 = S3::cost(jobs, rows, 31.f),
-                    c4 = S4::cost(jobs, rows, 46.f);
-        if (c1 <= c2 && c1 <= c3 && c1 <= c4)
+        const float c1 = S1::cost(jobs, rows, 20.f), c2 = S2::cost(jobs, rows, 25.f), c3 = S3::cost(jobs, rows, 31.f);
+        if (c1 <= c2 && c1 <= c3)
             S1::launch(jobs, p, rows, K, s);
-        else if (c2 <= c3 && c2 <= c4)
+        else if (c2 <= c3)
             S2::launch(jobs, p, rows, K, s);
-        else if (c3 <= c4)
-            S3::launch(jobs, p, rows, K, s);
         else
-            S4::launch(jobs, p, rows, K, s);
-    } else if constexpr (TYPE == kQ4_K) {
-        gemm_q4k_wide<<<columns(jobs, kQ4R) * blocks_for(rows, kQ4T), kQ4Block, 0, s>>>(jobs, p.ex, p.sx, p.xp, p.x, rows, K);
+            S3::launch(jobs, p, rows, K, s);
     } else {
-        gemm_q6k_wide<<<columns(jobs, kQ6R) * blocks_for(rows, kQ6T), kQ6Block, 0, s>>>(jobs, p.ex, p.xp, p.x, rows, K);
+        using S1 = Shape<TYPE, 4, 2, 1, 1>;
+        // 64 x 256 tiles or 128 x 256, us a round
+        constexpr float small = TYPE == kQ4_K ? 46.f : 67.f, wide = TYPE == kQ4_K ? 61.f : 90.f;
+        const unsigned grid = wide_grid(jobs, rows);
+        if (S1::cost(jobs, rows, small) <= wide * static_cast<float>(blocks_for(grid, 256)))
+            S1::launch(jobs, p, rows, K, s);
+        else if constexpr (TYPE == kQ4_K)
+            gemm_q4k_wide<<<grid, kQ4Block, 0, s>>>(jobs, p.ex, p.sx, p.xp, p.x, rows, K);
+        else
+            gemm_q6k_wide<<<grid, kQ6Block, 0, s>>>(jobs, p.ex, p.xp, p.x, rows, K);
     }
 }
 
@@ -1614,7 +1664,7 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
     if (any)
         if (const int rc = prepare_x(prep, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
     for (const int type : {static_cast<int>(kQ4_K), static_cast<int>(kQ6_K)})
-        for (const Path to : {Path::few, Path::sliced4, Path::sliced2, Path::wide}) {
+        for (const Path to : {Path::few, Path::sliced4, Path::sliced2, Path::whole}) {
             GemmJobs jobs{};
             for (int j = 0; j < n; ++j) {
                 const qwen_gemv_desc& e = descs[j];

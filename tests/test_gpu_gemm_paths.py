@@ -36,7 +36,8 @@ def _weight(kind, rows, K, seed):
     (16, 4100, 2048), (17, 64, 2048), (33, 129, 1024), (47, 300, 2048), (49, 96, 512),
     (127, 200, 2048), (128, 33, 2048), (129, 257, 2048), (129, 100, 1280),          # four slices / two / none (odd)
     (160, 80, 4096), (161, 80, 4096), (191, 500, 4608), (700, 2048, 512),
-    (768, 130, 2048), (769, 130, 2048), (769, 64, 2048), (783, 65, 1280),           # wide; thin matrices stay sliced
+    (320, 130, 2048), (321, 130, 2048), (640, 64, 2048), (641, 300, 2048),          # whole K: both tile sizes
+    (960, 64, 2048), (961, 70, 2048), (1024, 64, 2048), (1025, 64, 2048), (1025, 65, 1280), (1100, 3850, 1280), (1183, 3600, 256), (2048, 20, 4096), (2049, 20, 4096),
 ])
 def test_matmul_rows_edges(oracle, kind, T, M, K):
     r = np.random.default_rng(T * 131 + M + K)
@@ -54,7 +55,7 @@ def test_matmul_rows_edges(oracle, kind, T, M, K):
     assert np.all(got[T] == 5.0)
 
 
-@pytest.mark.parametrize("T", [2, 9, 20, 100, 200, 800])
+@pytest.mark.parametrize("T", [2, 9, 20, 100, 200, 400, 800, 1100])
 def test_matmul_rows_multi_keeps_the_bits(T):
     """Tile shapes follow the launch's total, sums do not: each matrix of a call gives the bits of its own call
     (thin matrices and both types among them)."""
@@ -62,7 +63,7 @@ def test_matmul_rows_multi_keeps_the_bits(T):
     K = 2048
     x = _dev(r.standard_normal((T, K)).astype(F32))
     jobs = [(_dev(_weight(kind, M, K, 20 + i)), kind, M * K, M, 0, None)
-            for i, (kind, M) in enumerate([("Q4_K", 8192), ("Q4_K", 32), ("Q6_K", 512), ("Q4_K", 2048), ("Q6_K", 48)])]
+            for i, (kind, M) in enumerate([("Q4_K", 8192), ("Q4_K", 32), ("Q6_K", 512), ("Q4_K", 2048), ("Q6_K", 48), ("Q6_K", 4096)])]
     for (w, kind, ne, M, off, _), got in zip(jobs, ops.matmul_rows_multi(jobs, x, K)):
         assert_bits_equal(got.cpu().numpy(), ops.matmul_rows(w, kind, ne, x, M, K).cpu().numpy(), what=f"{kind} {M}")
 
