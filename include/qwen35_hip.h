@@ -158,6 +158,16 @@ int qwen_gdn_gate_values_rows(const float* beta_raw, const float* alpha_raw, con
                               const float* dt_bias, float* beta, float* decay, int rows, int heads,
                               void* stream);
 
+/* qwen_gdn_frontend_rows and qwen_gdn_gate_values_rows of the same rows: the
+ * bits of the two calls, in one launch where the front end takes 16-byte loads
+ * (kernel 4, aligned buffers, heads of 64, 128 or 256). beta and decay may not
+ * overlap the front end's buffers. Other arguments and statuses as theirs. */
+int qwen_gdn_frontend_gates_rows(const float* x, const float* weight, const float* hist_in,
+                                 float* hist_out, float* y, int rows, int channels, int kernel,
+                                 int k_heads, int key_dim, float eps, const float* beta_raw,
+                                 const float* alpha_raw, const float* a, const float* dt_bias,
+                                 float* beta, float* decay, int heads, void* stream);
+
 /* One delta-rule step per value head h (key head h % key_heads), state
  * [value_heads x key_dim x value_dim] updated in place:
  *   S *= decay[h]; delta = (v - k^T S) * beta[h]; S += k delta^T; out = q^T S.

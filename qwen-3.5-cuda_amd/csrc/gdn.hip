@@ -17,6 +17,7 @@
 // head, U head groups per wave with all loads issued before any math.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "capi_common.hpp"
 #include "device_common.hpp"
@@ -42,13 +43,43 @@ constexpr int kGateUnroll = 4;   // head groups in flight per wave (norm_gate)
 // through LDS, so only wave 0 reads rows outside its tile (the rows before T0,
 // or the history when T0 == 0). Lanes past the last channel address a clamped
 // channel and skip their stores, so loads never branch.
-template <int LPH, int R, int W>
+//
+// GATES: workgroups from first_block on evaluate the rows' delta-rule gates, n
+// values in all. A prompt's gate launch is latency alone (rows x 32 values, 2.7
+// us at 9 rows, 4.9 at 4096); beside the convolution it costs nothing that shows:
+// a GDN layer over 9 rows 64.6 -> 55.1 us (a call less for the host, too), 77
+// rows 82.7 -> 80.6, 777 rows (Q6_K) 341 -> 336, 4096 rows 867 -> 860.
+struct GateRows {
+    const float* b;
+    const float* alpha;
+    const float* a;
+    const float* dt;
+    float* beta;
+    float* decay;
+    int64_t n;
+    int heads;
+    unsigned first_block;
+};
+
+template <int LPH, int R, int W, bool GATES>
 __global__ __launch_bounds__(W * kWave) void gdn_frontend_k4(const float* __restrict__ x, const float* __restrict__ w,
                                                           const float* hist_in, float* hist_out, float* __restrict__ y,
                                                           int rows, int C, int q_ch, int qk_ch, float eps, float qscale,
-                                                          int n_ctiles) {
+                                                          int n_ctiles, GateRows gates) {
     static_assert(R >= 3, "a wave hands its last three rows to the next wave");
     __shared__ float4 halo[W][3][kWave];
+    if constexpr (GATES) {
+        if (blockIdx.x >= gates.first_block) {  // the whole workgroup: no barrier is skipped
+            const int64_t step = static_cast<int64_t>(gridDim.x - gates.first_block) * (W * kWave);
+            for (int64_t i = static_cast<int64_t>(blockIdx.x - gates.first_block) * (W * kWave) + threadIdx.x;
+                 i < gates.n; i += step) {
+                const int h = static_cast<int>(i % gates.heads);
+                gates.beta[i] = gate_beta(gates.b[i]);
+                gates.decay[i] = gate_decay(gates.a[h], gates.alpha[i], gates.dt[h]);
+            }
+            return;
+        }
+    }
     const int lane = threadIdx.x & 63;
     const int wv = wave_in_block();
     const int cbase = (blockIdx.x % n_ctiles) * (4 * kWave);
@@ -279,15 +310,10 @@ void launch_qk_l2(float* q, float* k, int64_t stride, int rows, int heads, int d
     }
 }
 
-}  // namespace
-}  // namespace qk
-
-using namespace qk;
-
-extern "C" {
-
-int qwen_gdn_frontend_rows(const float* x, const float* weight, const float* hist_in, float* hist_out, float* y,
-                           int rows, int channels, int kernel, int k_heads, int key_dim, float eps, void* stream) {
+// The front end, and with gates.n > 0 the rows' gates: workgroups of the same launch on the vector path, else a
+// launch of gate_values_rows after it.
+int launch_frontend(const float* x, const float* weight, const float* hist_in, float* hist_out, float* y, int rows,
+                    int channels, int kernel, int k_heads, int key_dim, float eps, GateRows gates, void* stream) {
     QK_REQUIRE(rows >= 0 && channels >= 0, "gdn_frontend: negative size (rows=%d, channels=%d)", rows, channels);
     // kernel - 1 <= kConvTile keeps every history read inside the first time
     // tile, whose thread alone writes hist_out (in-place safety).
@@ -312,22 +338,67 @@ int qwen_gdn_frontend_rows(const float* x, const float* weight, const float* his
         const int n_wtiles = (rows + W * R - 1) / (W * R);
         const unsigned grid = static_cast<unsigned>(n_ctiles) * n_wtiles;
         const float qscale = k_heads > 0 ? host_rsqrt(key_dim) : 1.0f;
+        auto launch = [&](auto l) {
+            constexpr int LPH = decltype(l)::value;
+            if (gates.n > 0) {
+                gates.first_block = grid;
+                const unsigned extra = std::min<unsigned>(blocks_for(gates.n, W * kWave), 4096u);
+                gdn_frontend_k4<LPH, R, W, true><<<grid + extra, W * kWave, 0, s>>>(
+                    x, weight, hist_in, hist_out, y, rows, channels, q_ch, qk_ch, eps, qscale, n_ctiles, gates);
+            } else {
+                gdn_frontend_k4<LPH, R, W, false><<<grid, W * kWave, 0, s>>>(
+                    x, weight, hist_in, hist_out, y, rows, channels, q_ch, qk_ch, eps, qscale, n_ctiles, gates);
+            }
+        };
         if (lph == 64)
-            gdn_frontend_k4<64, R, W><<<grid, W * kWave, 0, s>>>(x, weight, hist_in, hist_out, y, rows, channels, q_ch,
-                                                                qk_ch, eps, qscale, n_ctiles);
+            launch(std::integral_constant<int, 64>{});
         else if (lph == 32)
-            gdn_frontend_k4<32, R, W><<<grid, W * kWave, 0, s>>>(x, weight, hist_in, hist_out, y, rows, channels, q_ch,
-                                                                qk_ch, eps, qscale, n_ctiles);
+            launch(std::integral_constant<int, 32>{});
         else
-            gdn_frontend_k4<16, R, W><<<grid, W * kWave, 0, s>>>(x, weight, hist_in, hist_out, y, rows, channels, q_ch,
-                                                                qk_ch, eps, qscale, n_ctiles);
+            launch(std::integral_constant<int, 16>{});
     } else {
         const int64_t threads = static_cast<int64_t>(channels) * n_ttiles;
         gdn_conv_any<<<blocks_for(threads, kBlock), kBlock, 0, s>>>(x, weight, hist_in, hist_out, y, rows, channels,
                                                                     kernel, n_ttiles);
         if (k_heads > 0) launch_qk_l2(y, y + q_ch, channels, rows, k_heads, key_dim, eps, s);
+        if (gates.n > 0) {
+            const int status = check_launch("gdn_frontend");
+            if (status != QWEN_STATUS_OK) return status;
+            return qwen_gdn_gate_values_rows(gates.b, gates.alpha, gates.a, gates.dt, gates.beta, gates.decay, rows,
+                                             gates.heads, stream);
+        }
     }
     return check_launch("gdn_frontend");
+}
+
+}  // namespace
+}  // namespace qk
+
+using namespace qk;
+
+extern "C" {
+
+int qwen_gdn_frontend_rows(const float* x, const float* weight, const float* hist_in, float* hist_out, float* y,
+                           int rows, int channels, int kernel, int k_heads, int key_dim, float eps, void* stream) {
+    return launch_frontend(x, weight, hist_in, hist_out, y, rows, channels, kernel, k_heads, key_dim, eps, GateRows{},
+                           stream);
+}
+
+int qwen_gdn_frontend_gates_rows(const float* x, const float* weight, const float* hist_in, float* hist_out, float* y,
+                                 int rows, int channels, int kernel, int k_heads, int key_dim, float eps,
+                                 const float* beta_raw, const float* alpha_raw, const float* a, const float* dt_bias,
+                                 float* beta, float* decay, int heads, void* stream) {
+    QK_REQUIRE(heads >= 0, "gdn_gate_values: negative size (rows=%d, heads=%d)", rows, heads);
+    if (rows <= 0 || channels <= 0 || heads == 0) {
+        const int status = qwen_gdn_frontend_rows(x, weight, hist_in, hist_out, y, rows, channels, kernel, k_heads,
+                                                  key_dim, eps, stream);
+        if (status != QWEN_STATUS_OK) return status;
+        return qwen_gdn_gate_values_rows(beta_raw, alpha_raw, a, dt_bias, beta, decay, rows, heads, stream);
+    }
+    QK_REQUIRE(beta_raw && alpha_raw && a && dt_bias && beta && decay, "gdn_gate_values: null pointer");
+    const GateRows gates{beta_raw, alpha_raw, a, dt_bias, beta, decay, static_cast<int64_t>(rows) * heads, heads, 0};
+    return launch_frontend(x, weight, hist_in, hist_out, y, rows, channels, kernel, k_heads, key_dim, eps, gates,
+                           stream);
 }
 
 int qwen_gdn_conv_step(const float* input, const float* weight, float* history, float* output, int channels,

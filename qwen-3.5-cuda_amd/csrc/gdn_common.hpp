@@ -37,6 +37,15 @@ __device__ __forceinline__ void history4(const float4 a, const float4 b, const f
     h2 = make_float4(a.z, b.y, d.x, d.w);
 }
 
+// softplus with the reference's threshold; log1p(exp(x)) evaluated with the
+// accurate device expf / log1pf.
+__device__ __forceinline__ float softplus20(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
+
+// The gate pair of src/cuda/gdn.cu:93-97, shared by gates_kernel, the
+// recurrence's fused-gate form and the front end's, so that all give the same bits.
+__device__ __forceinline__ float gate_beta(float b) { return 1.0f / (1.0f + expf(-b)); }
+__device__ __forceinline__ float gate_decay(float a, float alpha, float dt) { return expf(a * softplus20(alpha + dt)); }
+
 }  // namespace qk
 
 #endif  // QWEN35_GDN_COMMON_HPP

@@ -38,15 +38,6 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / kWave;
 
-// softplus with the reference's threshold; log1p(exp(x)) evaluated with the
-// accurate device expf / log1pf.
-__device__ __forceinline__ float softplus20(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
-
-// The gate pair of src/cuda/gdn.cu:93-97, shared by gates_kernel and the
-// recurrence's fused-gate form so that both give the same bits.
-__device__ __forceinline__ float gate_beta(float b) { return 1.0f / (1.0f + expf(-b)); }
-__device__ __forceinline__ float gate_decay(float a, float alpha, float dt) { return expf(a * softplus20(alpha + dt)); }
-
 // Fused-gate form of the recurrence: with `a` set, the kernels' beta / decay
 // arguments hold beta_raw / alpha_raw and the gates are evaluated per token
 // where they are used (a, dt_bias per value head).

@@ -49,6 +49,7 @@ SIGNATURES: dict[str, list] = {
     "qwen_gdn_conv_step": [_P, _P, _P, _P, _I, _I, _P],
     "qwen_gdn_qk_normalize": [_P, _P, _I, _I, _F, _P],
     "qwen_gdn_frontend_rows": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P],
+    "qwen_gdn_frontend_gates_rows": [_P] * 5 + [_I, _I, _I, _I, _I, _F] + [_P] * 6 + [_I, _P],
     "qwen_gdn_norm_gate": [_P, _P, _P, _P, _I, _I, _F, _P],
     "qwen_gdn_norm_gate_rows": [_P, _P, _P, _P, _I, _I, _I, _F, _P],
     "qwen_gdn_norm_gate_matmul": [_P, _P, _P, _P, _I, _I, _F, _P, _I, _U64, _P, _I, _U64, _P],

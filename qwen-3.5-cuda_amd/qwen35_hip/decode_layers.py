@@ -115,11 +115,11 @@ class GdnLayerDecode:
                                       for n in names], xs, self.dm, workspace=ws)
         proj = dict(zip(names, outs))
         conv = torch.empty((T, self.cd), **f)
-        ops.gdn_frontend_rows(proj["qkv"], self.conv_w, self.history, self._history_next, y=conv, k_heads=self.kh,
-                              key_dim=self.dk, eps=self.eps)
-        self.history, self._history_next = self._history_next, self.history
         beta, decay = torch.empty((T, self.vh), **f), torch.empty((T, self.vh), **f)
-        ops.gdn_gate_values_rows(proj["beta"], proj["alpha"], self.a, self.dt, beta=beta, decay=decay)
+        ops.gdn_frontend_gates_rows(proj["qkv"], self.conv_w, self.history, proj["beta"], proj["alpha"], self.a, self.dt,
+                                    hist_out=self._history_next, y=conv, beta=beta, decay=decay, k_heads=self.kh,
+                                    key_dim=self.dk, eps=self.eps)
+        self.history, self._history_next = self._history_next, self.history
         core = torch.empty((T, self.vd), **f)
         ops.gdn_recurrent_chunked(self.state, conv, beta, decay, self.kh, self.vh, self.dk, self.dv, out=core)
         normed = torch.empty_like(core)

@@ -176,6 +176,31 @@ def gdn_frontend_rows(x, weight, hist_in, hist_out=None, y=None, k_heads=16, key
     return y, hist_out
 
 
+def gdn_frontend_gates_rows(x, weight, hist_in, beta_raw, alpha_raw, a, dt_bias, hist_out=None, y=None, beta=None,
+                            decay=None, k_heads=16, key_dim=128, eps=1e-6, stream=None):
+    """gdn_frontend_rows and gdn_gate_values_rows of the same rows in one call -> (y, hist_out, beta, decay)."""
+    _dev(x, weight, hist_in, beta_raw, alpha_raw, a, dt_bias, dtype=torch.float32)
+    rows, c = _rows(x)
+    if weight.dim() != 2 or weight.shape[0] != c:
+        raise ValueError("weight must be [channels, kernel]")
+    kernel, heads = weight.shape[1], a.numel()
+    _same((c, kernel - 1), hist_in)
+    _same((heads,), dt_bias)
+    _same((rows, heads), beta_raw, alpha_raw)
+    hist_out = torch.empty_like(hist_in) if hist_out is None else hist_out
+    y = torch.empty_like(x) if y is None else y
+    beta = torch.empty_like(beta_raw) if beta is None else beta
+    decay = torch.empty_like(beta_raw) if decay is None else decay
+    _dev(hist_out, y, beta, decay, dtype=torch.float32)
+    _same(hist_in.shape, hist_out)
+    _same(x.shape, y)
+    _same((rows, heads), beta, decay)
+    check(load().qwen_gdn_frontend_gates_rows(_p(x), _p(weight), _p(hist_in), _p(hist_out), _p(y), rows, c, kernel,
+                                              k_heads, key_dim, eps, _p(beta_raw), _p(alpha_raw), _p(a), _p(dt_bias),
+                                              _p(beta), _p(decay), heads, _stream(stream)))
+    return y, hist_out, beta, decay
+
+
 def gdn_conv_step(x, weight, history, y=None, stream=None):
     """One token: x [C], weight [C, K], history [C, K-1] (updated in place)."""
     _dev(x, weight, history, dtype=torch.float32)

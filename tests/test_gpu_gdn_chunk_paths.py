@@ -52,3 +52,24 @@ def test_up_to_28_rows_are_the_token_loop():
     two = ops.gdn_recurrent_rows(b, qkv, beta, decay, 16, 32, 128, 128)
     assert_bits_equal(one.cpu().numpy(), two.cpu().numpy(), what="out")
     assert_bits_equal(a.cpu().numpy(), b.cpu().numpy(), what="state")
+
+
+@pytest.mark.parametrize("rows,kh,dim,kernel,heads,skew", [(1, 16, 128, 4, 32, 0), (3, 2, 64, 4, 3, 0), (24, 16, 128, 4, 32, 0),
+                                                           (25, 1, 256, 4, 1, 0), (777, 16, 128, 4, 33, 0),
+                                                           (9, 4, 32, 4, 8, 0), (9, 2, 128, 3, 8, 0), (9, 2, 128, 4, 8, 1)])
+def test_frontend_gates_is_the_two_calls(rows, kh, dim, kernel, heads, skew):
+    """One launch (heads of 64, 128 or 256 and 16-byte aligned buffers) and the general path, bit for bit against the
+    separate calls; the history in place as well."""
+    g = torch.Generator(device="cuda").manual_seed(rows + heads)
+    n = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    c = 4 * kh * dim
+    x, w, hist = n(rows * c + skew)[skew:].view(rows, c), n(c, kernel), n(c, kernel - 1)
+    b, al, a, dt = 9 * n(rows, heads), 9 * n(rows, heads), -torch.exp(n(heads)), n(heads)
+    b.view(-1)[0], al.view(-1)[-1] = float("inf"), float("nan")
+    y, h = ops.gdn_frontend_rows(x, w, hist, k_heads=kh, key_dim=dim)
+    beta, decay = ops.gdn_gate_values_rows(b, al, a, dt)
+    inplace = hist.clone()
+    for got in (ops.gdn_frontend_gates_rows(x, w, hist, b, al, a, dt, k_heads=kh, key_dim=dim),
+                ops.gdn_frontend_gates_rows(x, w, inplace, b, al, a, dt, hist_out=inplace, k_heads=kh, key_dim=dim)):
+        for name, u, v in zip(("y", "history", "beta", "decay"), got, (y, h, beta, decay)):
+            assert torch.equal(u.view(torch.int32), v.view(torch.int32)), name
