@@ -48,7 +48,7 @@ constexpr int kGateUnroll = 4;   // head groups in flight per wave (norm_gate)
 // values in all. A prompt's gate launch is latency alone (rows x 32 values, 2.7
 // us at 9 rows, 4.9 at 4096); beside the convolution it costs nothing that shows:
 // a GDN layer over 9 rows 64.6 -> 55.1 us (a call less for the host, too), 77
-// rows 82.7 -> 80.6, 777 rows (Q6_K) 341 -> 336, 4096 rows 867 -> 860.
+// rows 82.7 -> 80.6, 777 rows (Q6_K) 341 -> 336.
 struct GateRows {
     const float* b;
     const float* alpha;

@@ -169,6 +169,10 @@ __device__ __forceinline__ float split8(const float4& a, const float4& b, int e,
 // lane's two 16-byte pieces go to the round's LDS image of the fragments (slot lr ^ (chunk % 16) of its 16, so
 // neither side conflicts) and the workgroup writes the image out in order.
 // NIT > 0: K == 512 NIT, the row is held in registers (read once); NIT == 0: any K % 256 == 0, read twice.
+// gridDim.y is 1 or the number of rounds: then each workgroup still takes its rows' maxima over all of K, but splits
+// and writes round blockIdx.y alone. A short prompt's rounds are a serial chain on a few CUs (5 workgroups at 77
+// tokens): prep and a 256-row product at 77 tokens 18.4 -> 16.5 us (K = 2048), at 300 46.1 -> 45.0, at 300 and K = 4096
+// 40.3 -> 37.3. The lines of the launch say where it stops paying.
 template <int NIT>
 __global__ __launch_bounds__(1024) void gemm_prep_x(const float* __restrict__ x, int* __restrict__ ex,
                                                     float* __restrict__ sx, uint8_t* __restrict__ xp, int T, int K) {
@@ -199,7 +203,7 @@ __global__ __launch_bounds__(1024) void gemm_prep_x(const float* __restrict__ x,
         }
     }
     const int e = prep_exponent(wave_max_abs(m));
-    if (live && lane == 0) ex[t] = e;
+    if (live && lane == 0 && blockIdx.y == 0) ex[t] = e;
     const int es = e == kRowNonFinite ? 0 : e;   // a marked row's parts are not used
     uint8_t* out = xp + tile_base(blockIdx.x, K);
     const int c16 = lane & 15;                                             // chunk % 16 = 4 u + 2 (lk % 2) + j
@@ -230,9 +234,11 @@ __global__ __launch_bounds__(1024) void gemm_prep_x(const float* __restrict__ x,
     };
     if constexpr (NIT > 0) {
 #pragma unroll
-        for (int it = 0; it < NIT; ++it) round(it, v + 2 * it);
+        for (int it = 0; it < NIT; ++it)
+            if (gridDim.y == 1 || it == static_cast<int>(blockIdx.y)) round(it, v + 2 * it);
     } else {
         for (int it = 0; it < nit; ++it) {
+            if (gridDim.y != 1 && it != static_cast<int>(blockIdx.y)) continue;
             load(it, v);
             round(it, v);
         }
@@ -1437,6 +1443,8 @@ unsigned columns(GemmJobs& jobs, int rows) {
     return static_cast<unsigned>(jobs.start[jobs.n]);
 }
 
+constexpr unsigned kPrepSpread = 256;
+
 struct Prepared {
     const int* ex;
     const float* sx;
@@ -1457,7 +1465,10 @@ int prepare_x(bool prep, const float* x, int rows, int K, void* workspace, size_
     int* ex = reinterpret_cast<int*>(ws);
     float* sx = reinterpret_cast<float*>(ws + ws_exp_bytes(rows));
     uint8_t* xp = ws + ws_exp_bytes(rows) + ws_sum_bytes(rows, K);
-    const unsigned grid = blocks_for(rows, kTile);
+    // A workgroup per round while each has a CU: at 196 and 256 workgroups 0.0 and 1.1 us less, at 376 and 512 (two on
+    // a CU, every row read once per round) 2.3 us more at K = 2048, at 392 6.1 more at K = 4096.
+    const unsigned tiles = blocks_for(rows, kTile), rounds = blocks_for(K, 512);
+    const dim3 grid(tiles, static_cast<uint64_t>(tiles) * rounds <= kPrepSpread ? rounds : 1);
     switch (K) {
         case 512: gemm_prep_x<1><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;
         case 1024: gemm_prep_x<2><<<grid, 1024, 0, s>>>(x, ex, sx, xp, rows, K); break;

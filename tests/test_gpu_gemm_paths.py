@@ -103,3 +103,14 @@ def test_nonfinite_rows_in_every_form(oracle, kind, T):
     for t in (0, 4, T - 1):
         ref = oracle.gemv(w, ops.GGML_TYPES[kind], x[t], M, K)
         assert rel_err(got[t], ref, group=M).max() <= 1e-5
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T,K", [(1024, 2048), (1360, 1280), (512, 4096)])
+def test_prep_spread_over_workgroups_keeps_the_bits(kind, T, K):
+    """The last token count whose prep takes a workgroup per 512 elements of K, against one tile more (all of K in
+    one workgroup): the first T tokens get the same bits."""
+    w = _dev(_weight(kind, 300, K, 9))
+    x = torch.randn((T + 16, K), generator=torch.Generator().manual_seed(T)).cuda()
+    assert_bits_equal(ops.matmul_rows(w, kind, 300 * K, x[:T], 300, K).cpu().numpy(),
+                      ops.matmul_rows(w, kind, 300 * K, x, 300, K)[:T].cpu().numpy())
