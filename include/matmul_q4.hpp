@@ -25,7 +25,7 @@ void matmul_dispatch(const QuantTensor& weight, const float* x, float* y, int M,
 
 // matmul_dispatch for each of `rows` tokens in one call: y[t*M + m] = sum_k
 // W[element_offset + m*K + k] * x[t*K + k] (matrix cores for Q4_K / Q6_K at
-// rows >= 16, fp32 accuracy), with a device workspace of
+// 3 rows or more, fp32 accuracy), with a device workspace of
 // matmul_rows_workspace_bytes(rows, K) bytes. Throws as matmul_dispatch.
 // gdn_norm_gate of x, z [heads x dim] into normed, then matmul_dispatch of weight on
 // normed (K = heads * dim): the same bits, one launch for Q4_K weights on the per-row
