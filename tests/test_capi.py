@@ -244,3 +244,19 @@ def test_attn_decode_norm_rope_host_validation(lib):
     assert "rope_dim" in msg(lib)
     assert lib.qwen_attn_decode_norm_rope(p, p, p, p, NULL, p, 16, 2, 256, 10, p, p, 64, 1e7, 1e-6, p, 16, ST) == INV
     assert "workspace" in msg(lib)
+
+
+def test_gdn_frontend_gates_host_validation(lib):
+    """Refuses what either of the two calls refuses; no rows is no work."""
+    INV, OK = _lib.STATUS_INVALID_ARGUMENT, _lib.STATUS_OK
+    f = lib.qwen_gdn_frontend_gates_rows
+    front, gates = [FAKE] * 5, [FAKE] * 6
+    assert f(*front, 4, 64, 1, 0, 0, 1e-6, *gates, 2, ST) == INV        # kernel size
+    assert f(*front, 4, 64, 4, 1, 64, 1e-6, *gates, 2, ST) == INV       # q and k exceed the channels
+    assert f(*front, -1, 64, 4, 0, 0, 1e-6, *gates, 2, ST) == INV
+    assert f(*front, 4, 64, 4, 0, 0, 1e-6, *gates, -2, ST) == INV
+    for i in range(6):
+        assert f(*front, 4, 64, 4, 0, 0, 1e-6, *[NULL if j == i else FAKE for j in range(6)], 2, ST) == INV
+    for i in range(5):
+        assert f(*[NULL if j == i else FAKE for j in range(5)], 4, 64, 4, 0, 0, 1e-6, *gates, 2, ST) == INV
+    assert f(*[NULL] * 5, 0, 64, 4, 0, 0, 1e-6, *[NULL] * 6, 2, ST) == OK
