@@ -52,6 +52,7 @@
 #include "capi_common.hpp"
 #include "device_common.hpp"
 #include "gdn_common.hpp"
+#include "launch_rules.hpp"
 
 namespace qk {
 namespace {
@@ -60,7 +61,6 @@ constexpr int kC = 64;                        // tokens per chunk
 constexpr int kDK = 128;                      // key dim of the chunked path
 constexpr int kNB = 16;                       // state columns per workgroup (kernel B)
 constexpr int kLoopRows = 28;       // up to this many rows the token loop runs (below)
-constexpr int kSpreadGroups = 256;  // prep workgroups at one per CU
 constexpr int kThreads = 256;                 // prep
 constexpr int kWalkThreads = 512;             // state walk: two waves per SIMD
 constexpr int64_t kMaxWalkStride = 0x7fffffff / (4 * 64);   // floats; 64 rows of 4-byte elements below 2^31 bytes
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
                                                            const float* __restrict__ beta,
                                                            const float* __restrict__ decay, float* __restrict__ ws,
                                                            unsigned char* __restrict__ kq, int rows, int key_heads,
-                                                           int value_heads, int64_t qkv_stride) {
+                                                           int value_heads, int hstep, int64_t qkv_stride) {
     // The chunk's K as fp16 pairs while the products run; after them the same
     // storage holds A (strictly lower) and T of the value head in hand.
     __shared__ __align__(16) float kat[2 * kC * kLdA];
@@ -173,11 +173,10 @@ __global__ __launch_bounds__(kThreads) void gdn_chunk_prep(const float* __restri
     __shared__ float sglast;                       // gamma_{C-1}
     float(*Ab)[kLdA] = reinterpret_cast<float(*)[kLdA]>(kat);
     float(*T)[kLdA] = reinterpret_cast<float(*)[kLdA]>(kat + kC * kLdA);
-    const int c = blockIdx.x, src = blockIdx.y;   // chunk, key head
-    // With gridDim.z > 1 a key head's value heads are dealt to that many workgroups, each with the products of its
-    // own; only the first writes K and Q out.
-    const int h0 = src + key_heads * static_cast<int>(blockIdx.z), hstep = key_heads * static_cast<int>(gridDim.z);
-    const bool writes_kq = blockIdx.z == 0;
+    // Chunk, first value head (prep_grid: below value_heads), their key head. Where a key head's value heads have
+    // workgroups of their own, each makes the products and the first writes K and Q out.
+    const int c = blockIdx.x, h0 = blockIdx.y, src = h0 % key_heads;
+    const bool writes_kq = h0 < key_heads;
     const int t0 = c * kC;
     const int lane = threadIdx.x & 63;
     const int wv = wave_in_block();
@@ -888,13 +887,9 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     const int nchunks = (rows + kC - 1) / kC;
     float* ws = static_cast<float*>(workspace);
     unsigned char* kq = static_cast<unsigned char*>(workspace) + static_cast<size_t>(nchunks) * value_heads * kWsFloats * sizeof(float);
-    // A value head's share is a third of a prep workgroup's serial chain: while one workgroup per (chunk, value head)
-    // has a CU to itself, a key head's value heads go to workgroups of their own (both launches, 64 tokens 20.0 ->
-    // 16.2 us, 128 24.1 -> 20.7, 400 38.9 -> 36.3; two to a CU gains nothing, 777 tokens 52.1 -> 52.9).
-    const int kh = std::min(key_heads, value_heads), group = (value_heads + kh - 1) / kh;
-    const bool spread = static_cast<int64_t>(nchunks) * kh * group <= kSpreadGroups;
-    gdn_chunk_prep<<<dim3(nchunks, kh, spread ? group : 1), kThreads, 0, s>>>(
-        q, k, beta, decay, ws, kq, rows, key_heads, value_heads, qkv_stride);
+    const PrepGrid g = prep_grid(nchunks, key_heads, value_heads);
+    gdn_chunk_prep<<<dim3(nchunks, g.heads), kThreads, 0, s>>>(q, k, beta, decay, ws, kq, rows, key_heads, value_heads,
+                                                              g.step, qkv_stride);
     // One row: its stride is not used to step between rows, but the walk's
     // buffer range is one stride long, so it must cover the row's q, k, v and out.
     const int64_t row_extent = std::max<int64_t>(static_cast<int64_t>(key_heads) * key_dim,

@@ -1,0 +1,26 @@
+// Launch shapes and the index arithmetic that kernels derive from them, where the two have to agree. Plain C++ (no
+// HIP), so that a test walks them on the host over the sizes the entry points accept.
+#pragma once
+
+#include <cstdint>
+
+namespace qk {
+
+// Grid of the chunked GDN recurrence's prep (csrc/gdn_chunk.hip): x = chunk; y = the workgroup's first value head h0,
+// of which it takes h0, h0 + step, ... < value_heads. Value head h reads key head h % key_heads, and step is a multiple
+// of key_heads or covers every head, so a workgroup's heads share one key head; the workgroups with y < key_heads write
+// that head's K and Q out. y < heads <= value_heads: no workgroup starts past the last value head, also where
+// value_heads is no multiple of key_heads.
+// A value head's share is a third of a workgroup's serial chain: while one workgroup per (chunk, value head) has a CU
+// to itself, every value head has its own (both launches, 64 tokens 20.0 -> 16.2 us, 128 24.1 -> 20.7, 400 38.9 -> 36.3;
+// two to a CU gains nothing, 777 tokens 52.1 -> 52.9).
+constexpr int kSpreadGroups = 256;
+struct PrepGrid {
+    int heads, step;
+};
+constexpr PrepGrid prep_grid(int chunks, int key_heads, int value_heads) {
+    if (static_cast<int64_t>(chunks) * value_heads <= kSpreadGroups) return {value_heads, value_heads};
+    return {key_heads < value_heads ? key_heads : value_heads, key_heads};
+}
+
+}  // namespace qk

@@ -1,5 +1,6 @@
 """The chunked recurrence at the edges of its routes: the token loop up to 28 rows, prep workgroups per value head
-while they have a CU each, one per key head above (and with one, two or three value heads per key head)."""
+while they have a CU each, one per key head above (and with one, two or three value heads per key head, or uneven
+numbers of them)."""
 
 from __future__ import annotations
 
@@ -13,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,kh,vh", [(1, 16, 32), (28, 16, 32), (29, 16, 32), (64, 4, 4), (65, 4, 12), (512, 16, 32),
-                                        (513, 16, 32), (100, 8, 4)])
+                                        (513, 16, 32), (100, 8, 4), (64, 2, 3), (130, 16, 24), (700, 16, 24), (65, 3, 8)])
 def test_chunked_routes(rows, kh, vh):
     """Output and state against the recurrence in float64, under the bar of the other recurrence tests: 1e-5 of the
     larger of the value and its condition scale (here each head's largest terms, |q||S| of the readout)."""
