@@ -498,12 +498,15 @@ int qwen_matmul_dispatch(const void* weight, int type, uint64_t num_elements, co
  * for t < rows, m < M (x fp32 [rows x K], y fp32 [rows x M], row-major) -- the
  * reference's per-token matmul_dispatch over a prompt as one call. Q4_K and
  * Q6_K with K % 256 == 0, element_offset % 256 == 0, x 16-byte aligned and 3
- * rows or more (4 from K = 2304) run on the matrix cores: each token row is
- * scaled by a power of two and split exactly into two fp16 parts, the quants
- * enter as exact fp16 integers, products are exact and sums fp32 -- an fp32 dot
- * product's accuracy, not the reference's bits. From 16 rows on those cases
- * need a 16-byte aligned workspace of qwen_matmul_rows_workspace_bytes(rows, K)
- * bytes (QWEN_STATUS_INVALID_ARGUMENT otherwise); fewer rows ignore it, and the
+ * rows or more (4 from K = 2304 or M = 49152) run on the matrix cores with an
+ * fp32 dot product's accuracy, not the reference's bits. Below 16 rows x, the
+ * dequantized weights and all sums are fp32. From 16 rows on each token row is
+ * scaled by a power of two and held as two fp16 parts (22 bits, fewer in an
+ * element below 2^-18 of its row's largest), the quants enter as exact fp16
+ * integers, products are exact (Q6_K: but for one below 2^-22 of the others)
+ * and sums fp32; those calls need a 16-byte aligned workspace of
+ * qwen_matmul_rows_workspace_bytes(rows, K) bytes
+ * (QWEN_STATUS_INVALID_ARGUMENT otherwise); fewer rows ignore it, and the
  * other cases run qwen_matmul_dispatch once per token. A row of x holding an
  * infinity gives non-finite outputs (the NaN / infinity pattern may differ
  * from the reference's). rows == 0 is a no-op. Statuses and messages as

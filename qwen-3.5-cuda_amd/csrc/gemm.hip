@@ -4,11 +4,12 @@
 // matmul_dispatch (src/cuda/matmul_q4.cu:140-167,185-207) called once per
 // token; batched, it is a contraction for the matrix cores.
 //
-// Exact fp16 operands. A prep kernel scales each token row by a power of two,
+// Below 16 tokens all operands are fp32 (gemm_f32). From there on x enters as two
+// fp16 parts: a prep kernel (gemm_few itself) scales each token row by a power of two,
 // v = x * 2^e with max |v| in [2^14, 2^15), and splits it into two fp16 parts
-// v = h + l (h = fp16(v), l = fp16(v - h)): |v - h - l| <= 2^-22 |v| (or
-// 2^-25 absolute for the smallest values), so the products below carry an
-// fp32 dot product's accuracy. The weights enter as exact small integers:
+// v = h + l (h = fp16(v), l = fp16(v - h)): |v - h - l| <= 2^-22 |v|, or 2^-25
+// absolute below 2^-18 of the row's largest, so the sums below carry an fp32
+// dot product's accuracy unless they come from such elements alone. The weights enter as exact small integers:
 //   Q4_K: B = q * sc (q 0..15, sc 0..63: at most 945, exact in fp16), so the
 //         MFMA accumulator sums a whole 256-element block across its eight
 //         scale groups, and per block
@@ -27,16 +28,17 @@
 // and -1024 sc leaves q * sc (Q4_K; a shift more for every second pair). The
 // pairs are bytes (0, 2) and (1, 3) of a word; x is stored in that order.
 //
-// Four kernels, by token count (gemm_path below has the lines and both sides'
-// times): gemm_few (up to 16 tokens, 160 from K = 4096) converts x itself and
-// splits K over its waves; gemm_kquant splits K in 4, 2 or no slices over waves
-// of a workgroup with the tile shape that fills the 256 CUs in the fewest
-// rounds; gemm_q4k_wide and gemm_q6k_wide (128 x 256 tiles) take long prompts.
+// Five kernels, by token count (gemm_path below has the lines and both sides'
+// times): gemm_f32 below 16 tokens; gemm_few (16 tokens, up to 128 where 4 does not
+// divide the blocks of a row, up to 160 from K = 4096) converts x itself and splits
+// K over its waves; gemm_kquant splits K in 4, 2 or no slices over waves of a
+// workgroup with the tile shape that fills the 256 CUs in the fewest rounds;
+// gemm_q4k_wide and gemm_q6k_wide (128 x 256 tiles) take long prompts.
 // Measured, us for the GDN layer's input projections (M = 8192, 4096, 32, 32 at
 // K = 2048, one call) and output projection (M = 2048 at K = 4096), Q4_K:
 //   tokens                            9        77        300       777      4096
 //   one form for all (before)     103 / 30  71 / 131  77 / 134  146 / 136  510 / 175
-//   these kernels                  13 / 12  31 /  21  56 /  42  132 /  62  438 / 152
+//   these kernels                  16 / 10  31 /  21  56 /  42  132 /  62  410 / 152
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
@@ -736,18 +738,179 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+// ------------------------------------------------------------------ fewer than 16 tokens
+// In fp32 throughout: x enters as it is, the weights as the reference's dequantized values (d sc q - dmin m, or
+// d sc (q - 32): exact products and at most one rounding, src/cuda/matmul_q4.cu:76-126), on v_mfma_f32_16x16x4_f32.
+// These counts stand in for one fp32 GEMV per token, which keeps x's 24 bits at any magnitude; two fp16 parts with one
+// exponent for a token's 2048 elements keep 22, and fewer from 2^-18 of the largest down. Error against 64 bits with
+// one channel of weight zero at 1, 1e5 and 1e7 times the others: GEMV 1.0e-7, 1.1e-7, 1.2e-7, the fp16 parts 1.0e-7,
+// 3.0e-7, 3.3e-5, this 1.0e-7, 1.1e-7, 1.2e-7 (Q4_K, K = 2048; Q6_K GEMV 1.6e-7, this 1.1e-7). Infinities and NaNs
+// need no path of their own.
+//
+// A workgroup owns 16 WR weight rows; K is split in 8 slices, slice s the blocks s, s + 8, ..., NW waves taking 8 / NW
+// slices each. x and weights go straight to the operand registers (no LDS, no barrier before the end); the next
+// block's x is requested piece by piece as the current one's is used up. Sums of 16 products from zero, added per
+// block, per slice and over the slices as a tree, so the bits do not depend on WR or NW.
+//
+// What bounds it: the fp32 MFMAs (64 x 32 cycles for 16 rows and a block, 5.2 us at M = 12352, K = 2048 over the whole
+// chip) and their operands' decode (18-24 VALU instructions per 8 weights), after 4 us of launch and first loads.
+// us at 3 / 9 / 15 tokens, Q4_K, against the fp16 parts (flat over those counts) and a GEMV per token (at 3):
+//   M = 32, K = 2048       5.4 / 6.0 / 7.0      6.6    6.8
+//   2048 x 4096            9.0 / 9.9 / 11.9     11.2   12.2
+//   8192 + 512 + 512       11.8 / 13.6 / 16.1   11.9   14.0
+//   12352 in four          14.5 / 15.8 / 17.0   12.1   17.3
+// gfx950 has no faster unit that holds 24 bits: three bf16 parts of x (exact) take 6 products of the 16 x 16 x 32 form
+// with Q4_K's weights in two parts, and the splitting, and come out equal.
+template <int TYPE>
+struct WFloat;   // a lane's weights of depth (U, J) as fp32, in element order
+template <>
+struct WFloat<kQ4_K> {
+    uint32_t sc, mn;   // the half's four scales and minima (scale_min_k4, src/cuda/matmul_q4.cu:18-26)
+    float d, dmin;
+    __device__ __forceinline__ void block(const WBlock<kQ4_K>& b, int lk) {
+        d = half_bits(b.hd.x & 0xffffu);
+        dmin = half_bits(b.hd.x >> 16);
+        sc = lk < 2 ? b.hd.y & 0x3f3f3f3fu : (b.hd.w & 0x0f0f0f0fu) | ((b.hd.y >> 2) & 0x30303030u);
+        mn = lk < 2 ? b.hd.z & 0x3f3f3f3fu : ((b.hd.w >> 4) & 0x0f0f0f0fu) | ((b.hd.z >> 2) & 0x30303030u);
+    }
+    template <int U, int J>
+    __device__ __forceinline__ void get(const WBlock<kQ4_K>& b, int, float (&w)[8]) const {
+        const float s = d * static_cast<float>(byte_of(sc, U)), m = dmin * static_cast<float>(byte_of(mn, U));   // exact
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint32_t q = (word_of(b.q[U >> 1], 2 * J + i) >> (4 * (U & 1))) & 0x0f0f0f0fu;
+            asm("" : "+v"(q));   // four v_cvt_f32_ubyte
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[4 * i + k] = __builtin_fmaf(static_cast<float>(byte_of(q, k)), s, -m);
+        }
+    }
+};
+template <>
+struct WFloat<kQ6_K> {
+    float d;
+    __device__ __forceinline__ void block(const WBlock<kQ6_K>& b, int) { d = half_bits(b.d); }
+    template <int U, int J>
+    __device__ __forceinline__ void get(const WBlock<kQ6_K>& b, int lk, float (&w)[8]) const {
+        const uint32_t sw = (U < 2 ? b.sc.x : b.sc.y) >> (16 * (U & 1) + 8 * (lk & 1));
+        const float s = d * static_cast<float>(static_cast<int8_t>(sw & 0xffu));   // exact
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            uint32_t q = ((word_of(b.q[U & 1], 2 * J + i) >> (4 * (U >> 1))) & 0x0f0f0f0fu) |
+                         (((word_of(b.qh, 2 * J + i) >> (2 * U)) & 0x03030303u) << 4);
+            asm("" : "+v"(q));
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[4 * i + k] = __builtin_fmaf(static_cast<float>(byte_of(q, k)), s, -32.0f * s);
+        }
+    }
+};
+
+constexpr int kF32Slices = 8;
+
+template <int TYPE, int WR, int NW>
+__global__ __launch_bounds__(NW * kWave) void gemm_f32(const GemmJobs jobs, const float* __restrict__ x, int T, int K) {
+    constexpr int BB = TYPE == kQ4_K ? 144 : 210, NS = kF32Slices;
+    static_assert(NS % NW == 0 && WR <= NW, "shape");
+    __shared__ f32x4_t part[NS * WR * kWave];
+    const GemmJob job = gemm_job(jobs, static_cast<int>(blockIdx.x));
+    float* __restrict__ y = job.y;
+    const int M = job.M;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+    const int wv = wave_in_block();
+    const int nb = K >> 8;
+    const int r0 = job.mb * 16 * WR;
+    const uint8_t* wbase = job.w + (job.ub0 + static_cast<uint64_t>(r0) * nb) * BB;
+    uint32_t wo[WR];   // the lane's row, from the workgroup's first (the matrix's last again past the end)
+#pragma unroll
+    for (int rt = 0; rt < WR; ++rt)
+        wo[rt] = static_cast<uint32_t>(min(16 * rt + lr, M - 1 - r0)) * static_cast<uint32_t>(nb) * BB;
+    WBlock<TYPE> wc[WR];
+    auto w_load = [&](int b) {
+        const uint8_t* p = wbase + static_cast<size_t>(b) * BB;
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) wc[rt].load(p, wo[rt], lk);
+    };
+    // token lr (the last one again past the end), the lane's 16 elements of depths 2 u and 2 u + 1
+    const float* xl = x + static_cast<size_t>(min(lr, T - 1)) * K + 128 * (lk >> 1) + 16 * (lk & 1);
+    float4 v[16];
+    auto x_load = [&](int b, int u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[4 * u + i] = ld4(xl + 256 * b + 32 * u + 4 * i);
+    };
+    if (wv < nb) {
+        w_load(wv);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x_load(wv, u);
+    }
+#pragma unroll 1
+    for (int sl = wv; sl < NS; sl += NW) {
+        f32x4_t tot[WR];
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) tot[rt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int b = sl; b < nb; b += NS) {
+            // the wave's next block: of this slice, or the first of its next one
+            const bool same = b + NS < nb;
+            const int next = same ? b + NS : sl + NW;
+            const bool more = same || (next < NS && next < nb);
+            f32x4_t C[2][WR][2], sum[WR];
+            WFloat<TYPE> wf[WR];
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) wf[rt].block(wc[rt], lk);
+            auto add = [&](int d) {
+#pragma unroll
+                for (int rt = 0; rt < WR; ++rt) {
+                    const f32x4_t c = C[d & 1][rt][0] + C[d & 1][rt][1];
+                    sum[rt] = d == 0 ? c : sum[rt] + c;
+                }
+            };
+            static_for<8>([&](auto dI) {
+                constexpr int D = decltype(dI)::value, U = D >> 1, J = D & 1;
+                const float4 a0 = v[2 * D], a1 = v[2 * D + 1];
+                const float a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+                for (int rt = 0; rt < WR; ++rt) {
+                    float w[8];
+                    wf[rt].template get<U, J>(wc[rt], lk, w);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        C[J][rt][i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            a[i], w[i], i < 2 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : C[J][rt][i & 1], 0, 0, 0);
+                }
+                if constexpr (J == 1) {
+                    if (more) x_load(next, U);
+                }
+                if constexpr (D > 0) add(D - 1);
+            });
+            add(7);
+#pragma unroll
+            for (int rt = 0; rt < WR; ++rt) tot[rt] += sum[rt];
+            if (more) w_load(next);
+        }
+#pragma unroll
+        for (int rt = 0; rt < WR; ++rt) part[(sl * WR + rt) * kWave + lane] = tot[rt];
+    }
+    __syncthreads();
+    if (wv >= WR) return;
+    auto at = [&](int sl) { return part[(sl * WR + wv) * kWave + lane]; };
+    const f32x4_t s = ((at(0) + at(1)) + (at(2) + at(3))) + ((at(4) + at(5)) + (at(6) + at(7)));
+    const int mrow = r0 + 16 * wv + lr;
+    if (mrow >= M) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (4 * lk + i < T) y[static_cast<size_t>(4 * lk + i) * M + mrow] = s[i];
+}
+
 // ------------------------------------------------------------------ a few tokens
-// Up to 16 tokens per workgroup and no prep pass (nor workspace): the workgroup converts its tokens' rows itself,
+// 16 tokens per workgroup and no prep pass: the workgroup converts its tokens' rows itself,
 // 2048 elements of K (a round: 8 blocks) at a time, into an LDS image of the fragments (slot lr ^ c of its 16,
 // c = 4 u + 2 (lk % 2) + j, so that neither the stores nor the loads conflict), with one exponent per token and
 // round. Wave w takes block w of every round for the workgroup's 16 WR rows; its first block's weights are
 // requested before the conversion. A round's sums are unscaled (exactly) and added to the wave's totals, and the
 // 8 waves' totals are added in wave order through LDS.
 //
-// These counts were one fp32 GEMV per token before, so the sums are kept to its accuracy (relative errors against
-// 64 bits at K = 2048 / 4096: GEMV Q4_K 1.8e-7, Q6_K 1.6e-7): the products of x's low parts, 2^-11 of the others,
-// have an accumulator of their own, and Q4_K's quants enter as q - 8, so that a block's sum is no larger than its
-// result; the 8 d sum_g sc_g S_g taken out joins the min terms in fp32.
+// The products of x's low parts, 2^-11 of the others, have an accumulator of their own, and Q4_K's quants enter as
+// q - 8, so that a block's sum is no larger than its result; the 8 d sum_g sc_g S_g taken out joins the min terms in
+// fp32.
 template <int TYPE, int WR>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_few(
     const GemmJobs jobs, const float* __restrict__ x, int T, int K) {
@@ -1483,13 +1646,14 @@ int prepare_x(bool prep, const float* x, int rows, int K, void* workspace, size_
 // How a matrix of a call is computed. A matrix alone and among others takes the same path and adds in the same
 // order, so the rule looks at the token count, K and the matrix itself only; which tile shape a path then uses
 // (the sums are the same bits in all of its shapes) depends on the whole launch.
-enum class Path { gemv, few, sliced4, sliced2, whole };
+enum class Path { gemv, f32, few, sliced4, sliced2, whole };
 
 // Measured at K = 2048 (M = 12352 in four matrices) and K = 4096 (M = 2048), Q4_K, us including the prep pass:
-//   few against one GEMV per token: 12 / 12 at every count up to 16; GEMV 6 / 3.6 per token, so it starts at 3
-//     tokens (4 where K takes two rounds). Against sliced4 at 17..32 tokens 22 / 12 and 18 / 26, at 128 tokens
-//     74 / 19 and 44 / 26, against sliced2 at 300 tokens 50 and 42 at K = 4096: few up to 16 tokens, up to 160 from
-//     K = 4096.
+//   f32 against one GEMV per token: above, GEMV 6 / 3.6 per token, so it starts at 3 tokens (4 from K = 2304: at
+//     2048 x 6144, 3 tokens, Q6_K 14.0 against 11.7). At 3 tokens a GEMV's better use of the memory tells in large
+//     matrices: M = 32768 28 against 32, 65536 51 against 45 (Q6_K 34 and 39, 66 and 57).
+//   few against sliced4 at 17..32 tokens 22 / 12 and 18 / 26, at 128 tokens 74 / 19 and 44 / 26, against sliced2 at
+//     300 tokens 50 and 42 at K = 4096: few at 16 tokens, up to 160 from K = 4096.
 //   sliced4 against whole at K = 2048: 77 tokens 31 and 48, 128 tokens 44 and 49, 200 tokens 58 and 53.
 //   sliced2 against whole at K = 4096: 777 tokens 58 and 82, 1500 tokens 86 and 109, 2100 tokens 160 and 113. With
 //     many rows the chip is full without the slices.
@@ -1499,7 +1663,8 @@ enum class Path { gemv, few, sliced4, sliced2, whole };
 // Q6_K times are about 1.5x these; the same lines hold within 10%.
 Path gemm_path(int rows, int K, int M) {
     const int nb = K / 256;
-    if (rows < (nb > 8 ? 4 : 3)) return Path::gemv;
+    if (rows < (nb > 8 ? 4 : 3) || (rows == 3 && M >= 49152)) return Path::gemv;
+    if (rows < kGemmMinRows) return Path::f32;
     if (rows <= (nb >= 16 ? 160 : nb % 4 ? 128 : 16)) return Path::few;
     if (rows <= 128) return Path::sliced4;
     if (M <= 64 && rows > 1024 && nb % 2 == 0) return Path::sliced2;
@@ -1526,9 +1691,30 @@ struct Shape {
     }
 };
 
+template <int TYPE, int WR, int NW>
+void launch_f32(GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
+    gemm_f32<TYPE, WR, NW><<<columns(jobs, 16 * WR), NW * kWave, 0, s>>>(jobs, p.x, rows, K);
+}
+
 template <int TYPE>
 void launch_gemm(Path path, GemmJobs& jobs, const Prepared& p, int rows, int K, hipStream_t s) {
-    if (path == Path::few) {
+    if (path == Path::f32) {
+        // A slice per wave while each workgroup of 16 rows has a CU (2048 x 4096, 9 tokens: 9.9 us, 10.5 with two
+        // slices). Above, two slices, and 16 rows (less work in a part-full round) or 32 (x, read by every workgroup,
+        // half as often: more with the tokens): us = 4 + workgroups per CU, rounded up, times a workgroup's time at
+        // K = 2048, within 10% from M = 8192 to 248320. Q6_K's 32 rows in 4 waves are 5-10% behind 8 waves.
+        constexpr bool q4 = TYPE == kQ4_K;
+        const unsigned n1 = columns(jobs, 16);
+        const float t = static_cast<float>(rows);
+        const float c1 = ((q4 ? 2.4f : 3.5f) + 0.1f * t) * static_cast<float>(blocks_for(n1, 256)),
+                    c2 = ((q4 ? 5.6f : 7.0f) + 0.08f * t) * static_cast<float>(blocks_for(columns(jobs, 32), 256));
+        if (n1 <= 256)
+            launch_f32<TYPE, 1, 8>(jobs, p, rows, K, s);
+        else if (c1 <= c2)
+            launch_f32<TYPE, 1, 4>(jobs, p, rows, K, s);
+        else
+            launch_f32<TYPE, 2, q4 ? 4 : 8>(jobs, p, rows, K, s);
+    } else if (path == Path::few) {
         // rounds of 256 workgroups times a round's measured time, 16, 32 and 64 rows a workgroup
         const int64_t tb = blocks_for(rows, kTile);
         const float c1 = 8.5f * blocks_for(columns(jobs, 16) * tb, 256), c2 = 9.5f * blocks_for(columns(jobs, 32) * tb, 256),
@@ -1619,7 +1805,7 @@ int qwen_matmul_rows(const void* weight, int type, uint64_t num_elements, const 
     if (path == Path::gemv) return per_token(weight, type, num_elements, x, y, rows, M, K, element_offset, stream);
     const hipStream_t s = as_stream(stream);
     Prepared p;
-    if (const int rc = prepare_x(path != Path::few, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
+    if (const int rc = prepare_x(path != Path::few && path != Path::f32, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
     GemmJobs jobs{};
     jobs.w[0] = static_cast<const uint8_t*>(weight);
     jobs.y[0] = y;
@@ -1656,7 +1842,7 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
         const qwen_gemv_desc& e = descs[j];
         path[j] = gemm && gemm_job_ok(e.type, e.element_offset, e.M, K) ? gemm_path(rows, K, e.M) : Path::gemv;
         any |= path[j] != Path::gemv;
-        prep |= path[j] != Path::gemv && path[j] != Path::few;
+        prep |= path[j] != Path::gemv && path[j] != Path::f32 && path[j] != Path::few;
         all_gemv &= path[j] == Path::gemv;
     }
     if (all_gemv) {   // every matrix in one call per token (each output the bits of its own GEMV)
@@ -1675,7 +1861,7 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
     if (any)
         if (const int rc = prepare_x(prep, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
     for (const int type : {static_cast<int>(kQ4_K), static_cast<int>(kQ6_K)})
-        for (const Path to : {Path::few, Path::sliced4, Path::sliced2, Path::whole}) {
+        for (const Path to : {Path::f32, Path::few, Path::sliced4, Path::sliced2, Path::whole}) {
             GemmJobs jobs{};
             for (int j = 0; j < n; ++j) {
                 const qwen_gemv_desc& e = descs[j];

@@ -1,6 +1,6 @@
 """matmul_rows over the token counts where its kernels and tile shapes change.
 
-The rule (csrc/gemm.hip, gemm_path) takes a GEMV per token below 3 (4) tokens, then three
+The rule (csrc/gemm.hip, gemm_path) takes a GEMV per token below 3 (4) tokens, then four
 matrix-core forms and the wide tiles; the sliced forms choose a tile shape by the launch's
 total. Each case sits at an edge of that rule, of a tile (16, 32, 48, 64, 128 tokens; 16 to 256
 rows) or of a K split (blocks per row that 2, 4 or 8 slices do not divide), against the oracle's
@@ -32,7 +32,9 @@ def _weight(kind, rows, K, seed):
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("T,M,K", [
-    (2, 48, 2048), (3, 17, 2048), (3, 300, 256), (4, 65, 4096), (15, 130, 2304),    # GEMV / few, partial rounds of K
+    (2, 48, 2048), (3, 17, 2048), (3, 300, 256), (4, 65, 4096), (15, 130, 2304),    # GEMV / fp32, partial rounds of K
+    (3, 4097, 2048), (9, 4113, 256), (15, 8200, 1280), (14, 16400, 512), (3, 2048, 4096), (5, 4100, 4352),   # fp32: 16 or 32 rows, 1 or 2 slices
+    (3, 49151, 256), (3, 49152, 256),                                               # fp32 / GEMV by the matrix
     (16, 4100, 2048), (17, 64, 2048), (33, 129, 1024), (47, 300, 2048), (49, 96, 512),
     (127, 200, 2048), (128, 33, 2048), (129, 257, 2048), (129, 100, 1280),          # four slices / two / none (odd)
     (160, 80, 4096), (161, 80, 4096), (191, 500, 4608), (700, 2048, 512),
@@ -55,7 +57,7 @@ def test_matmul_rows_edges(oracle, kind, T, M, K):
     assert np.all(got[T] == 5.0)
 
 
-@pytest.mark.parametrize("T", [2, 9, 20, 100, 200, 400, 800, 1100])
+@pytest.mark.parametrize("T", [2, 3, 9, 15, 20, 100, 200, 400, 800, 1100])
 def test_matmul_rows_multi_keeps_the_bits(T):
     """Tile shapes follow the launch's total, sums do not: each matrix of a call gives the bits of its own call
     (thin matrices and both types among them)."""
@@ -70,7 +72,7 @@ def test_matmul_rows_multi_keeps_the_bits(T):
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 def test_few_tokens_as_exact_as_the_gemv(kind):
-    """Below 16 tokens the matrix-core form replaces one fp32 GEMV per token: its 2-norm error against float64 is no
+    """Below 16 tokens the fp32 matrix-core form replaces one fp32 GEMV per token: its 2-norm error against float64 is no
     larger than the GEMV's (both sums have the same bound; the margin is the spread over inputs)."""
     r = np.random.default_rng(3)
     M, K, T = 1024, 2048, 12
@@ -86,10 +88,37 @@ def test_few_tokens_as_exact_as_the_gemv(kind):
 
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T,M,K", [(12, 1024, 2048), (3, 4112, 1024), (15, 512, 4608), (7, 8208, 256)])
+def test_few_tokens_keep_small_channels_beside_a_large_one(kind, T, M, K):
+    """A channel far above the others whose weights are zero leaves the others' 24 bits, as in the GEMV that these
+    counts stand in for, and so do rows of very small or large values: the same bar as above. (Each M is on another
+    tile shape: 16 rows with a slice or two of K per wave, 32 rows.)"""
+    r = np.random.default_rng(T)
+    blocks = _weight(kind, M, K, 9).reshape(M, K // 256, -1).copy()
+    if kind == "Q4_K":   # scale and minimum of elements 0..31 of each row
+        blocks[:, 0, 4] &= 0xC0
+        blocks[:, 0, 8] &= 0xC0
+    else:                # scale of elements 0..15
+        blocks[:, 0, 192] = 0
+    w = _dev(blocks.reshape(-1))
+    full = ops.dequant_gather_rows(w, kind, M * K, torch.arange(M, dtype=torch.int32, device="cuda"), K).double().cpu().numpy()
+    assert not full[:, 5].any()
+    for big, scale in [(1e5, 1), (1e7, 1), (1e12, 1), (1e30, 1), (1, 1e-30), (1, 1e30)]:
+        x = (r.standard_normal((T, K)) * scale).astype(F32)
+        x[:, 5] = big * scale
+        dx = _dev(x)
+        ref = x.astype(np.float64) @ full.T
+        few = ops.matmul_rows(w, kind, M * K, dx, M, K).cpu().numpy()
+        one = np.stack([ops.matmul_dispatch(w, kind, M * K, dx[t], M, K).cpu().numpy() for t in range(T)])
+        err = [np.linalg.norm(v - ref) / np.linalg.norm(ref) for v in (few, one)]
+        assert err[0] <= 1.1 * err[1], (big, scale, err)
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("T", [5, 40, 150, 800])
 def test_nonfinite_rows_in_every_form(oracle, kind, T):
     """A token row with an infinity gives the reference's pattern, a NaN row NaN, a zero row +0; others are
-    unaffected (two rounds of K for the few-token form)."""
+    unaffected (two rounds of K for the form with one exponent a round)."""
     M, K = 96, 4096 if T == 150 else 2048
     w = _weight(kind, M, K, 7)
     x = np.random.default_rng(T).standard_normal((T, K)).astype(F32)
