@@ -47,6 +47,7 @@
 #include "capi_common.hpp"
 #include "device_common.hpp"
 #include "ggml_common.hpp"
+#include "launch_rules.hpp"
 
 namespace qk {
 namespace {
@@ -467,7 +468,7 @@ struct GemmShape {
     static constexpr size_t ring = size_t{4} * FR * 1024, fold = KW > 1 ? size_t{8} * SPW * WT * WR * 1024 : 0;
     static constexpr size_t kept = SPW == 2 ? size_t{8} * WT * WR * 1024 : 0;
     static constexpr size_t lds = ring + kept > fold ? ring + kept : fold;
-    static_assert(FR % 8 == 0 && SPW >= 1 && SPW <= 2 && (KW > 1 || SPW == SL), "shape");
+    static_assert(rows <= kGemmTileRows && FR % 8 == 0 && SPW >= 1 && SPW <= 2 && (KW > 1 || SPW == SL), "shape");
 };
 
 // A value the compiler may not fold into its users (keeps v_fmac_f32 from
@@ -1587,16 +1588,15 @@ __global__ __launch_bounds__(kQ6Block) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // Token rows that the matrix-core paths take; x's fragments and a matrix's rows are addressed with 32-bit byte
-// offsets (Q6_K: within a workgroup's rows only).
+// offsets (gemm_offsets_fit).
 bool gemm_rows_ok(int rows, int K, const float* x) {
     return K % 256 == 0 && aligned16(x) && rows <= kGemmMaxRows &&
            4 * static_cast<uint64_t>(rows) * static_cast<uint64_t>(K) < (uint64_t{1} << 32);
 }
 
 bool gemm_job_ok(int type, uint64_t element_offset, int M, int K) {
-    if (element_offset % 256 != 0) return false;
-    if (type == kQ6_K) return true;
-    return type == kQ4_K && static_cast<uint64_t>(M) * static_cast<uint64_t>(K / 256) * 144 < (uint64_t{1} << 32);
+    return element_offset % 256 == 0 &&
+           (type == kQ4_K ? gemm_offsets_fit(true, 144, M, K) : type == kQ6_K && gemm_offsets_fit(false, 210, M, K));
 }
 
 // Workgroup columns of `rows` weight rows each, matrix after matrix.
@@ -1672,7 +1672,7 @@ Path gemm_path(int rows, int K, int M) {
     return Path::whole;
 }
 
-constexpr int kWideRows = 256, kWideTokens = 128;   // tile of the wide kernels
+constexpr int kWideRows = kGemmTileRows, kWideTokens = 128;   // tile of the wide kernels, the tallest
 static_assert(kQ4R == kWideRows && kQ4T == kWideTokens && kQ6R == kWideRows && kQ6T == kWideTokens, "wide tiles");
 
 unsigned wide_grid(GemmJobs& jobs, int rows) { return columns(jobs, kWideRows) * blocks_for(rows, kWideTokens); }

@@ -23,4 +23,13 @@ constexpr PrepGrid prep_grid(int chunks, int key_heads, int value_heads) {
     return {key_heads < value_heads ? key_heads : value_heads, key_heads};
 }
 
+// Whether a lane's byte offset into a K-quant matrix's rows (csrc/gemm.hip), row * blocks of a row * block bytes and the
+// block's own, stays below 2^32: Q4_K offsets may start at the matrix's first row (the 128 x 256 tiles), Q6_K ones at
+// the first of a workgroup's rows, of which no tile has more than kGemmTileRows.
+constexpr int kGemmTileRows = 256;
+constexpr bool gemm_offsets_fit(bool from_first_row, int block_bytes, int M, int K) {
+    const uint64_t rows = from_first_row || M < kGemmTileRows ? M : kGemmTileRows;
+    return rows * static_cast<uint64_t>(K / 256) * static_cast<uint64_t>(block_bytes) < (uint64_t{1} << 32);
+}
+
 }  // namespace qk

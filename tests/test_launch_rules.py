@@ -19,6 +19,9 @@ extern "C" void prep_grid(int chunks, int kh, int vh, int* out) {
     out[0] = g.heads;
     out[1] = g.step;
 }
+extern "C" int offsets_fit(int q4, int block_bytes, int M, int K) {
+    return qk::gemm_offsets_fit(q4 != 0, block_bytes, M, K);
+}
 """
 
 
@@ -49,3 +52,14 @@ def test_chunked_prep_heads_stay_in_range(rules, chunks):
                     written.append(y % kh)
             assert sorted(taken) == [(h, h % kh) for h in range(vh)], (kh, vh)
             assert written == list(range(min(kh, vh))), (kh, vh)
+
+
+@pytest.mark.parametrize("q4,block", [(1, 144), (0, 210)])
+def test_gemm_row_offsets_fit_32_bits(rules, q4, block):
+    """A matrix takes the matrix-core kernels only while the largest byte offset that a lane forms fits 32 bits: Q4_K's
+    from the matrix's first row, Q6_K's from a workgroup's (256 rows at most: K up to 20 million)."""
+    for K in (256, 2048, 4096, 1 << 20, 20_000_000 // 256 * 256, 20_500_000 // 256 * 256, 1 << 25, (1 << 28), (1 << 31) - 256):
+        for M in (1, 2, 15, 16, 100, 255, 256, 257, 4096, 248320, (1 << 31) - 1):
+            rows = M if q4 else min(M, 256)
+            last = ((rows - 1) * (K // 256) + K // 256) * block   # one past the last row's last byte
+            assert bool(rules.offsets_fit(q4, block, M, K)) == (last < 1 << 32), (M, K)
