@@ -878,6 +878,10 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     const size_t need = qwen_gdn_recurrent_chunked_workspace_bytes(rows, value_heads);
     QK_REQUIRE(workspace_bytes >= need, "gdn_recurrent_chunked: workspace of %zu bytes, %zu needed", workspace_bytes,
                need);
+    // One row needs no stride; the limit that longer calls have on theirs holds for its length.
+    QK_REQUIRE(rows > 1 || std::max(static_cast<int64_t>(key_heads) * key_dim,
+                                    static_cast<int64_t>(value_heads) * value_dim) <= kMaxWalkStride,
+               "gdn_recurrent_chunked: row too long for the chunked walk");
     // A few tokens: the token loop, 0.25 us a token from 8 us, against the two launches' 15.6 us for one chunk (9
     // tokens 10.1 us, 32 tokens 16.0 against 15.6, 48 tokens 20.0 against 16.0). Its error is the smaller one.
     if (rows <= kLoopRows)
@@ -890,15 +894,9 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     const PrepGrid g = prep_grid(nchunks, key_heads, value_heads);
     gdn_chunk_prep<<<dim3(nchunks, g.heads), kThreads, 0, s>>>(q, k, beta, decay, ws, kq, rows, key_heads, value_heads,
                                                               g.step, qkv_stride);
-    // One row: its stride is not used to step between rows, but the walk's
-    // buffer range is one stride long, so it must cover the row's q, k, v and out.
-    const int64_t row_extent = std::max<int64_t>(static_cast<int64_t>(key_heads) * key_dim,
-                                                 static_cast<int64_t>(value_heads) * value_dim);
-    const int64_t qs = rows == 1 ? std::max(qkv_stride, row_extent) : qkv_stride;
-    const int64_t os = rows == 1 ? std::max(out_stride, row_extent) : out_stride;
-    QK_REQUIRE(qs <= kMaxWalkStride && os <= kMaxWalkStride, "gdn_recurrent_chunked: row too long for the chunked walk");
     gdn_chunk_state<<<(value_dim / kNB) * value_heads, kWalkThreads, 0, s>>>(state, v, ws, kq, out, rows, key_heads,
-                                                                             value_heads, value_dim, qs, os);
+                                                                             value_heads, value_dim, qkv_stride,
+                                                                             out_stride);
     return check_launch("gdn_recurrent_chunked");
 }
 

@@ -187,6 +187,15 @@ def test_gdn_value_dim_limit_on_every_recurrent_path(lib):
     assert msg(lib) == "GDN value dimension exceeds kernel limit"
 
 
+def test_gdn_chunked_refuses_a_row_past_its_limit(lib):
+    """One row of more than 2^31 / 256 floats (value heads x 128, or key heads x 128) is refused before any launch, as
+    the strides of longer calls are limited, whichever kernel would run it."""
+    p, huge = ctypes.c_void_p(1 << 20), 1 << 62
+    for kh, vh in ((16, 65536), (65536, 32)):
+        st = lib.qwen_gdn_recurrent_chunked(p, p, p, p, p, p, p, 1, kh, vh, 128, 128, 8192, 4096, p, huge, ST)
+        assert st == _lib.STATUS_INVALID_ARGUMENT and "row too long" in msg(lib)
+
+
 def test_swiglu_routed_shared_validation(lib):
     INV, OK = _lib.STATUS_INVALID_ARGUMENT, _lib.STATUS_OK
     f = lib.qwen_swiglu_routed_shared_bf16
