@@ -402,10 +402,12 @@ int qwen_moe_route_swiglu(const float* logits, int32_t* idx, float* weights, int
  *   out = sum_j weights[j] * Wd_e hidden[j]  (e = idx[j], j < n_sel)
  *       + sigmoid(shared_logit[0]) * Wsd shared_hidden
  * hidden [n_sel x inter], shared_hidden [shared_dim], out [d_model] (written, not
- * accumulated). Down expert e at element offset e * expert_stride. One launch for
- * inter = 512, shared_dim a multiple of 2048 up to 4096, n_sel <= 8 and Q4_K / Q6_K
- * weights; other shapes run the same steps as separate launches through `workspace`,
- * which must hold qwen_moe_down_combine_workspace_bytes() bytes in every case.
+ * accumulated; it may take the place of hidden or shared_hidden). Down expert e at
+ * element offset e * expert_stride. One launch for inter = 512, shared_dim 512 or a
+ * multiple of 2048 up to 4096, n_sel <= 8, Q4_K / Q6_K weights and out apart from the
+ * hidden rows; other calls run the same steps as separate launches through
+ * `workspace`, which must hold qwen_moe_down_combine_workspace_bytes() bytes in every
+ * case.
  * Bit-equal to the separate calls (qwen_moe_expert_matmul, qwen_matmul_dispatch,
  * qwen_moe_weighted_sum_rows into a zeroed out, qwen_moe_shared_add_rows); an invalid
  * expert id makes out NaN. No counterpart entry point in the reference (it fuses the

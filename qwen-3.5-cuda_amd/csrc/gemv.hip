@@ -38,6 +38,7 @@
 #include "capi_common.hpp"
 #include "device_common.hpp"
 #include "ggml_common.hpp"
+#include "launch_rules.hpp"
 #include "moe_common.hpp"
 
 namespace qk {
@@ -2173,15 +2174,19 @@ int qwen_moe_down_combine(const void* w_down, int down_type, uint64_t down_eleme
     const auto* wsd = static_cast<const uint8_t*>(w_shared_down);
     const auto kq = [](int t) { return t == kQ4_K || t == kQ6_K; };
     const bool fused = kq(down_type) && kq(shared_type) && inter == kDcInter &&
-                       (shared_dim == 512 || (shared_dim % 2048 == 0 && shared_dim <= 4096)) && d_model % 4 == 0 && n_sel <= 8 && expert_stride % 2048 == 0 &&
-                       aligned16(wd) && aligned16(wsd) && aligned16(hidden) && aligned16(shared_hidden);
+                       (shared_dim == 512 || (shared_dim % 2048 == 0 && shared_dim <= 4096)) && d_model % 4 == 0 &&
+                       n_sel <= 8 && expert_stride % 2048 == 0 && aligned16(wd) && aligned16(wsd) &&
+                       aligned16(hidden) && aligned16(shared_hidden) &&
+                       !floats_overlap(out, d_model, hidden, static_cast<size_t>(n_sel) * inter) &&
+                       !floats_overlap(out, d_model, shared_hidden, shared_dim);
     if (fused) {
         const DownCombine a{wd, expert_stride / 256, n_experts, idx, weights, n_sel, hidden, wsd, shared_hidden,
                             shared_logit, out, d_model};
         launch_down_combine(a, down_type, shared_type, shared_dim / 2048, s);
         return check_launch("moe_down_combine");
     }
-    // Other shapes: the same steps as separate launches through the workspace.
+    // Other shapes, and out in the place of the hidden rows (other workgroups' inputs in the one launch): the same steps
+    // as separate launches through the workspace.
     auto* eo = static_cast<float*>(workspace);
     auto* so = reinterpret_cast<float*>(reinterpret_cast<char*>(eo) + align16(4 * n_sel * static_cast<size_t>(d_model)));
     int rc = launch_gemv(wd, down_type, down_elements, hidden, eo, d_model, inter, 0,

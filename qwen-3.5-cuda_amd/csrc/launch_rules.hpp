@@ -2,6 +2,7 @@
 // HIP), so that a test walks them on the host over the sizes the entry points accept.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 namespace qk {
@@ -30,6 +31,13 @@ constexpr int kGemmTileRows = 256;
 constexpr bool gemm_offsets_fit(bool from_first_row, int block_bytes, int M, int K) {
     const uint64_t rows = from_first_row || M < kGemmTileRows ? M : kGemmTileRows;
     return rows * static_cast<uint64_t>(K / 256) * static_cast<uint64_t>(block_bytes) < (uint64_t{1} << 32);
+}
+
+// Whether n floats at a and m floats at b share a byte. Calls that stand in for a sequence of launches, in which an
+// output may replace an input that the sequence has finished with, run as that sequence where the two overlap.
+inline bool floats_overlap(const float* a, size_t n, const float* b, size_t m) {
+    const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + 4 * m && y < x + 4 * n;
 }
 
 }  // namespace qk

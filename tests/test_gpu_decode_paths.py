@@ -64,6 +64,27 @@ def test_down_combine_small_shared_expert(td, ts, k, dm):
         assert_bits_equal(got.cpu().numpy(), separate(idx).cpu().numpy(), what=f"{td} {ts} k={k} {dm}")
 
 
+@pytest.mark.parametrize("S", [512, 2048])
+def test_down_combine_into_its_inputs(S):
+    """out in the place of the routed or the shared hidden rows: the bits of a call with an out of its own."""
+    E, inter, k, dm = 5, 512, 4, 512
+    r = np.random.default_rng(S)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    wd, wsd = dev(synth.q4k_table(E * dm, inter, seed_tensor=3)), dev(synth.q4k_table(dm, S, seed_tensor=11))
+    ids, wts = dev(np.array([3, 0, 4, 1], np.int32)), dev(r.random(k).astype(np.float32))
+    hid, shid = dev(r.standard_normal((k, inter)).astype(np.float32)), dev(r.standard_normal(S).astype(np.float32))
+    logit = dev(r.standard_normal(1).astype(np.float32))
+
+    def call(h, sh, out=None):
+        return ops.moe_down_combine(wd, "Q4_K", E * dm * inter, dm * inter, E, ids, wts, h, inter, wsd, "Q4_K", dm * S,
+                                    sh, logit, dm, out=out)
+
+    ref = call(hid, shid).cpu().numpy()
+    h, sh = hid.clone(), shid.clone()
+    assert_bits_equal(call(h, shid, out=h[1]).cpu().numpy(), ref, what="into hidden")
+    assert_bits_equal(call(hid, sh, out=sh[S - dm:]).cpu().numpy(), ref, what="into shared_hidden")
+
+
 @pytest.mark.parametrize("n", [512, 516, 1024, 2048, 2052, 4096])
 def test_residual_norm_of_few_rows_keeps_the_bits(n):
     """Up to 256 rows a row has a wave per chunk, above one wave: a row gives the same bits alone, among 256 and among

@@ -22,6 +22,9 @@ extern "C" void prep_grid(int chunks, int kh, int vh, int* out) {
 extern "C" int offsets_fit(int q4, int block_bytes, int M, int K) {
     return qk::gemm_offsets_fit(q4 != 0, block_bytes, M, K);
 }
+extern "C" int overlap(uintptr_t a, size_t n, uintptr_t b, size_t m) {
+    return qk::floats_overlap(reinterpret_cast<const float*>(a), n, reinterpret_cast<const float*>(b), m);
+}
 """
 
 
@@ -63,3 +66,12 @@ def test_gemm_row_offsets_fit_32_bits(rules, q4, block):
             rows = M if q4 else min(M, 256)
             last = ((rows - 1) * (K // 256) + K // 256) * block   # one past the last row's last byte
             assert bool(rules.offsets_fit(q4, block, M, K)) == (last < 1 << 32), (M, K)
+
+
+def test_floats_overlap(rules):
+    f = rules.overlap
+    f.argtypes = [ctypes.c_size_t] * 4
+    base, n, m = 1 << 20, 6, 4
+    for shift in range(-4 * m - 8, 4 * n + 9, 2):
+        bytes_a, bytes_b = set(range(4 * n)), set(range(shift, shift + 4 * m))
+        assert bool(f(base, n, base + shift, m)) == bool(bytes_a & bytes_b) == bool(f(base + shift, m, base, n)), shift
