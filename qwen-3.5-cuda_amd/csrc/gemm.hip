@@ -1594,6 +1594,12 @@ bool gemm_rows_ok(int rows, int K, const float* x) {
            4 * static_cast<uint64_t>(rows) * static_cast<uint64_t>(K) < (uint64_t{1} << 32);
 }
 
+// Below 16 tokens a call stands in for one GEMV per token, after which a token's x may be overwritten: an output that
+// overlaps x takes them.
+bool outputs_apart(int rows, int M, int K, const float* x, const float* y) {
+    return rows >= kGemmMinRows || !floats_overlap(x, static_cast<size_t>(rows) * K, y, static_cast<size_t>(rows) * M);
+}
+
 bool gemm_job_ok(int type, uint64_t element_offset, int M, int K) {
     return element_offset % 256 == 0 &&
            (type == kQ4_K ? gemm_offsets_fit(true, 144, M, K) : type == kQ6_K && gemm_offsets_fit(false, 210, M, K));
@@ -1801,7 +1807,9 @@ int qwen_matmul_rows(const void* weight, int type, uint64_t num_elements, const 
     QK_REQUIRE(rows >= 0, "matmul_rows: negative rows %d", rows);
     if (rows == 0) return ok();
     QK_REQUIRE(x && y, "matmul_rows: null pointer");
-    const Path path = gemm_rows_ok(rows, K, x) && gemm_job_ok(type, element_offset, M, K) ? gemm_path(rows, K, M) : Path::gemv;
+    const bool gemm = gemm_rows_ok(rows, K, x) && gemm_job_ok(type, element_offset, M, K) &&
+                      outputs_apart(rows, M, K, x, y);
+    const Path path = gemm ? gemm_path(rows, K, M) : Path::gemv;
     if (path == Path::gemv) return per_token(weight, type, num_elements, x, y, rows, M, K, element_offset, stream);
     const hipStream_t s = as_stream(stream);
     Prepared p;
@@ -1835,7 +1843,8 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
     QK_REQUIRE(rows >= 0, "matmul_rows_multi: negative rows %d", rows);
     if (rows == 0) return ok();
     QK_REQUIRE(x, "matmul_rows_multi: null x");
-    const bool gemm = gemm_rows_ok(rows, K, x);
+    bool gemm = gemm_rows_ok(rows, K, x);
+    for (int j = 0; j < n; ++j) gemm &= outputs_apart(rows, descs[j].M, K, x, descs[j].y);
     Path path[64];
     bool any = false, prep = false, all_gemv = true;
     for (int j = 0; j < n; ++j) {

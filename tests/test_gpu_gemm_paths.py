@@ -114,6 +114,24 @@ def test_few_tokens_keep_small_channels_beside_a_large_one(kind, T, M, K):
         assert err[0] <= 1.1 * err[1], (big, scale, err)
 
 
+@pytest.mark.parametrize("T", [3, 15])
+def test_few_tokens_over_their_inputs(T):
+    """Below 16 tokens a token's outputs may lie where the tokens before it were read: one GEMV per token then, with
+    its bits, in a single call and in one of several matrices."""
+    M = K = 512
+    w, v = _dev(_weight("Q4_K", M, K, 5)), _dev(_weight("Q6_K", 48, K, 6))
+    x = _dev(np.random.default_rng(T).standard_normal((T, K)).astype(F32))
+    ref = torch.stack([ops.matmul_dispatch(w, "Q4_K", M * K, x[t], M, K) for t in range(T)]).cpu().numpy()
+    buf = torch.cat([torch.zeros((1, K), device="cuda"), x])
+    ops.matmul_rows(w, "Q4_K", M * K, buf[1:], M, K, out=buf[:-1])
+    assert_bits_equal(buf[:-1].cpu().numpy(), ref)
+    buf = torch.cat([torch.zeros((1, K), device="cuda"), x])
+    other = ops.matmul_rows_multi([(v, "Q6_K", 48 * K, 48, 0, None), (w, "Q4_K", M * K, M, 0, buf[:-1])], buf[1:], K)[0]
+    assert_bits_equal(buf[:-1].cpu().numpy(), ref)
+    one = torch.stack([ops.matmul_dispatch(v, "Q6_K", 48 * K, x[t], 48, K) for t in range(T)])
+    assert_bits_equal(other.cpu().numpy(), one.cpu().numpy())
+
+
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("T", [5, 40, 150, 800])
 def test_nonfinite_rows_in_every_form(oracle, kind, T):
