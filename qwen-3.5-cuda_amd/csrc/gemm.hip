@@ -1846,11 +1846,10 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
     bool gemm = gemm_rows_ok(rows, K, x);
     for (int j = 0; j < n; ++j) gemm &= outputs_apart(rows, descs[j].M, K, x, descs[j].y);
     Path path[64];
-    bool any = false, prep = false, all_gemv = true;
+    bool prep = false, all_gemv = true;
     for (int j = 0; j < n; ++j) {
         const qwen_gemv_desc& e = descs[j];
         path[j] = gemm && gemm_job_ok(e.type, e.element_offset, e.M, K) ? gemm_path(rows, K, e.M) : Path::gemv;
-        any |= path[j] != Path::gemv;
         prep |= path[j] != Path::gemv && path[j] != Path::f32 && path[j] != Path::few;
         all_gemv &= path[j] == Path::gemv;
     }
@@ -1866,9 +1865,8 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
         return ok();
     }
     const hipStream_t s = as_stream(stream);
-    Prepared p{};
-    if (any)
-        if (const int rc = prepare_x(prep, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
+    Prepared p;
+    if (const int rc = prepare_x(prep, x, rows, K, workspace, workspace_bytes, s, p)) return rc;
     for (const int type : {static_cast<int>(kQ4_K), static_cast<int>(kQ6_K)})
         for (const Path to : {Path::f32, Path::few, Path::sliced4, Path::sliced2, Path::whole}) {
             GemmJobs jobs{};
@@ -1887,8 +1885,7 @@ int qwen_matmul_rows_multi(const qwen_gemv_desc* descs, int n, const float* x, i
             }
             if (jobs.n) launch_gemm(to, type, jobs, p, rows, K, s);
         }
-    if (any)
-        if (const int rc = check_launch("matmul_rows_multi")) return rc;
+    if (const int rc = check_launch("matmul_rows_multi")) return rc;
     for (int j = 0; j < n; ++j) {   // the rest: one GEMV per token
         const qwen_gemv_desc& e = descs[j];
         if (path[j] != Path::gemv) continue;
