@@ -511,8 +511,9 @@ int qwen_matmul_dispatch(const void* weight, int type, uint64_t num_elements, co
  * integers, products are exact (Q6_K: but for one below 2^-22 of the others)
  * and sums fp32; those calls need a 16-byte aligned workspace of
  * qwen_matmul_rows_workspace_bytes(rows, K) bytes
- * (QWEN_STATUS_INVALID_ARGUMENT otherwise); fewer rows ignore it, and the
- * other cases run qwen_matmul_dispatch once per token. A row of x holding an
+ * (QWEN_STATUS_INVALID_ARGUMENT otherwise); fewer rows ignore it. The other
+ * cases, and fewer than 16 rows with y overlapping x, run qwen_matmul_dispatch
+ * once per token and ignore it. A row of x holding an
  * infinity gives non-finite outputs (the NaN / infinity pattern may differ
  * from the reference's). rows == 0 is a no-op. Statuses and messages as
  * qwen_matmul_dispatch; rows < 0 or a NULL x / y -> QWEN_STATUS_INVALID_ARGUMENT.
@@ -556,9 +557,12 @@ int qwen_matmul_dispatch_multi(const qwen_gemv_desc* descs, int n, const float* 
 /* qwen_matmul_rows for n matrices of the same x [rows x K]: y_j [rows x M_j] =
  * x W_j^T for each descriptor (split must be 0), with the results of n
  * qwen_matmul_rows calls bit for bit. x is prepared once (at most one prep
- * launch) and the Q4_K / Q6_K matrices of one type run in one GEMM launch (up
- * to 8 per launch; from 769 rows on, matrices of up to 64 rows in one of their
- * own); other types and offsets take the per-token path.
+ * launch) and the Q4_K / Q6_K matrices of one type and kernel run in one GEMM
+ * launch (up to 8 per launch). Matrices of one call take different kernels
+ * from 1025 rows on (those of up to 64 rows have a launch of their own, K a
+ * multiple of 512) and at 161 to 2048 rows from K = 4096 (below and from 4096
+ * rows of the matrix); other types and offsets take the per-token path, and so
+ * do all matrices below 16 rows where an output overlaps x.
  * Validation as qwen_matmul_dispatch_multi; workspace as qwen_matmul_rows
  * (qwen_matmul_rows_workspace_bytes(rows, K)). 0 <= n <= 64.
  * ref: the per-token calls of src/layer_gdn.cpp:83-86, src/layer_attn.cpp:85-87 over a prompt */

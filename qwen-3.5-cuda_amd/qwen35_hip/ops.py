@@ -875,7 +875,7 @@ def matmul_rows(weight, ggml_type, num_elements: int, x, M: int, K: int, element
 def matmul_rows_multi(jobs, x, K: int, workspace=None, stream=None):
     """jobs: (weight uint8 tensor, ggml type, num_elements, M, element_offset, out float32 [rows, M]
     or None); y_j = x W_j^T for every job from one x [rows, K] (one prep, one GEMM launch per
-    K-quant type). Returns the outputs."""
+    K-quant type and kernel). Returns the outputs."""
     _dev(x, dtype=torch.float32)
     if x.dim() != 2 or x.shape[1] != K:
         raise ValueError(f"x must be [rows, {K}], got {tuple(x.shape)}")

@@ -9,6 +9,7 @@ import torch
 
 from conftest import assert_bits_equal
 from qwen35_hip import ops
+from qwen35_hip._lib import check
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +54,27 @@ def test_up_to_28_rows_are_the_token_loop():
     two = ops.gdn_recurrent_rows(b, qkv, beta, decay, 16, 32, 128, 128)
     assert_bits_equal(one.cpu().numpy(), two.cpu().numpy(), what="out")
     assert_bits_equal(a.cpu().numpy(), b.cpu().numpy(), what="state")
+
+
+def test_row_strides_past_the_walks_limit_are_the_token_loop():
+    """29 rows, the first count of the chunked kernels, at a stride of 2^31 / 256 floats and more: the token loop's bits
+    (a row of the 0.97 GB buffer holds the 2 key and 2 value heads; the rest is never read)."""
+    rows, stride, kh, vh, dv = 29, 8_400_000, 2, 2, 32
+    g = torch.Generator(device="cuda").manual_seed(8)
+    wide = torch.zeros((rows, stride), device="cuda")
+    wide[:, :2 * kh * 128 + vh * dv] = 0.1 * torch.randn((rows, 2 * kh * 128 + vh * dv), generator=g, device="cuda")
+    beta, decay = torch.rand((2, rows, vh), generator=g, device="cuda")
+    state = torch.randn((vh, 128, dv), generator=g, device="cuda")
+    lib, p = ops.load(), wide.data_ptr()
+    ws = torch.empty(lib.qwen_gdn_recurrent_chunked_workspace_bytes(rows, vh), dtype=torch.uint8, device="cuda")
+    res = []
+    for fn, extra in ((lib.qwen_gdn_recurrent_chunked, (ws.data_ptr(), ws.numel())), (lib.qwen_gdn_recurrent_rows, ())):
+        s, out = state.clone(), torch.empty((rows, vh * dv), device="cuda")
+        check(fn(s.data_ptr(), p, p + 4 * kh * 128, p + 8 * kh * 128, beta.data_ptr(), decay.data_ptr(), out.data_ptr(),
+                 rows, kh, vh, 128, dv, stride, vh * dv, *extra, torch.cuda.current_stream().cuda_stream))
+        res.append((out.cpu().numpy(), s.cpu().numpy()))
+    assert_bits_equal(res[0][0], res[1][0], what="out")
+    assert_bits_equal(res[0][1], res[1][1], what="state")
 
 
 @pytest.mark.parametrize("rows,kh,dim,kernel,heads,skew", [(1, 16, 128, 4, 32, 0), (3, 2, 64, 4, 3, 0), (24, 16, 128, 4, 32, 0),

@@ -153,6 +153,36 @@ def test_nonfinite_rows_in_every_form(oracle, kind, T):
 
 
 @pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("T,M,K", [(1183, 3600, 256), (200, 96, 4096), (18, 40, 1280)])
+def test_nonfinite_rows_in_the_other_tiles(oracle, kind, T, M, K):
+    """The same in the 128 x 256 tiles (both token halves, the ragged last tile), two slices of K, and the form that
+    converts x itself."""
+    w = _weight(kind, M, K, 7)
+    x = np.random.default_rng(T).standard_normal((T, K)).astype(F32)
+    inf = sorted({0, 70 % T, T - 1})
+    x[inf, K // 2] = [np.inf, -np.inf, np.inf][:len(inf)]
+    x[[1, T - 2], 7] = np.nan
+    x[5] = 0.0
+    got = ops.matmul_rows(_dev(w), kind, M * K, _dev(x), M, K).cpu().numpy()
+    for t in inf:
+        ref = oracle.gemv(w, ops.GGML_TYPES[kind], x[t], M, K)
+        assert np.array_equal(np.isnan(got[t]), np.isnan(ref))
+        assert np.array_equal(got[t][np.isinf(ref)], ref[np.isinf(ref)])
+    assert np.isnan(got[[1, T - 2]]).all() and np.array_equal(got[5].view(np.uint32), np.zeros(M, np.uint32))
+    for t in (2, 6, T - 3):
+        assert rel_err(got[t], oracle.gemv(w, ops.GGML_TYPES[kind], x[t], M, K), group=M).max() <= 1e-5
+
+
+@pytest.mark.parametrize("T", [3, 15, 40])
+def test_rows_off_16_byte_alignment_are_the_gemv(T):
+    M, K = 96, 2048
+    w = _dev(_weight("Q4_K", M, K, 7))
+    x = torch.randn(T * K + 1, generator=torch.Generator().manual_seed(T)).cuda()[1:].view(T, K)
+    one = torch.stack([ops.matmul_dispatch(w, "Q4_K", M * K, x[t], M, K) for t in range(T)])
+    assert_bits_equal(ops.matmul_rows(w, "Q4_K", M * K, x, M, K).cpu().numpy(), one.cpu().numpy())
+
+
+@pytest.mark.parametrize("kind", ["Q4_K", "Q6_K"])
 @pytest.mark.parametrize("T,K", [(1024, 2048), (1360, 1280), (512, 4096)])
 def test_prep_spread_over_workgroups_keeps_the_bits(kind, T, K):
     """The last token count whose prep takes a workgroup per 512 elements of K, against one tile more (all of K in

@@ -553,8 +553,8 @@ def _check_gdn_recurrence(oracle, qkv, beta, decay, state, out, new_state, kh, v
                                         (700, "normal"), (150, "fast_decay"), (150, "beta_one"),
                                         (128, "tiny_late_beta")])
 def test_gdn_recurrent_chunked(oracle, rows, gates):
-    """The chunked prefill form against the oracle's token loop at the Qwen3.5 GDN shape:
-    partial last chunks, several chunks, decays that underflow to zero inside a chunk
+    """The prefill form (chunked from 29 rows on, the token loop below) against the oracle's
+    token loop at the Qwen3.5 GDN shape: partial last chunks, several chunks, decays that underflow to zero inside a chunk
     (the ratios are running products), beta near 1 (the triangular solve's
     largest off-diagonal terms), and fast decay with beta ~1e-17 on the second half of
     each chunk, ending in that half: the final state (~1e-23 for some heads) is then
@@ -600,9 +600,9 @@ def test_gdn_recurrent_chunked_head_maps(oracle, kh, vh):
 def test_gdn_recurrent_chunked_strides(oracle):
     """Row strides the chunked state walk addresses with 32-bit lane offsets from a
     per-chunk base: a qkv row padded past q | k | v and an output row padded past its
-    values (the padding stays untouched); one row with strides 0 (the walk reads a
-    range one stride long, so the library widens it to the row); and a qkv stride past
-    the walk's 32-bit limit, which runs the token loop (the same bits as calling it)."""
+    values (the padding stays untouched); one row with strides 0 (the token loop, which
+    does not step between rows); and a qkv stride past the walk's 32-bit limit, which
+    runs the token loop at any row count (the same bits as calling it)."""
     import ctypes
     from qwen35_hip._lib import check
 
@@ -1586,8 +1586,8 @@ GEMM_CASES = [   # kind, tokens, M, K, first row (element offset = row * K)
 def test_matmul_rows(oracle, kind, T, M, K, row0):
     """matmul_rows (T tokens in one call) against the oracle's GEMV of each
     token (src/cuda/matmul_q4.cu:140-167): the matrix-core path for Q4_K / Q6_K
-    at 16 tokens or more (ragged token and row tiles, a row offset), the
-    per-token GEMV below 16 tokens, for K % 256 != 0 and for other types.
+    (fp32 below 16 tokens; ragged token and row tiles, a row offset), the
+    per-token GEMV for K % 256 != 0 and for other types.
     Output rows past T stay untouched."""
     t = ops.GGML_TYPES[kind]
     r = rng(T * 31 + M + K)
