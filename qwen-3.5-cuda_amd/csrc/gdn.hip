@@ -47,8 +47,9 @@ constexpr int kGateUnroll = 4;   // head groups in flight per wave (norm_gate)
 // GATES: workgroups from first_block on evaluate the rows' delta-rule gates, n
 // values in all. A prompt's gate launch is latency alone (rows x 32 values, 2.7
 // us at 9 rows, 4.9 at 4096); beside the convolution it costs nothing that shows:
-// a GDN layer over 9 rows 64.6 -> 55.1 us (a call less for the host, too), 77
-// rows 82.7 -> 80.6, 777 rows (Q6_K) 341 -> 336.
+// a GDN layer over 9 rows 64.6 -> 55.1 us (bound by the host, which has a call
+// less; 55 to 60 from machine to machine), 77 rows 82.7 -> 80.6, 777 rows (Q6_K)
+// 341 -> 336.
 struct GateRows {
     const float* b;
     const float* alpha;

@@ -18,7 +18,8 @@
 // The decay ratios are running products, never quotients, so decays that
 // underflow give exact zeros rather than 0/0.
 //
-// Kernel A (one workgroup per (chunk, key head), all chunks in parallel): the
+// Kernel A (one workgroup per (chunk, key head), or per value head of a short
+// prompt, all chunks in parallel): the
 // chunk's K and Q as fp16 pairs (below), K K^T and Q K^T from them once, then
 // for each value head that reads this key head the ratios and T as a blocked
 // inverse (16 x 16 diagonal blocks by forward substitution, the others as fp32

@@ -939,8 +939,8 @@ __global__ __launch_bounds__(kGemvBlock) void gemv_q6k_direct_multi(const float*
 // 4q .. 4q+3; wave w
 //   * decodes the unit of rows 4q .. 4q+3 of routed expert j = w + 4t (t < KT)
 //     against that expert's hidden row;
-//   * computes row 4q + w of the shared expert's down projection (SS = 0: wave
-//     3, which has one routed expert fewer when k < 8, all four rows);
+//   * computes row 4q + w of the shared expert's down projection (SS = 0: all
+//     four rows, in every wave alike; wave 3's are taken);
 // with the per-row kernel's units, lane map and reductions, so each expert
 // output and the shared output have the bits of the separate launches (the
 // expert GEMVs, the shared GEMV). Lanes 0..3 of wave 0 then combine
