@@ -880,14 +880,19 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     QK_REQUIRE(workspace_bytes >= need, "gdn_recurrent_chunked: workspace of %zu bytes, %zu needed", workspace_bytes,
                need);
     // One row needs no stride; the limit that longer calls have on theirs holds for its length.
-    QK_REQUIRE(rows > 1 || std::max(static_cast<int64_t>(key_heads) * key_dim,
-                                    static_cast<int64_t>(value_heads) * value_dim) <= kMaxWalkStride,
-               "gdn_recurrent_chunked: row too long for the chunked walk");
+    const int64_t qk = static_cast<int64_t>(key_heads) * key_dim, vals = static_cast<int64_t>(value_heads) * value_dim;
+    const int64_t extent = std::max(qk, vals);
+    QK_REQUIRE(rows > 1 || extent <= kMaxWalkStride, "gdn_recurrent_chunked: row too long for the chunked walk");
     // A few tokens: the token loop, 0.25 us a token from 8 us, against the two launches' 15.6 us for one chunk (9
-    // tokens 10.1 us, 32 tokens 16.0 against 15.6, 48 tokens 20.0 against 16.0). Its error is the smaller one.
-    if (rows <= kLoopRows)
+    // tokens 10.1 us, 32 tokens 16.0 against 15.6, 48 tokens 20.0 against 16.0). Its error is the smaller one. Outputs
+    // that lie over q or k need the chunked kernels, which have read all of both before the first output.
+    const size_t span = static_cast<size_t>((rows - 1) * qkv_stride + qk),
+                 out_span = static_cast<size_t>((rows - 1) * out_stride + vals);
+    if (rows <= kLoopRows && !floats_overlap(out, out_span, q, span) && !floats_overlap(out, out_span, k, span))
         return qwen_gdn_recurrent_rows(state, q, k, v, beta, decay, out, rows, key_heads, value_heads, key_dim,
                                        value_dim, qkv_stride, out_stride, stream);
+    // The walk's buffer range is one stride long, so one row's must cover its values.
+    const int64_t vs = rows == 1 ? extent : qkv_stride, os = rows == 1 ? extent : out_stride;
     const hipStream_t s = as_stream(stream);
     const int nchunks = (rows + kC - 1) / kC;
     float* ws = static_cast<float*>(workspace);
@@ -896,8 +901,7 @@ int qwen_gdn_recurrent_chunked(float* state, const float* q, const float* k, con
     gdn_chunk_prep<<<dim3(nchunks, g.heads), kThreads, 0, s>>>(q, k, beta, decay, ws, kq, rows, key_heads, value_heads,
                                                               g.step, qkv_stride);
     gdn_chunk_state<<<(value_dim / kNB) * value_heads, kWalkThreads, 0, s>>>(state, v, ws, kq, out, rows, key_heads,
-                                                                             value_heads, value_dim, qkv_stride,
-                                                                             out_stride);
+                                                                             value_heads, value_dim, vs, os);
     return check_launch("gdn_recurrent_chunked");
 }
 

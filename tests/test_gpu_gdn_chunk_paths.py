@@ -14,20 +14,20 @@ from qwen35_hip._lib import check
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows,kh,vh", [(1, 16, 32), (28, 16, 32), (29, 16, 32), (64, 4, 4), (65, 4, 12), (512, 16, 32),
-                                        (513, 16, 32), (100, 8, 4), (64, 2, 3), (130, 16, 24), (700, 16, 24), (65, 3, 8)])
-def test_chunked_routes(rows, kh, vh):
-    """Output and state against the recurrence in float64, under the bar of the other recurrence tests: 1e-5 of the
-    larger of the value and its condition scale (here each head's largest terms, |q||S| of the readout)."""
+def _inputs(rows, kh, vh):
     g = torch.Generator(device="cuda").manual_seed(rows * 7 + vh)
     n = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
     qk = torch.nn.functional.normalize(n(rows, 2 * kh, 128), dim=-1)
     qk[:, :kh] /= 128 ** 0.5
     qkv = torch.cat([qk.reshape(rows, -1), n(rows, vh * 128)], 1).contiguous()
     beta, decay = torch.sigmoid(n(rows, vh)), torch.exp(-torch.rand((rows, vh), generator=g, device="cuda") * 2)
-    state = 0.1 * n(vh, 128, 128)
-    got_s = state.clone()
-    got = ops.gdn_recurrent_chunked(got_s, qkv, beta, decay, kh, vh, 128, 128)
+    return qk, qkv, beta, decay, 0.1 * n(vh, 128, 128)
+
+
+def _check(got, got_s, qk, qkv, beta, decay, state, kh, vh):
+    """Output and state against the recurrence in float64, under the bar of the other recurrence tests: 1e-5 of the
+    larger of the value and its condition scale (here each head's largest terms, |q||S| of the readout)."""
+    rows = qk.shape[0]
     idx = torch.arange(vh, device="cuda") % kh
     S, out, cond = state.double(), [], []
     for t in range(rows):
@@ -44,6 +44,15 @@ def test_chunked_routes(rows, kh, vh):
     assert bool(((got_s.double() - S).abs() <= 1e-5 * torch.maximum(S.abs(), rms)).all())
 
 
+@pytest.mark.parametrize("rows,kh,vh", [(1, 16, 32), (28, 16, 32), (29, 16, 32), (64, 4, 4), (65, 4, 12), (512, 16, 32),
+                                        (513, 16, 32), (100, 8, 4), (64, 2, 3), (130, 16, 24), (700, 16, 24), (65, 3, 8)])
+def test_chunked_routes(rows, kh, vh):
+    qk, qkv, beta, decay, state = _inputs(rows, kh, vh)
+    got_s = state.clone()
+    got = ops.gdn_recurrent_chunked(got_s, qkv, beta, decay, kh, vh, 128, 128)
+    _check(got, got_s, qk, qkv, beta, decay, state, kh, vh)
+
+
 def test_up_to_28_rows_are_the_token_loop():
     g = torch.Generator(device="cuda").manual_seed(5)
     qkv = torch.randn((28, 8192), generator=g, device="cuda")
@@ -54,6 +63,24 @@ def test_up_to_28_rows_are_the_token_loop():
     two = ops.gdn_recurrent_rows(b, qkv, beta, decay, 16, 32, 128, 128)
     assert_bits_equal(one.cpu().numpy(), two.cpu().numpy(), what="out")
     assert_bits_equal(a.cpu().numpy(), b.cpu().numpy(), what="state")
+
+
+@pytest.mark.parametrize("rows", [1, 9, 28, 29])
+@pytest.mark.parametrize("part", ["q", "k", "v"])
+def test_outputs_over_their_inputs(rows, part):
+    """Outputs over the q, k or v of their own rows (q and k are read by other workgroups, the v of a column only by the
+    one that writes it)."""
+    kh, vh, lib = 16, 16, ops.load()
+    qk, qkv, beta, decay, state = _inputs(rows, kh, vh)
+    buf, s, row = qkv.clone(), state.clone(), qkv.shape[1]
+    q = buf.data_ptr()
+    out = q + 4 * 2048 * "qkv".index(part)
+    ws = torch.empty(lib.qwen_gdn_recurrent_chunked_workspace_bytes(rows, vh), dtype=torch.uint8, device="cuda")
+    check(lib.qwen_gdn_recurrent_chunked(s.data_ptr(), q, q + 4 * 2048, q + 8 * 2048, beta.data_ptr(), decay.data_ptr(),
+                                         out, rows, kh, vh, 128, 128, 0 if rows == 1 else row, 0 if rows == 1 else row,
+                                         ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    first = 2048 * "qkv".index(part)
+    _check(buf[:, first:first + 2048], s, qk, qkv, beta, decay, state, kh, vh)
 
 
 def test_row_strides_past_the_walks_limit_are_the_token_loop():
