@@ -225,7 +225,7 @@ int qwen_gdn_decode_step(const float* x, const float* conv_weight, const float* 
  * Arguments as qwen_gdn_recurrent_rows plus a caller-owned device workspace of
  * at least qwen_gdn_recurrent_chunked_workspace_bytes(rows, value_heads)
  * (16-byte aligned; contents scratch). Up to 28 rows run the token loop, whose
- * time is below that of one chunk, under the same checks (the workspace and the
+ * time is below that of one chunk, unless out overlaps q or k, under the same checks (the workspace and the
  * limit of 2^31 / 256 floats on a row among them). Shapes the chunked kernels do
  * not cover (key_dim != 128, value_dim not a multiple of 16, unaligned q / k,
  * row strides above that limit) run the token loop and need no workspace. The
